@@ -953,3 +953,52 @@ def test_predict_frames_rejects_out_of_range(gpu):
         lib.pd_dev_free(q)
     clf.close()
 
+
+
+def _tie_ts(kind, rng, n_classes, n_samples, levels):
+    """Images of a few distinct depths (many candidates with equal responses,
+    so many (threshold, candidate) pairs with equal or nearly equal gains)."""
+    ts = pa.TrainingSet(n_classes)
+    for _ in range(3):
+        w, h = 64, 48
+        im = rng.choice(np.linspace(1000, 4000, levels).astype(np.uint16), (h, w))
+        if kind == pa.PD_FEAT_DEPTH_F32:
+            im = (im / 1000.0).astype(np.float32)
+        lab = (1 + rng.integers(0, n_classes, (h, w))).astype(np.uint8)
+        smp = np.sort(rng.integers(0, w * h, n_samples)).astype(np.uint32)
+        ts << pa.TrainingSetImage(im, w, h, lab, n_classes, smp)
+    return ts
+
+
+@pytest.mark.parametrize("kind,n_classes,nF,nT,levels,samples", [
+    (pa.PD_FEAT_DEPTH_U16, 8, 70, 20, 1, 300),     # one depth: every pair one-sided, all gains equal
+    (pa.PD_FEAT_DEPTH_U16, 8, 70, 20, 2, 300),     # three responses: large groups of equal gains
+    (pa.PD_FEAT_DEPTH_U16, 16, 130, 32, 3, 700),
+    (pa.PD_FEAT_DEPTH_U16, 64, 65, 16, 3, 900),    # most classes
+    (pa.PD_FEAT_DEPTH_U16, 4, 65, 64, 3, 900),     # most thresholds
+    (pa.PD_FEAT_DEPTH_U16, 2, 64, 2, 4, 5000),     # two pairs per column, larger counts
+    (pa.PD_FEAT_DEPTH_F32, 5, 100, 9, 2, 40),      # small nodes, bucket padding
+    (pa.PD_FEAT_DEPTH_U16, 1, 64, 10, 3, 100),     # one class: every gain 0
+])
+def test_pruned_split_search_equals_exhaustive(gpu, kind, n_classes, nF, nT, levels, samples):
+    """The fused split search evaluates exactly only the pairs whose
+    approximate gain is within the error bound of the tile's largest: with
+    groups of equal and nearly equal gains the winner (lowest pair index), its
+    FP32 gain and the whole tree stay the oracle's."""
+    rng = np.random.default_rng(1000 + n_classes + nT)
+    ts = _tie_ts(kind, rng, n_classes, samples, levels)
+    b, t = (60.0, 0.8) if kind == pa.PD_FEAT_DEPTH_F32 else (60000.0, 800.0)
+    p = pa.TreeTrainerParameters(nF, nT, [-b] * 4, [b] * 4, -t, t, 5)
+    tr = pa.HIPTreeTrainer(kind, n_classes)
+    tr.set_training_set(ts)
+    tree = pa.Tree(3, 7, kind, n_classes)
+    diag = tr.train(tree, ts, p, 1, 7, diagnostics=True)
+    ref = orc.train_tree(orc.Tset(kind, ts), p, ts.priors, 3, 7)
+    assert np.array_equal(tree.left_children, ref["left_children"])
+    assert tree.features.tobytes() == ref["features"].tobytes()
+    assert tree.thresholds.tobytes() == ref["thresholds"].tobytes()
+    assert tree.posteriors.tobytes() == ref["posteriors"].tobytes()
+    trained = ref["left_children"] >= 0
+    assert np.array_equal(diag["node_k"][trained], ref["node_k"][trained])
+    assert diag["node_gain"][trained].tobytes() == ref["node_gain"][trained].tobytes()
+    tr.close()
