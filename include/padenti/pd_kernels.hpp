@@ -470,30 +470,54 @@ __global__ __launch_bounds__(NWAVES * 64) void k_hist(
     }
   }
   __syncthreads();
-  // Per (t, f): rank L_t = #{t' < nT : thr_t' < thr_t} (used by the flush)
-  // and the stable sort position (ties by index) that scatters the column's
-  // thresholds into sorted order; slots nT..NS-1 hold the padding value.
-  for (uint32_t t = wave * SPW + sub; t < (uint32_t)NS; t += NW * SPW) {
-    if (t >= nT) {
-      sth[t * FPW + col] = pad_threshold<T>();
-      continue;
+  // Per (t, f): the stable sort position (ties by index) that scatters the
+  // column's thresholds into sorted order; slots nT..NS-1 hold the padding
+  // value, which is below nothing.  A group of waves sorts the column's
+  // thresholds TS at a time against one pass over all of them (one threshold a
+  // pass with two compares each read the column TS times: histograms of a tree of
+  // depth 20, 4000 x 32 candidates, 123 -> 119 ms).
+  {
+    constexpr uint32_t G = NW * SPW;                          // thresholds per step
+    constexpr int TS = (NTP + (int)G - 1) / (int)G;           // thresholds per lane
+    T th[TS];
+    uint32_t P[TS];
+#pragma unroll
+    for (int i = 0; i < TS; i++) {
+      const uint32_t t = (uint32_t)i * G + wave * SPW + sub;
+      th[i] = st[(t < (uint32_t)NTP ? t : 0u) * FPW + col];
+      P[i] = 0u;
     }
-    const T th = st[t * FPW + col];
-    uint32_t L = 0, P = 0;
 #pragma unroll 4
     for (int t2 = 0; t2 < NTP; t2++) {
       const T o = st[t2 * FPW + col];
-      const bool live = (uint32_t)t2 < nT;
-      L += (live && o < th) ? 1u : 0u;
-      P += (live && (o < th || (o == th && (uint32_t)t2 < t))) ? 1u : 0u;
+#pragma unroll
+      for (int i = 0; i < TS; i++) {
+        const uint32_t t = (uint32_t)i * G + wave * SPW + sub;
+        P[i] += ((uint32_t)t2 < t ? o <= th[i] : o < th[i]) ? 1u : 0u;
+      }
     }
-    sl[t * FPW + col] = (uint8_t)L;
-    sth[P * FPW + col] = th;
+#pragma unroll
+    for (int i = 0; i < TS; i++) {
+      const uint32_t t = (uint32_t)i * G + wave * SPW + sub;
+      if (t < nT) {
+        sth[P[i] * FPW + col] = th[i];
+        sl[t * FPW + col] = (uint8_t)P[i];   // L_t once equal thresholds are counted out, below
+      }
+    }
+    for (uint32_t t = nT + wave * SPW + sub; t < (uint32_t)NS; t += G) sth[t * FPW + col] = pad_threshold<T>();
   }
   T p[FD];
 #pragma unroll
   for (int j = 0; j < FD; j++) p[j] = sp[j * FPW + col];
   __syncthreads();   // staging read by every wave: the bins may now take its place
+  // rank L_t = #{t' < nT : thr_t' < thr_t} (used by the flush): the sorted
+  // position of the first threshold equal to thr_t
+  for (uint32_t t = wave * SPW + sub; t < nT; t += NW * SPW) {
+    uint32_t l = sl[t * FPW + col];
+    const T th = sth[l * FPW + col];
+    while (l > 0u && !(sth[(l - 1u) * FPW + col] < th)) l--;
+    sl[t * FPW + col] = (uint8_t)l;
+  }
   for (uint32_t i = tid; i < nC * (uint32_t)(RW * bin_row_words<WIDE, (int)FPW>()); i += NTH) bins[i] = 0u;
   __syncthreads();
 
