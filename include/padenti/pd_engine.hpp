@@ -88,6 +88,20 @@ Bounds<F> make_bounds(const pd_train_params &P)
   return b;
 }
 
+// Every candidate drawn from the bounds may take the hook's fast form: its
+// offset parameters (the first four) lie in [lo, hi], so within RECIP_MAX.
+template <class F>
+bool fast_bounds(const Bounds<F> &b)
+{
+  if constexpr (has_fast<F>::value) {
+    for (int j = 0; j < 4; j++)
+      if (!(std::fabs((float)b.lo[j]) <= RECIP_MAX && std::fabs((float)b.hi[j]) <= RECIP_MAX)) return false;
+    return true;
+  } else {
+    return false;
+  }
+}
+
 inline void check_params(const pd_train_params &P, int fd, bool is_short)
 {
   require(P.n_features >= 1, "n_features must be >= 1");
@@ -730,7 +744,7 @@ struct Trainer final : TrainerBase {
                        d_slot_mode.as<uint8_t>(), d_slot_hidx.as<int32_t>(), d_tot.as<uint32_t>(),
                        d_slot_h.as<float>(), bnd, tree, nF,
                        nT, nC, d_H.as<uint32_t>(), d_cand_key.as<unsigned long long>(), d_cand_left.as<uint32_t>(),
-                       d_map_cur, d_perm_cur, d_ctab_cur, ac);
+                       d_map_cur, d_perm_cur, d_ctab_cur, fast_bounds(bnd) ? 1u : 0u, ac);
     HIPCHK(hipGetLastError());
   }
 
@@ -2013,6 +2027,7 @@ struct Forest final : ForestBase {
   std::vector<uint32_t> h_tree_off, h_leaf_off;
   std::vector<uint32_t> depths;
   uint32_t max_depth = 1;
+  bool fast_nodes = true;   // every node's offset parameters are within RECIP_MAX
   DevBuf d_nodes, d_leaf_post, d_leaf_id, d_tree_off, d_leaf_off;
   DevBuf d_img, d_mask, d_out, d_leaf, d_frames;
   // auto-context hooks: the trees' breadth-first arrays (the hook reads them)
@@ -2082,6 +2097,8 @@ struct Forest final : ForestBase {
         order.push_back(2 * i + 2);
         r.thr = thrs[i];
         for (int j = 0; j < F::FeatDim; j++) r.p[j] = feats[i * F::FeatDim + j];
+        if constexpr (has_fast<F>::value)
+          for (int j = 0; j < 4; j++) fast_nodes = fast_nodes && std::fabs((float)r.p[j]) <= RECIP_MAX;
       } else {
         const uint32_t leaf = (uint32_t)h_leaf_id.size() - leaf_base;
         r.left = -1 - (int32_t)leaf;
@@ -2120,8 +2137,17 @@ struct Forest final : ForestBase {
   void launch(uint32_t blocks, const I *pix, const FrameDesc *frames, uint32_t n_frames, const uint8_t *masks,
               uint32_t tree0, uint32_t ntr, uint32_t steps, float *out_post, int32_t *out_leaf)
   {
+    if constexpr (has_fast<F>::value) {
+      if (fast_nodes) return launch_k<NCM, true>(blocks, pix, frames, n_frames, masks, tree0, ntr, steps, out_post, out_leaf);
+    }
+    launch_k<NCM, false>(blocks, pix, frames, n_frames, masks, tree0, ntr, steps, out_post, out_leaf);
+  }
+  template <int NCM, bool FAST>
+  void launch_k(uint32_t blocks, const I *pix, const FrameDesc *frames, uint32_t n_frames, const uint8_t *masks,
+                uint32_t tree0, uint32_t ntr, uint32_t steps, float *out_post, int32_t *out_leaf)
+  {
     const uint32_t per_xcc = (blocks + n_xcc - 1) / n_xcc;
-    hipLaunchKernelGGL((k_predict<F, NCM>), dim3(per_xcc * n_xcc), dim3(256), 0, stream, pix, frames, n_frames, blocks,
+    hipLaunchKernelGGL((k_predict<F, NCM, FAST>), dim3(per_xcc * n_xcc), dim3(256), 0, stream, pix, frames, n_frames, blocks,
                        n_xcc, per_xcc, masks, d_nodes.as<Rec>(), d_tree_off.as<uint32_t>() + tree0, ntr, steps,
                        d_leaf_post.as<float>(), d_leaf_id.as<int32_t>(), d_leaf_off.as<uint32_t>() + tree0, nC,
                        out_post, out_leaf);

@@ -205,43 +205,107 @@ PD_HD int offset_of_num(float q, float p)
 #endif
 }
 
-// Texel of channel `ch` at x + round(px/d), y + round(py/d) with an integer
-// depth d > 0 (IntDivPrep) and an integer pixel type, or `bg` when the offset
-// leaves the image; the value is returned as an int so that a hook's
+// Denominator of the unsigned 16-bit depth hooks: y = (1/d)(1 + e) with
+// 2^-52 < e < 2^-50 for an integer depth 1 <= d <= 65535 (the double
+// reciprocal, one rounding of it and of the product with 1 + 2^-51), 0 for
+// d = 0.
+struct RecipPrep {
+  double y;
+};
+
+PD_HD RecipPrep recip_prep(uint32_t d) { return RecipPrep{d ? (1.0 / (double)d) * (1.0 + 0x1p-51) : 0.0}; }
+
+// x + round(RN(p/d)), half away from zero, in the low word of one double FMA
+// (d = 0: x).  Adding 1.5 * 2^52 leaves the sum's unit at 1, so the FMA rounds
+// the exact product p * y to the nearest integer and its low 32 bits are that
+// integer plus x in two's complement.  Valid for |p| <= RECIP_MAX = 2^22:
+//  * ulp(p) <= 1/2, so every (n + 1/2) d is a multiple of ulp(p): p/d is either
+//    exactly a half-integer or at least ulp(p)/d away from it, a relative
+//    distance above 2^-24.  RN(p/d) (float) then reaches n + 1/2 only when p/d
+//    does: half an ulp of the quotient is at most 2^-24 p/d < ulp(p)/d;
+//  * y's excess e < 2^-50 is far below that distance and, being positive,
+//    carries an exact half-integer past the tie, away from zero.
+// |p * y| stays below 2^24, so the low word never wraps.
+constexpr float RECIP_MAX = 4194304.0f;
+PD_HD uint32_t recip_coord(uint32_t x, double p, RecipPrep dp)
+{
+  const uint64_t cb = 0x4338000000000000ull + x;   // the double 1.5 * 2^52 + x
+  double c;
+  memcpy(&c, &cb, 8);
+  const double s = __builtin_fma(p, dp.y, c);
+  uint64_t b;
+  memcpy(&b, &s, 8);
+  return (uint32_t)b;
+}
+
+// The same coordinate for any finite p: (float)(p * y) is RN(p/d) (a rounding
+// midpoint of the float quotient is never closer to p/d than 2^-41 of it, see
+// int_div), then the saturating rounding of offset_of_num.
+PD_HD uint32_t recip_coord_any(uint32_t x, float p, RecipPrep dp)
+{
+  return x + (uint32_t)offset_of_num((float)((double)p * dp.y), p);
+}
+
+// Texel of channel `ch` of coordinates (ox, oy) of an integer pixel type, or
+// `bg` outside the image; the value is returned as an int so that a hook's
 // difference of two probes is one integer subtraction (exact, as the float
 // one is for values below 2^24).  Only the load is predicated: lanes whose
 // probe leaves the image issue no memory access.
 template <typename ImgT, int NCH>
-PD_HD int probe_int(const ImageView<ImgT, NCH> &im, int x, int y, const IntDivPrep &dp, float px, float py, int ch,
-                    int bg)
+PD_HD int probe_at(const ImageView<ImgT, NCH> &im, uint32_t ox, uint32_t oy, int ch, int bg)
 {
-  static_assert(sizeof(ImgT) <= 2 && ImgT(-1) > ImgT(0), "probe_int reads unsigned 8- or 16-bit pixels");
-  const uint32_t ox = (uint32_t)x + (uint32_t)offset_of_num(int_div(px, dp), px);
-  const uint32_t oy = (uint32_t)y + (uint32_t)offset_of_num(int_div(py, dp), py);
+  static_assert(sizeof(ImgT) <= 2 && ImgT(-1) > ImgT(0), "probe_at reads unsigned 8- or 16-bit pixels");
   int v = bg;
   if (ox < (uint32_t)im.w && oy < (uint32_t)im.h) v = (int)im.at((int)ox, (int)oy, ch);
   return v;
 }
+
+// Offset parameters of a hook with a fast form (kFastParams below), converted
+// once per candidate or visited node.
+struct FastParams {
+  double p[4];
+  int ca, cb;
+};
+
+// A functor with
+//   static constexpr bool kFastParams = true;
+//   static FastParams fast_params(const FeatType *p);
+//   static FeatType eval_fast(view, x, y, Prep, const FastParams &);
+// gives eval_prep's result through eval_fast for parameters whose first four
+// entries are at most RECIP_MAX in magnitude; callers check that bound once per
+// launch (feature bounds) or per forest.
+template <class F, class = void>
+struct has_fast : std::false_type {};
+template <class F>
+struct has_fast<F, std::void_t<decltype(F::kFastParams)>> : std::integral_constant<bool, F::kFastParams> {};
 
 // C2/C3: uint16 depth in millimetres, float response; p in pixel*mm,
 // out-of-image reads 10000 mm, d(x) == 0 -> 0.
 struct DepthU16Feature {
   using ImgType = uint16_t;
   using FeatType = float;
-  using Prep = IntDivPrep;
+  using Prep = RecipPrep;
   static constexpr int nChannels = 1;
   static constexpr int FeatDim = 4;
   static constexpr int kind = 1;
   static constexpr int kProbeRowA = 1, kProbeRowB = 3;   // row offsets of the two probes
-  PD_HD static Prep prepare(const ImageView<uint16_t, 1> &im, int x, int y)
-  {
-    return int_div_prep((float)im.at(x, y, 0));
-  }
+  static constexpr bool kFastParams = true;
+  PD_HD static Prep prepare(const ImageView<uint16_t, 1> &im, int x, int y) { return recip_prep(im.at(x, y, 0)); }
+  // (a zero depth makes both offsets 0: the two probes read the same texel)
   PD_HD static float eval_prep(const ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const float *p)
   {
-    if (!(dp.d > 0.0f)) return 0.0f;
-    const int a = probe_int(im, x, y, dp, p[0], p[1], 0, 10000);
-    const int b = probe_int(im, x, y, dp, p[2], p[3], 0, 10000);
+    const int a = probe_at(im, recip_coord_any(x, p[0], dp), recip_coord_any(y, p[1], dp), 0, 10000);
+    const int b = probe_at(im, recip_coord_any(x, p[2], dp), recip_coord_any(y, p[3], dp), 0, 10000);
+    return (float)(a - b);
+  }
+  PD_HD static FastParams fast_params(const float *p)
+  {
+    return FastParams{{(double)p[0], (double)p[1], (double)p[2], (double)p[3]}, 0, 0};
+  }
+  PD_HD static float eval_fast(const ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const FastParams &f)
+  {
+    const int a = probe_at(im, recip_coord(x, f.p[0], dp), recip_coord(y, f.p[1], dp), 0, 10000);
+    const int b = probe_at(im, recip_coord(x, f.p[2], dp), recip_coord(y, f.p[3], dp), 0, 10000);
     return (float)(a - b);
   }
   PD_HD static float eval(const ImageView<uint16_t, 1> &im, int x, int y, const float *p)
@@ -257,7 +321,7 @@ struct DepthU16Feature {
 struct RGBDFeature {
   using ImgType = uint16_t;
   using FeatType = float;
-  using Prep = IntDivPrep;
+  using Prep = RecipPrep;
   static constexpr int nChannels = 4;
   static constexpr int FeatDim = 6;
   static constexpr int kind = 2;
@@ -268,15 +332,24 @@ struct RGBDFeature {
     if (c >= 3.0f) return 3;
     return (int)c;
   }
-  PD_HD static Prep prepare(const ImageView<uint16_t, 4> &im, int x, int y)
-  {
-    return int_div_prep((float)im.at(x, y, 3));
-  }
+  static constexpr bool kFastParams = true;
+  PD_HD static Prep prepare(const ImageView<uint16_t, 4> &im, int x, int y) { return recip_prep(im.at(x, y, 3)); }
   PD_HD static float eval_prep(const ImageView<uint16_t, 4> &im, int x, int y, Prep dp, const float *p)
   {
-    if (!(dp.d > 0.0f)) return 0.0f;
-    const int a = probe_int(im, x, y, dp, p[0], p[1], chan(p[4]), 10000);
-    const int b = probe_int(im, x, y, dp, p[2], p[3], chan(p[5]), 10000);
+    if (!(dp.y > 0.0)) return 0.0f;
+    const int a = probe_at(im, recip_coord_any(x, p[0], dp), recip_coord_any(y, p[1], dp), chan(p[4]), 10000);
+    const int b = probe_at(im, recip_coord_any(x, p[2], dp), recip_coord_any(y, p[3], dp), chan(p[5]), 10000);
+    return (float)(a - b);
+  }
+  PD_HD static FastParams fast_params(const float *p)
+  {
+    return FastParams{{(double)p[0], (double)p[1], (double)p[2], (double)p[3]}, chan(p[4]), chan(p[5])};
+  }
+  PD_HD static float eval_fast(const ImageView<uint16_t, 4> &im, int x, int y, Prep dp, const FastParams &f)
+  {
+    if (!(dp.y > 0.0)) return 0.0f;
+    const int a = probe_at(im, recip_coord(x, f.p[0], dp), recip_coord(y, f.p[1], dp), f.ca, 10000);
+    const int b = probe_at(im, recip_coord(x, f.p[2], dp), recip_coord(y, f.p[3], dp), f.cb, 10000);
     return (float)(a - b);
   }
   PD_HD static float eval(const ImageView<uint16_t, 4> &im, int x, int y, const float *p)

@@ -139,6 +139,17 @@ __device__ __forceinline__ typename F::FeatType hist_eval(const typename F::ImgT
   return eval_hook<F>(view, rec_x(r), rec_y(r), unpack_prep<typename F::Prep>(r.z, r.w), p, ac, rec_img(r));
 }
 
+// The same through the hook's fast form.
+template <class F>
+__device__ __forceinline__ typename F::FeatType hist_eval_fast(const typename F::ImgType *__restrict__ pixels,
+                                                               const ImgDesc *__restrict__ imgs, uint4 r,
+                                                               const FastParams &fp)
+{
+  const ImgDesc d = imgs[rec_img(r)];
+  ImageView<typename F::ImgType, F::nChannels> view{pixels + d.off, (int)d.w, (int)d.h};
+  return F::eval_fast(view, rec_x(r), rec_y(r), unpack_prep<typename F::Prep>(r.z, r.w), fp);
+}
+
 // Rank r = #{t : !(v <= thr_t)} of response v by a branch-free binary search
 // over the column's sorted thresholds (the predicate is true exactly on a
 // prefix of the sorted list; a NaN response makes it true everywhere), then
@@ -407,7 +418,7 @@ __global__ __launch_bounds__(NWAVES * 64) void k_hist(
     Bounds<F> bnd, uint32_t tree,
     uint32_t nF, uint32_t nT, uint32_t nC, uint32_t *__restrict__ H, unsigned long long *__restrict__ cand_key,
     uint32_t *__restrict__ cand_left, const uint32_t *__restrict__ cand_map, const uint16_t *__restrict__ perm,
-    const typename F::FeatType *__restrict__ ctab, AcArgs ac)
+    const typename F::FeatType *__restrict__ ctab, uint32_t fast, AcArgs ac)
 {
   using T = typename F::FeatType;
   constexpr int FD = F::FeatDim;
@@ -527,36 +538,45 @@ __global__ __launch_bounds__(NWAVES * 64) void k_hist(
   // thr_t; if v > thr_t then thr_t and every thr <= thr_t are below v, so
   // r(v) >= L_t + 1.
   const uint32_t end = it.begin + it.count;
-  if constexpr (SPW == 1) {
-    // two samples per wave and step, each wave-uniform (scalar record loads).
-    // (A variant with unpredicated probes that issued both samples' gathers
-    // before either bin update measured slower: the gathers are bound by
-    // throughput, not latency.)
-    uint32_t i = it.begin + wave;
-    for (; i + NW < end; i += 2 * NW) {
-      const uint4 ra = recs[i];
-      const uint4 rb = recs[i + NW];
-      hist_add<F, NTP, WIDE>(hist_eval<F>(pixels, imgs, ra, p, ac), __builtin_amdgcn_readfirstlane(rec_cls(ra) * CROW),
-                             sth, nT, fv, lane, bins);
-      hist_add<F, NTP, WIDE>(hist_eval<F>(pixels, imgs, rb, p, ac), __builtin_amdgcn_readfirstlane(rec_cls(rb) * CROW),
-                             sth, nT, fv, lane, bins);
+  auto scan_samples = [&](auto eval) {
+    if constexpr (SPW == 1) {
+      // two samples per wave and step, each wave-uniform (scalar record loads).
+      // (A variant with unpredicated probes that issued both samples' gathers
+      // before either bin update measured slower: the gathers are bound by
+      // throughput, not latency.)
+      uint32_t i = it.begin + wave;
+      for (; i + NW < end; i += 2 * NW) {
+        const uint4 ra = recs[i];
+        const uint4 rb = recs[i + NW];
+        hist_add<F, NTP, WIDE>(eval(ra), __builtin_amdgcn_readfirstlane(rec_cls(ra) * CROW), sth, nT, fv, lane, bins);
+        hist_add<F, NTP, WIDE>(eval(rb), __builtin_amdgcn_readfirstlane(rec_cls(rb) * CROW), sth, nT, fv, lane, bins);
+      }
+      if (i < end) {
+        const uint4 ra = recs[i];
+        hist_add<F, NTP, WIDE>(eval(ra), __builtin_amdgcn_readfirstlane(rec_cls(ra) * CROW), sth, nT, fv, lane, bins);
+      }
+    } else {
+      // SPW consecutive samples per wave step, one per group of FPW lanes
+      // (per-lane record loads; a lane past the chunk's end re-reads its first
+      // record and adds nothing)
+      for (uint32_t i = it.begin + wave * SPW; i < end; i += NW * SPW) {
+        const uint32_t s = i + sub;
+        const bool sv = s < end;
+        const uint4 r = recs[sv ? s : it.begin];
+        hist_add<F, NTP, WIDE, (int)FPW>(eval(r), rec_cls(r) * CROW, sth, nT, fv && sv, col, bins);
+      }
     }
-    if (i < end) {
-      const uint4 ra = recs[i];
-      hist_add<F, NTP, WIDE>(hist_eval<F>(pixels, imgs, ra, p, ac), __builtin_amdgcn_readfirstlane(rec_cls(ra) * CROW),
-                             sth, nT, fv, lane, bins);
+  };
+  // the hook's fast form where the launch's feature bounds allow it
+  if constexpr (has_fast<F>::value) {
+    if (fast) {
+      const FastParams fp = F::fast_params(p);
+      scan_samples([&](const uint4 &r) { return hist_eval_fast<F>(pixels, imgs, r, fp); });
+    } else {
+      scan_samples([&](const uint4 &r) { return hist_eval<F>(pixels, imgs, r, p, ac); });
     }
   } else {
-    // SPW consecutive samples per wave step, one per group of FPW lanes
-    // (per-lane record loads; a lane past the chunk's end re-reads its first
-    // record and adds nothing)
-    for (uint32_t i = it.begin + wave * SPW; i < end; i += NW * SPW) {
-      const uint32_t s = i + sub;
-      const bool sv = s < end;
-      const uint4 r = recs[sv ? s : it.begin];
-      hist_add<F, NTP, WIDE, (int)FPW>(hist_eval<F>(pixels, imgs, r, p, ac), rec_cls(r) * CROW, sth, nT, fv && sv,
-                                       col, bins);
-    }
+    scan_samples([&](const uint4 &r) { return hist_eval<F>(pixels, imgs, r, p, ac); });
   }
   __syncthreads();
 
@@ -1232,7 +1252,8 @@ static_assert(sizeof(FrameDesc) == 48, "frame table entries are 48 bytes");
 // Node records: while every active lane of a wave is at one node (the top
 // levels of a spatially coherent block) the record is read once through the
 // scalar cache instead of 64 lanes through the texture path.
-template <class F, int NCM>
+// FAST: every node's offset parameters allow the hook's fast form.
+template <class F, int NCM, bool FAST>
 __global__ __launch_bounds__(256) void k_predict(
     const typename F::ImgType *__restrict__ pixels, const FrameDesc *__restrict__ frames, uint32_t n_frames,
     uint32_t n_blocks, uint32_t n_xcc, uint32_t per_xcc, const uint8_t *__restrict__ masks,
@@ -1278,7 +1299,9 @@ __global__ __launch_bounds__(256) void k_predict(
           break;
         }
         // (auto-context hooks never come here: they predict through node maps)
-        const T v = eval_hook<F>(view, x, y, prep, rec.p, AcArgs{}, 0u);
+        T v;
+        if constexpr (FAST) v = F::eval_fast(view, x, y, prep, F::fast_params(rec.p));
+        else v = eval_hook<F>(view, x, y, prep, rec.p, AcArgs{}, 0u);
         n = rec.left + ((v <= rec.thr) ? 0 : 1);
       }
       const uint32_t li = leaf_off[t] + (uint32_t)leaf;

@@ -1002,3 +1002,48 @@ def test_pruned_split_search_equals_exhaustive(gpu, kind, n_classes, nF, nT, lev
     assert np.array_equal(diag["node_k"][trained], ref["node_k"][trained])
     assert diag["node_gain"][trained].tobytes() == ref["node_gain"][trained].tobytes()
     tr.close()
+
+
+@pytest.mark.parametrize("kind", [pa.PD_FEAT_DEPTH_U16, pa.PD_FEAT_RGBD_U16X4])
+@pytest.mark.parametrize("bound", [1000.0, 4194304.0, 4194308.0, 3e9])
+def test_fast_offset_form_equals_oracle(gpu, kind, bound):
+    """Offsets through one double FMA (feature bounds up to 2^22) and through
+    the general form (above): histograms, trees and leaf ids are the oracle's,
+    with depths for which half-integer quotients and offsets just inside and
+    outside the image occur (1, powers of two, small and the largest depths)."""
+    rng = np.random.default_rng(77)
+    w, h, n_classes = 45, 33, 3
+    ch = 4 if kind == pa.PD_FEAT_RGBD_U16X4 else 1
+    ts = pa.TrainingSet(n_classes)
+    for _ in range(2):
+        d = rng.choice(np.array([0, 1, 2, 3, 64, 128, 1000, 4096, 40000, 65535], np.uint16), (h, w))
+        im = d if ch == 1 else np.stack([rng.integers(0, 256, (h, w)).astype(np.uint16)] * 3 + [d], axis=-1)
+        lab = (1 + rng.integers(0, n_classes, (h, w))).astype(np.uint8)
+        smp = np.sort(rng.integers(0, w * h, 400)).astype(np.uint32)
+        ts << pa.TrainingSetImage(im, w, h, lab, n_classes, smp)
+    fd = L.FEATURES[kind][3]
+    lo, hi = [-bound] * fd, [bound] * fd
+    if ch == 4:
+        lo[4:], hi[4:] = [0.0, 0.0], [4.0, 4.0]
+    p = pa.TreeTrainerParameters(150, 6, lo, hi, -3000.0, 3000.0, 5)
+    tr = pa.HIPTreeTrainer(kind, n_classes)
+    tr.set_training_set(ts)
+    o = orc.Tset(kind, ts)
+    nodes = np.array([0, 4], dtype=np.int32)
+    sample_node = rng.choice([0, 4, -1], 800).astype(np.int32)
+    H = tr.hist_nodes(p, 2, nodes, sample_node)
+    assert np.array_equal(H, orc.hist_nodes(o, p, 2, nodes, sample_node))
+    tree = pa.Tree(2, 6, kind, n_classes)
+    tr.train(tree, ts, p, 1, 6)
+    ref = orc.train_tree(o, p, ts.priors, 2, 6)
+    assert np.array_equal(tree.left_children, ref["left_children"])
+    assert tree.features.tobytes() == ref["features"].tobytes()
+    assert tree.posteriors.tobytes() == ref["posteriors"].tobytes()
+    tr.close()
+    clf = pa.HIPClassifier(kind, n_classes)
+    clf << tree
+    im = ts.images[0]
+    got = clf.predict_leaves(0, im.data, w, h)
+    assert np.array_equal(got, orc.predict_leaves(kind, im.data.reshape(h, w, ch) if ch > 1 else im.data.reshape(h, w),
+                                                  None, tree).reshape(h, w))
+    clf.close()

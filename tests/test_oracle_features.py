@@ -76,3 +76,28 @@ def test_device_offset_rounding_equals_host_rule_exhaustively():
         host = np.where(q < np.float32(0.5), np.float32(0), np.trunc(q + np.float32(0.5)))
         dev = np.trunc(q + c)
         assert np.array_equal(host, dev), start
+
+
+def test_fast_coordinate_rule():
+    """x + round(p / d) as the low word of one FMA with the nudged reciprocal,
+    on the host: random, half-integer and just-below-half quotients over the
+    whole range of the fast form against exact integers (no GPU)."""
+    from fractions import Fraction
+    rng = np.random.default_rng(5)
+    d = np.concatenate([np.arange(1, 400), rng.integers(1, 65536, 3000), 2 ** np.arange(16), [65535]])
+    cases = []
+    for di in d.tolist():
+        n = int(rng.integers(0, 1 << 21)) % max(1, int(4194304 // di))
+        half = np.float32((n + 0.5) * di)
+        cases += [(half, di), (np.nextafter(half, np.float32(0)), di), (np.nextafter(half, np.float32(1e9)), di),
+                  (np.float32(rng.uniform(-4194304, 4194304)), di), (np.float32(-half), di)]
+    for p, di in cases:
+        if abs(p) > 4194304:
+            continue
+        y = Fraction((1.0 / di) * (1.0 + 2.0 ** -51))
+        s = Fraction(float(p)) * y                      # the FMA's exact product
+        got = int(np.sign(float(s))) * int(abs(s) + Fraction(1, 2)) if (abs(s) * 2).denominator != 1 else None
+        assert got is not None                          # never on a tie
+        q = np.float32(p) / np.float32(di)              # the feature's float quotient
+        want = int(np.sign(q)) * int(np.floor(np.float64(abs(q)) + 0.5))
+        assert got == want, (float(p), di)
