@@ -680,7 +680,13 @@ struct Trainer final : TrainerBase {
     if (chunk) return std::max<uint32_t>(64u, std::min<uint32_t>(chunk, 32768u));
     const uint64_t target_blocks = (uint64_t)cu_count * tune.blocks_per_cu;
     uint64_t c = (level_samples * ftiles + target_blocks - 1) / target_blocks;
-    c = std::max<uint64_t>(c, 1024u);
+    // at least 1024 samples an item (shorter ones pay for the candidate set-up
+    // and the histogram flush), down to 64 where the level would otherwise
+    // leave CUs without two items: a wave walks its samples one after the
+    // other, so a level of few items lasts as long as one of them (8192 samples
+    // x 100 candidates: 92 us a level in 16 items of 1024, 17 us in 256 of 64)
+    const uint64_t two_per_cu = level_samples * ftiles / (2u * (uint64_t)cu_count);
+    c = std::max<uint64_t>(c, std::min<uint64_t>(std::max<uint64_t>(two_per_cu, 64u), 1024u));
     c = std::min<uint64_t>(c, 32768u);
     return (uint32_t)c;
   }
@@ -823,8 +829,10 @@ struct Trainer final : TrainerBase {
         hslots.push_back(q);
       }
       for (uint32_t k = 0; k < chunks; k++) {
-        const uint32_t b = si.begin + k * ch;
-        const uint32_t c = cnt ? std::min(ch, cnt - k * ch) : 0u;
+        // equal shares (at most ch samples each)
+        const uint32_t o = (uint32_t)((uint64_t)cnt * k / chunks);
+        const uint32_t b = si.begin + o;
+        const uint32_t c = (uint32_t)((uint64_t)cnt * (k + 1) / chunks) - o;
         if (direct) {
           groups.push_back(uint4{q, b, c, 0u});
           continue;
@@ -838,14 +846,49 @@ struct Trainer final : TrainerBase {
     size_t n_items = 0;
     const HistItem *h_items = nullptr;
     if (direct) {
-      const size_t X = n_xcc, ng = groups.size(), rows = (ng + X - 1) / X;
-      n_items = rows * ftiles * X;
+      // Groups in node order, except that the smallest ones (a tenth of the
+      // samples together) come last, largest first, so that a level does not
+      // end on a long block; each goes to the XCD with the fewest samples so
+      // far.  Dealt round robin, one of 47 random-sized groups an XCD is some
+      // 8% above the mean; sorted by size throughout, the blocks resident on a
+      // CU run their gather-bound and their split phases at the same time.
+      // 351 nodes of 500..6000 samples, 2000 x 20 candidates: 5.7 -> 5.2 ms a
+      // level, 968 nodes 7.6 -> 6.8 ms (round robin -> this); sorted by size
+      // throughout, the histograms of a 16-level tree took 77.7 ms instead of 73.2
+      // (round robin 75.0).
+      const size_t X = n_xcc, ng = groups.size();
+      std::vector<uint32_t> order(ng), xcd(ng);
+      for (size_t g = 0; g < ng; g++) order[g] = (uint32_t)g;
+      uint64_t all = 0;
+      for (const uint4 &g : groups) all += g.z;
+      std::vector<uint32_t> by_size(order);
+      std::stable_sort(by_size.begin(), by_size.end(),
+                       [&](uint32_t x, uint32_t y) { return groups[x].z > groups[y].z; });
+      uint64_t rest = 0;
+      size_t cut = ng;   // by_size[cut..) come last
+      while (cut > 0 && rest + groups[by_size[cut - 1]].z <= all / 10) rest += groups[by_size[--cut]].z;
+      std::vector<uint8_t> last(ng, 0);
+      for (size_t i = cut; i < ng; i++) last[by_size[i]] = 1;
+      size_t w = 0;
+      for (size_t g = 0; g < ng; g++)
+        if (!last[g]) order[w++] = (uint32_t)g;
+      std::copy(by_size.begin() + cut, by_size.end(), order.begin() + w);
+      std::vector<uint64_t> load(X, 0), len(X, 0);
+      for (uint32_t g : order) {
+        const size_t x = std::min_element(load.begin(), load.end()) - load.begin();
+        xcd[g] = (uint32_t)x;
+        load[x] += groups[g].z + 64u;   // (a block costs something without samples too)
+        len[x] += ftiles;
+      }
+      n_items = *std::max_element(len.begin(), len.end()) * X;
       HistItem *pin = (HistItem *)stage.alloc(std::max<size_t>(n_items, 1) * sizeof(HistItem));
       std::fill(pin, pin + n_items, HistItem{NULL_SLOT, 0u, 0u, 0u});
-      for (size_t g = 0; g < ng; g++) {
+      std::fill(len.begin(), len.end(), 0);
+      for (uint32_t g : order) {
         const uint4 gr = groups[g];
-        HistItem *dst = pin + (g / X) * ftiles * X + g % X;
+        HistItem *dst = pin + len[xcd[g]] * X + xcd[g];
         for (uint32_t ft = 0; ft < ftiles; ft++) dst[(size_t)ft * X] = HistItem{gr.x, gr.y, gr.z, ft};
+        len[xcd[g]] += ftiles;
       }
       h_items = pin;
     } else {
