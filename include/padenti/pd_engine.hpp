@@ -461,10 +461,23 @@ struct Trainer final : TrainerBase {
   DevBuf d_pixels, d_imgs, d_recs;
   // level state
   DevBuf d_actA, d_actB, d_slotA, d_slotB;
-  DevBuf d_H, d_items, d_slot_node, d_slot_mode, d_slot_hidx, d_zero, d_tot, d_slot_h, d_best, d_res;
-  DevBuf d_cand_key, d_cand_left, d_hlist;
-  DevBuf d_tleft, d_tfeat, d_tthr, d_rslot_node, d_slot_next, d_cursor, d_ccount;
-  DevBuf d_flags, d_rank, d_sbegin, d_scan_tmp;
+  DevBuf d_H, d_out;
+  DevBuf d_cand_key, d_cand_left;
+  // a histogram slice's host tables on the device (one upload, see hist_slice)
+  struct SliceTables {
+    HistItem *items;              // work items in launch order
+    int32_t *slot_node;           // [ns]
+    int32_t *slot_hidx;           // [ns] H block of the slot, -1: searched in the kernel
+    uint8_t *slot_mode;           // [ns]
+    uint32_t *tot;                // [ns][nC]
+    float *slot_h;                // [ns] node entropy
+    uint32_t *zero;               // H blocks that several items add into
+    uint32_t *hlist;              // slot of each H block
+    unsigned long long *best;     // [ns] split keys, uploaded as zeros
+  } sl{};
+  DevBuf d_slice, d_route;
+  DevBuf d_tleft, d_tfeat, d_tthr, d_ccount;
+  DevBuf d_flags, d_rank, d_scan_tmp;
   // auto-context hooks: node-id maps of every image (two buffers), the
   // pixels that are routed (labelled), map offsets, the tree's posteriors
   DevBuf d_acmapA, d_acmapB, d_acsel, d_acoff, d_acblk, d_tpost;
@@ -496,6 +509,48 @@ struct Trainer final : TrainerBase {
     if (bytes) std::copy((const char *)pin, (const char *)pin + bytes, (char *)dst);
     stage.reset();
   }
+  // Several host arrays uploaded as one: each add() reserves a 16-byte aligned
+  // piece, commit() copies the whole staging to the device buffer and at()
+  // gives a piece's device address (a small copy costs about 3 us of the GPU's
+  // time and as much of the host's).
+  struct Upload {
+    Trainer &t;
+    DevBuf &dst;
+    std::vector<std::pair<const void *, size_t>> src;   // source (null: left to the caller), bytes
+    std::vector<size_t> off;
+    size_t bytes = 0;
+    char *pin = nullptr;
+    size_t add(const void *p, size_t n)
+    {
+      src.push_back({p, n});
+      off.push_back(bytes);
+      bytes += (n + 15) & ~(size_t)15;
+      return off.size() - 1;
+    }
+    // pinned staging with the sources copied in (pieces without one: host())
+    void stage()
+    {
+      dst.grow(std::max<size_t>(bytes, 16));
+      pin = (char *)t.stage.alloc(std::max<size_t>(bytes, 16));
+      for (size_t i = 0; i < src.size(); i++)
+        if (src[i].first && src[i].second) std::memcpy(pin + off[i], src[i].first, src[i].second);
+    }
+    void commit()
+    {
+      if (bytes) HIPCHK(hipMemcpyAsync(dst.p, pin, bytes, hipMemcpyHostToDevice, t.stream));
+    }
+    template <class T2>
+    T2 *host(size_t i) const
+    {
+      return (T2 *)(pin + off[i]);
+    }
+    template <class T2>
+    T2 *at(size_t i) const
+    {
+      return (T2 *)((char *)dst.p + off[i]);
+    }
+  };
+
   DevBuf d_sub_act, d_sub_idx, d_sub_cls, d_sub_sel, d_map2;
   DevBuf d_st_flags, d_st_pos, d_st_tmp, d_st_meta, d_st_rate, d_st_tot;
   DevBuf d_frac, d_gmax, d_ynet, d_score, d_score2, d_net_sel, d_full, d_gbest, d_top, d_ebase, d_eslots;
@@ -746,9 +801,8 @@ struct Trainer final : TrainerBase {
       HIPCHK(hipFuncSetAttribute((const void *)k_hist<F, NTP, NW, WIDE, SPW>,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_hist<F, NTP, NW, WIDE, SPW>), dim3(n_items), dim3(NW * 64), lds, stream, d_pixels.as<I>(),
-                       d_imgs.as<ImgDesc>(), act, d_items.as<HistItem>(), item_base, d_slot_node.as<int32_t>(),
-                       d_slot_mode.as<uint8_t>(), d_slot_hidx.as<int32_t>(), d_tot.as<uint32_t>(),
-                       d_slot_h.as<float>(), bnd, tree, nF,
+                       d_imgs.as<ImgDesc>(), act, sl.items, item_base, sl.slot_node, sl.slot_mode, sl.slot_hidx, sl.tot,
+                       sl.slot_h, bnd, tree, nF,
                        nT, nC, d_H.as<uint32_t>(), d_cand_key.as<unsigned long long>(), d_cand_left.as<uint32_t>(),
                        d_map_cur, d_perm_cur, d_ctab_cur, fast_bounds(bnd) ? 1u : 0u, ac);
     HIPCHK(hipGetLastError());
@@ -844,7 +898,7 @@ struct Trainer final : TrainerBase {
     }
     // direct: the items are written into pinned staging and copied from there
     size_t n_items = 0;
-    const HistItem *h_items = nullptr;
+    std::vector<uint32_t> order, xcd;   // launch order of the groups and their XCDs (direct)
     if (direct) {
       // Groups in node order, except that the smallest ones (a tenth of the
       // samples together) come last, largest first, so that a level does not
@@ -857,7 +911,8 @@ struct Trainer final : TrainerBase {
       // throughout, the histograms of a 16-level tree took 77.7 ms instead of 73.2
       // (round robin 75.0).
       const size_t X = n_xcc, ng = groups.size();
-      std::vector<uint32_t> order(ng), xcd(ng);
+      order.resize(ng);
+      xcd.resize(ng);
       for (size_t g = 0; g < ng; g++) order[g] = (uint32_t)g;
       uint64_t all = 0;
       for (const uint4 &g : groups) all += g.z;
@@ -881,56 +936,53 @@ struct Trainer final : TrainerBase {
         len[x] += ftiles;
       }
       n_items = *std::max_element(len.begin(), len.end()) * X;
-      HistItem *pin = (HistItem *)stage.alloc(std::max<size_t>(n_items, 1) * sizeof(HistItem));
-      std::fill(pin, pin + n_items, HistItem{NULL_SLOT, 0u, 0u, 0u});
-      std::fill(len.begin(), len.end(), 0);
-      for (uint32_t g : order) {
-        const uint4 gr = groups[g];
-        HistItem *dst = pin + len[xcd[g]] * X + xcd[g];
-        for (uint32_t ft = 0; ft < ftiles; ft++) dst[(size_t)ft * X] = HistItem{gr.x, gr.y, gr.z, ft};
-        len[xcd[g]] += ftiles;
-      }
-      h_items = pin;
     } else {
       item_start[ns] = (uint32_t)items.size();
       group_start.push_back((uint32_t)items.size());
       if (mode == PD_MODE_LEVEL_BATCHED) xcd_order(items, group_start, group_pos);
       n_items = items.size();
-      h_items = items.data();
     }
-    d_items.grow(std::max<size_t>(n_items, 1) * sizeof(HistItem));
-    d_slot_node.grow(ns * sizeof(int32_t));
-    d_slot_mode.grow(ns);
-    d_slot_hidx.grow(ns * sizeof(int32_t));
-    d_tot.grow((size_t)ns * nC * sizeof(uint32_t));
     d_H.grow(per * std::max<size_t>(hslots.size(), 1) * sizeof(uint32_t), hist_budget);
     d_cand_key.grow((size_t)ns * ftiles * sizeof(unsigned long long));
     d_cand_left.grow((size_t)ns * ftiles * nC * sizeof(uint32_t));
-    if (direct) {
-      if (n_items)
-        HIPCHK(hipMemcpyAsync(d_items.p, h_items, n_items * sizeof(HistItem), hipMemcpyHostToDevice, stream));
-    } else {
-      h2d(d_items.p, h_items, n_items * sizeof(HistItem));
-    }
-    h2d(d_slot_node.p, snode.data(), ns * sizeof(int32_t));
-    h2d(d_slot_mode.p, smode.data(), ns);
-    h2d(d_slot_hidx.p, shidx.data(), ns * sizeof(int32_t));
-    h2d(d_tot.p, tot.data(), (size_t)ns * nC * sizeof(uint32_t));
     std::vector<float> sh(ns);
     for (uint32_t q = 0; q < ns; q++) sh[q] = slot_entropy(&tot[(size_t)q * nC], nC);
-    d_slot_h.grow(ns * sizeof(float));
-    h2d(d_slot_h.p, sh.data(), ns * sizeof(float));
-    if (!zero.empty()) {
-      d_zero.grow(zero.size() * sizeof(uint32_t));
-      h2d(d_zero.p, zero.data(), zero.size() * sizeof(uint32_t));
+    Upload up{*this, d_slice};
+    const size_t u_items = up.add(direct ? nullptr : items.data(), n_items * sizeof(HistItem));
+    const size_t u_node = up.add(snode.data(), ns * sizeof(int32_t));
+    const size_t u_hidx = up.add(shidx.data(), ns * sizeof(int32_t));
+    const size_t u_mode = up.add(smode.data(), ns);
+    const size_t u_tot = up.add(tot.data(), (size_t)ns * nC * sizeof(uint32_t));
+    const size_t u_h = up.add(sh.data(), ns * sizeof(float));
+    const size_t u_zero = up.add(zero.data(), zero.size() * sizeof(uint32_t));
+    const size_t u_list = up.add(hslots.data(), hslots.size() * sizeof(uint32_t));
+    const std::vector<uint64_t> no_key(ns, 0ull);
+    const size_t u_best = up.add(no_key.data(), ns * sizeof(uint64_t));
+    up.stage();
+    if (direct) {
+      HistItem *it = up.template host<HistItem>(u_items);
+      std::fill(it, it + n_items, HistItem{NULL_SLOT, 0u, 0u, 0u});
+      std::vector<uint64_t> len(n_xcc, 0);
+      for (uint32_t g : order) {
+        const uint4 gr = groups[g];
+        HistItem *dst = it + len[xcd[g]] * n_xcc + xcd[g];
+        for (uint32_t ft = 0; ft < ftiles; ft++) dst[(size_t)ft * n_xcc] = HistItem{gr.x, gr.y, gr.z, ft};
+        len[xcd[g]] += ftiles;
+      }
     }
+    up.commit();
+    sl = SliceTables{up.template at<HistItem>(u_items), up.template at<int32_t>(u_node),
+                     up.template at<int32_t>(u_hidx),   up.template at<uint8_t>(u_mode),
+                     up.template at<uint32_t>(u_tot),   up.template at<float>(u_h),
+                     up.template at<uint32_t>(u_zero),  up.template at<uint32_t>(u_list),
+                     up.template at<unsigned long long>(u_best)};
     d_perm_cur = nullptr;
     if constexpr (probe_rows<F>::on) {
       if (probe_order && nF > 64 && nF <= 65536u) {
         d_perm.grow((size_t)ns * nF * sizeof(uint16_t));
         const uint32_t segs = (nF + ORDER_MAX - 1) / ORDER_MAX;
         hipLaunchKernelGGL((k_cand_order<F>), dim3(ns, segs), dim3(ORDER_THREADS), 0, stream, tree,
-                           d_slot_node.as<int32_t>(), nF, bnd, d_map_cur, d_perm.as<uint16_t>());
+                           sl.slot_node, nF, bnd, d_map_cur, d_perm.as<uint16_t>());
         HIPCHK(hipGetLastError());
         d_perm_cur = d_perm.as<uint16_t>();
       }
@@ -949,7 +1001,7 @@ struct Trainer final : TrainerBase {
         ctab_elems * sizeof(T) <= cand_table_budget) {
       const uint64_t n_thr = (uint64_t)ns * ftiles * fpw;
       hipLaunchKernelGGL((k_cand_table<F>), dim3((uint32_t)((n_thr + 255) / 256)), dim3(256), 0, stream, tree,
-                         d_slot_node.as<int32_t>(), ns, nF, nT, fpw, ftiles, bnd, d_map_cur, d_perm_cur,
+                         sl.slot_node, ns, nF, nT, fpw, ftiles, bnd, d_map_cur, d_perm_cur,
                          d_ctab.as<T>());
       HIPCHK(hipGetLastError());
       d_ctab_cur = d_ctab.as<T>();
@@ -958,7 +1010,7 @@ struct Trainer final : TrainerBase {
       const size_t total = zero.size() * per;
       const uint32_t blocks = (uint32_t)std::min<size_t>((total + 255) / 256, (size_t)cu_count * 64);
       hipLaunchKernelGGL(k_zero_slots, dim3(blocks), dim3(256), 0, stream, d_H.as<uint32_t>(),
-                         d_zero.as<uint32_t>(), (uint32_t)zero.size(), per);
+                         sl.zero, (uint32_t)zero.size(), per);
       HIPCHK(hipGetLastError());
     }
     uint32_t launches = 0;
@@ -982,9 +1034,17 @@ struct Trainer final : TrainerBase {
     return launches;
   }
 
-  // Split search over the H blocks: block i belongs to slot hlist[i].
+  // Split search over the nh H blocks of the current slice (block i belongs to
+  // slot sl.hlist[i]).
+  void launch_split(uint32_t nh, uint32_t nT, uint32_t nF, int mode, float *all_gains)
+  {
+    if (nC <= 8) launch_split_t<8>(nh, nT, nF, mode, all_gains);
+    else if (nC <= 16) launch_split_t<16>(nh, nT, nF, mode, all_gains);
+    else if (nC <= 32) launch_split_t<32>(nh, nT, nF, mode, all_gains);
+    else launch_split_t<64>(nh, nT, nF, mode, all_gains);
+  }
   template <int NCM>
-  void launch_split_t(uint32_t nh, const uint32_t *d_list, uint32_t nT, uint32_t nF, int mode, float *all_gains)
+  void launch_split_t(uint32_t nh, uint32_t nT, uint32_t nF, int mode, float *all_gains)
   {
     const uint32_t npairs = nT * nF;
     const uint32_t ppb = SPLIT_THREADS * 8;
@@ -992,14 +1052,12 @@ struct Trainer final : TrainerBase {
     const size_t per = (size_t)nC * npairs;
     if (mode == PD_MODE_LEVEL_BATCHED) {
       hipLaunchKernelGGL((k_split<NCM>), dim3(nh * bps), dim3(SPLIT_THREADS), 0, stream, d_H.as<uint32_t>(),
-                         d_tot.as<uint32_t>(), nC, nT, nF, bps, ppb, d_best.as<unsigned long long>(), all_gains,
-                         d_list);
+                         sl.tot, nC, nT, nF, bps, ppb, sl.best, all_gains, sl.hlist);
       HIPCHK(hipGetLastError());
     } else {
       for (uint32_t i = 0; i < nh; i++) {
         hipLaunchKernelGGL((k_split<NCM>), dim3(bps), dim3(SPLIT_THREADS), 0, stream, d_H.as<uint32_t>() + i * per,
-                           d_tot.as<uint32_t>(), nC, nT, nF, bps, ppb, d_best.as<unsigned long long>(), all_gains,
-                           d_list + i);
+                           sl.tot, nC, nT, nF, bps, ppb, sl.best, all_gains, sl.hlist + i);
         HIPCHK(hipGetLastError());
       }
     }
@@ -1011,7 +1069,6 @@ struct Trainer final : TrainerBase {
   // winners' parameters and thresholds of the slots of a level, filled by
   // split_slice through evaluate when set (train() sets them per level)
   std::vector<T> *lvl_par = nullptr, *lvl_thr = nullptr;
-  DevBuf d_wpar, d_wthr;
 
   // With `win` (the slice's candidate map, tree and bounds) the winners'
   // parameters and thresholds come back too (wpar [ns][FD], wthr [ns]).
@@ -1025,46 +1082,32 @@ struct Trainer final : TrainerBase {
                    std::vector<uint32_t> &res_out, float *all_gains = nullptr, const WinnerArgs *win = nullptr)
   {
     const uint32_t nh = (uint32_t)hslots.size();
-    d_best.grow((size_t)ns * sizeof(uint64_t));
-    d_res.grow((size_t)ns * (nC + 2) * sizeof(uint32_t));
-    d_hlist.grow(std::max<size_t>(nh, 1) * sizeof(uint32_t));
-    HIPCHK(hipMemsetAsync(d_best.p, 0, (size_t)ns * sizeof(uint64_t), stream));
-    if (nh) {
-      h2d(d_hlist.p, hslots.data(), nh * sizeof(uint32_t));
-      const uint32_t *dl = d_hlist.as<uint32_t>();
-      if (nC <= 8) launch_split_t<8>(nh, dl, nT, nF, mode, all_gains);
-      else if (nC <= 16) launch_split_t<16>(nh, dl, nT, nF, mode, all_gains);
-      else if (nC <= 32) launch_split_t<32>(nh, dl, nT, nF, mode, all_gains);
-      else launch_split_t<64>(nh, dl, nT, nF, mode, all_gains);
-    }
+    if (nh) launch_split(nh, nT, nF, mode, all_gains);
+    // one device buffer, one copy back: res [ns][nC + 2], then (with win) the
+    // winners' parameters [ns][FD] and thresholds [ns]
+    const size_t br = (size_t)ns * (nC + 2) * sizeof(uint32_t), o_par = (br + 15) & ~(size_t)15;
+    const size_t bp = (size_t)ns * FD * sizeof(T), o_thr = (o_par + bp + 15) & ~(size_t)15;
+    const size_t bt = ns * sizeof(T), bytes = win ? o_thr + bt : br;
+    d_out.grow(std::max<size_t>(bytes, 16));
+    char *dev = d_out.as<char>();
     const uint32_t threads = ns * (nC + 2);
-    hipLaunchKernelGGL(k_finalize, dim3((threads + 255) / 256), dim3(256), 0, stream, d_H.as<uint32_t>(),
-                       d_best.as<unsigned long long>(), d_slot_mode.as<uint8_t>(), d_slot_hidx.as<int32_t>(),
-                       d_cand_key.as<unsigned long long>(), d_cand_left.as<uint32_t>(), ns, nC, nT, nF,
-                       hist_fpw(nT), d_res.as<uint32_t>());
+    hipLaunchKernelGGL((k_finalize<F>), dim3((threads + 255) / 256), dim3(256), 0, stream, d_H.as<uint32_t>(), sl.best,
+                       sl.slot_mode, sl.slot_hidx, d_cand_key.as<unsigned long long>(), d_cand_left.as<uint32_t>(), ns,
+                       nC, nT, nF, hist_fpw(nT), (uint32_t *)dev, win ? win->tree : 0u, sl.slot_node,
+                       win ? win->d_map : nullptr, win ? *win->bnd : Bounds<F>{}, win ? (T *)(dev + o_par) : nullptr,
+                       win ? (T *)(dev + o_thr) : nullptr);
     HIPCHK(hipGetLastError());
-    res_out.resize((size_t)ns * (nC + 2));
-    if (!win) {
-      d2h_sync(res_out.data(), d_res.p, res_out.size() * sizeof(uint32_t));
-      return;
-    }
-    d_wpar.grow((size_t)ns * FD * sizeof(T));
-    d_wthr.grow((size_t)ns * sizeof(T));
-    hipLaunchKernelGGL((k_winner_params<F>), dim3((ns + 255) / 256), dim3(256), 0, stream, win->tree,
-                       d_slot_node.as<int32_t>(), d_res.as<uint32_t>(), ns, nC, nF, win->d_map, *win->bnd,
-                       d_wpar.as<T>(), d_wthr.as<T>());
-    HIPCHK(hipGetLastError());
-    win->wpar->resize((size_t)ns * FD);
-    win->wthr->resize(ns);
-    const size_t br = res_out.size() * sizeof(uint32_t), bp = (size_t)ns * FD * sizeof(T), bt = ns * sizeof(T);
-    void *pr = stage.alloc(br), *pp = stage.alloc(bp), *pt = stage.alloc(bt);
-    HIPCHK(hipMemcpyAsync(pr, d_res.p, br, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipMemcpyAsync(pp, d_wpar.p, bp, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipMemcpyAsync(pt, d_wthr.p, bt, hipMemcpyDeviceToHost, stream));
+    char *pin = (char *)stage.alloc(std::max<size_t>(bytes, 16));
+    if (bytes) HIPCHK(hipMemcpyAsync(pin, dev, bytes, hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
-    std::copy((const char *)pr, (const char *)pr + br, (char *)res_out.data());
-    std::copy((const char *)pp, (const char *)pp + bp, (char *)win->wpar->data());
-    std::copy((const char *)pt, (const char *)pt + bt, (char *)win->wthr->data());
+    res_out.resize((size_t)ns * (nC + 2));
+    std::copy(pin, pin + br, (char *)res_out.data());
+    if (win) {
+      win->wpar->resize((size_t)ns * FD);
+      win->wthr->resize(ns);
+      std::copy(pin + o_par, pin + o_par + bp, (char *)win->wpar->data());
+      std::copy(pin + o_thr, pin + o_thr + bt, (char *)win->wthr->data());
+    }
     stage.reset();
   }
 
@@ -1250,15 +1293,7 @@ struct Trainer final : TrainerBase {
     d_map_cur = nullptr;
     const uint32_t nh = (uint32_t)hslots.size();
     d_full.ensure((size_t)ns * screen * sizeof(float));
-    d_best.ensure((size_t)ns * sizeof(uint64_t));
-    d_hlist.ensure(std::max<size_t>(nh, 1) * sizeof(uint32_t));
-    HIPCHK(hipMemsetAsync(d_best.p, 0, (size_t)ns * sizeof(uint64_t), stream));
-    h2d(d_hlist.p, hslots.data(), nh * sizeof(uint32_t));
-    const uint32_t *dl = d_hlist.as<uint32_t>();
-    if (nC <= 8) launch_split_t<8>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_full.as<float>());
-    else if (nC <= 16) launch_split_t<16>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_full.as<float>());
-    else if (nC <= 32) launch_split_t<32>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_full.as<float>());
-    else launch_split_t<64>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_full.as<float>());
+    launch_split(nh, 1, screen, PD_MODE_LEVEL_BATCHED, d_full.as<float>());
     d_gbest.ensure((size_t)ns * sizeof(float));
     hipLaunchKernelGGL(k_slot_max, dim3(ns), dim3(256), 0, stream, d_full.as<float>(), screen, d_gbest.as<float>());
     // the best half-R estimates of every emitting slot
@@ -1513,15 +1548,7 @@ struct Trainer final : TrainerBase {
         }
       } else {
         const uint32_t nh = (uint32_t)hslots.size();
-        d_best.ensure((size_t)ns * sizeof(uint64_t));
-        d_hlist.ensure(std::max<size_t>(nh, 1) * sizeof(uint32_t));
-        HIPCHK(hipMemsetAsync(d_best.p, 0, (size_t)ns * sizeof(uint64_t), stream));
-        h2d(d_hlist.p, hslots.data(), nh * sizeof(uint32_t));
-        const uint32_t *dl = d_hlist.as<uint32_t>();
-        if (nC <= 8) launch_split_t<8>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_gains.as<float>());
-        else if (nC <= 16) launch_split_t<16>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_gains.as<float>());
-        else if (nC <= 32) launch_split_t<32>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_gains.as<float>());
-        else launch_split_t<64>(nh, dl, 1, screen, PD_MODE_LEVEL_BATCHED, d_gains.as<float>());
+        launch_split(nh, 1, screen, PD_MODE_LEVEL_BATCHED, d_gains.as<float>());
       }
       d_sub_sel.ensure((size_t)ns * keep * sizeof(uint32_t));
       hipLaunchKernelGGL(mlp::k_topk, dim3(ns), dim3(256), 0, stream, rank, screen, keep, keep,
@@ -1670,9 +1697,6 @@ struct Trainer final : TrainerBase {
     nodeTot[0] = (uint32_t)S;
     std::copy(root_tot.begin(), root_tot.end(), classTot.begin());
 
-    d_tleft.ensure(N * sizeof(int32_t));
-    d_tfeat.ensure(N * FD * sizeof(T));
-    d_tthr.ensure(N * sizeof(T));
     d_actA.ensure(S * sizeof(uint4));
     d_actB.ensure(S * sizeof(uint4));
     d_slotA.ensure(S * sizeof(uint32_t));
@@ -1686,6 +1710,9 @@ struct Trainer final : TrainerBase {
     if constexpr (uses_context<F>::value) {
       // the device tree mirrors the host one: all -2, root posterior = priors;
       // every labelled pixel starts at the root
+      d_tleft.ensure(N * sizeof(int32_t));
+      d_tfeat.ensure(N * FD * sizeof(T));
+      d_tthr.ensure(N * sizeof(T));
       d_tpost.ensure(N * nC * sizeof(float));
       hipLaunchKernelGGL(k_fill_i32, dim3((uint32_t)std::min<size_t>((N + 255) / 256, 65535)), dim3(256), 0, stream,
                          d_tleft.as<int32_t>(), (uint64_t)N, -2);
@@ -1814,15 +1841,15 @@ struct Trainer final : TrainerBase {
         if (ls) ls[d - 1] = st;
         break;
       }
-      // upload this level's node range for routing
-      const size_t lv0 = ((size_t)1 << (d - 1)) - 1, lvn = (size_t)1 << (d - 1);
-      h2d(d_tleft.as<int32_t>() + lv0, left + lv0, lvn * sizeof(int32_t));
-      h2d(d_tfeat.as<T>() + lv0 * FD, feats + lv0 * FD, lvn * FD * sizeof(T));
-      h2d(d_tthr.as<T>() + lv0, thrs + lv0, lvn * sizeof(T));
       if constexpr (uses_context<F>::value) {
-        // the children (next level) as the hook will read them: leftChild -1
-        // and their posteriors (the reference's device copy reads the
-        // posteriors from the wrong offset, _learn_best_featthr.hpp:270-274)
+        // the device tree a hook reads: this level's nodes and the children
+        // (next level) as the hook will read them: leftChild -1 and their
+        // posteriors (the reference's device copy reads the posteriors from
+        // the wrong offset, _learn_best_featthr.hpp:270-274)
+        const size_t lv0 = ((size_t)1 << (d - 1)) - 1, lvn = (size_t)1 << (d - 1);
+        h2d(d_tleft.as<int32_t>() + lv0, left + lv0, lvn * sizeof(int32_t));
+        h2d(d_tfeat.as<T>() + lv0 * FD, feats + lv0 * FD, lvn * FD * sizeof(T));
+        h2d(d_tthr.as<T>() + lv0, thrs + lv0, lvn * sizeof(T));
         const size_t c0 = lv0 + lvn, cn = std::min(2 * lvn, N - c0);
         h2d(d_tleft.as<int32_t>() + c0, left + c0, cn * sizeof(int32_t));
         h2d(d_tpost.as<float>() + c0 * nC, post + c0 * nC, cn * nC * sizeof(float));
@@ -1835,11 +1862,10 @@ struct Trainer final : TrainerBase {
       // next frontier (children with more than perLeafSamplesThr samples,
       // _impl_init.hpp:343-355), in node order
       std::vector<SlotInfo> next;
-      std::vector<int32_t> snext(2 * slots.size(), -1), rnode(slots.size());
+      std::vector<int32_t> snext(2 * slots.size(), -1);
       std::vector<uint32_t> nbegin;   // first entry of each next slot
       uint32_t run = 0;
       for (size_t q = 0; q < slots.size(); q++) {
-        rnode[q] = slots[q].node;
         if (!split_flag[q]) continue;
         for (int side = 0; side < 2; side++) {
           const int32_t ch_node = 2 * slots[q].node + 1 + side;
@@ -1856,17 +1882,18 @@ struct Trainer final : TrainerBase {
       std::vector<uint32_t> sbegin(nq + 1);
       for (uint32_t q = 0; q < nq; q++) sbegin[q] = slots[q].begin;
       sbegin[nq] = (uint32_t)n_act;
-      d_rslot_node.ensure(nq * sizeof(int32_t));
-      d_slot_next.ensure(2 * (size_t)nq * sizeof(int32_t));
-      d_ccount.ensure(2 * (size_t)nq * sizeof(uint32_t));
-      d_cursor.ensure(std::max<size_t>(nbegin.size(), 1) * sizeof(uint32_t));
-      d_sbegin.ensure((nq + 1) * sizeof(uint32_t));
+      d_ccount.grow(2 * (size_t)nq * sizeof(uint32_t));
       d_flags.ensure((n_act + 1) * sizeof(unsigned long long));
       d_rank.ensure((n_act + 1) * sizeof(unsigned long long));
-      h2d(d_rslot_node.p, rnode.data(), nq * sizeof(int32_t));
-      h2d(d_slot_next.p, snext.data(), 2 * (size_t)nq * sizeof(int32_t));
-      h2d(d_sbegin.p, sbegin.data(), (nq + 1) * sizeof(uint32_t));
-      h2d(d_cursor.p, nbegin.data(), nbegin.size() * sizeof(uint32_t));
+      // the level's splits by slot, in one upload
+      Upload up{*this, d_route};
+      const size_t u_split = up.add(split_flag.data(), nq), u_par = up.add(win_par.data(), (size_t)nq * FD * sizeof(T));
+      const size_t u_thr = up.add(win_thr.data(), nq * sizeof(T));
+      const size_t u_next = up.add(snext.data(), 2 * (size_t)nq * sizeof(int32_t));
+      const size_t u_begin = up.add(sbegin.data(), (nq + 1) * sizeof(uint32_t));
+      const size_t u_cursor = up.add(nbegin.data(), nbegin.size() * sizeof(uint32_t));
+      up.stage();
+      up.commit();
       size_t tmp_bytes = 0;
       HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, d_flags.as<unsigned long long>(),
                                               d_rank.as<unsigned long long>(), (int)(n_act + 1), stream));
@@ -1874,20 +1901,17 @@ struct Trainer final : TrainerBase {
       HIPCHK(hipEventRecord(e3.e, stream));
       const uint32_t nb = (uint32_t)((n_act + 1 + 255) / 256);
       hipLaunchKernelGGL((k_route_flags<F>), dim3(nb), dim3(256), 0, stream, d_pixels.as<I>(), d_imgs.as<ImgDesc>(),
-                         act, aslot, (uint32_t)n_act, d_rslot_node.as<int32_t>(), d_tleft.as<int32_t>(),
-                         d_tfeat.as<T>(), d_tthr.as<T>(), d_flags.as<unsigned long long>(), ac);
+                         act, aslot, (uint32_t)n_act, up.template at<uint8_t>(u_split), up.template at<T>(u_par),
+                         up.template at<T>(u_thr), d_flags.as<unsigned long long>(), ac);
       HIPCHK(hipGetLastError());
       HIPCHK(hipcub::DeviceScan::ExclusiveSum(d_scan_tmp.p, tmp_bytes, d_flags.as<unsigned long long>(),
                                               d_rank.as<unsigned long long>(), (int)(n_act + 1), stream));
-      if (n_act) {
-        hipLaunchKernelGGL(k_route_scatter, dim3((uint32_t)((n_act + 255) / 256)), dim3(256), 0, stream, act, aslot,
-                           (uint32_t)n_act, d_flags.as<unsigned long long>(), d_rank.as<unsigned long long>(),
-                           d_sbegin.as<uint32_t>(), d_slot_next.as<int32_t>(), d_cursor.as<uint32_t>(), act_next,
-                           aslot_next, (uint32_t)S);
-        HIPCHK(hipGetLastError());
-      }
-      hipLaunchKernelGGL(k_route_counts, dim3((nq + 255) / 256), dim3(256), 0, stream, d_rank.as<unsigned long long>(),
-                         d_sbegin.as<uint32_t>(), nq, d_ccount.as<uint32_t>());
+      const uint64_t ts = std::max<uint64_t>(n_act, nq);
+      hipLaunchKernelGGL(k_route_scatter, dim3((uint32_t)((ts + 255) / 256)), dim3(256), 0, stream, act, aslot,
+                         (uint32_t)n_act, d_flags.as<unsigned long long>(), d_rank.as<unsigned long long>(),
+                         up.template at<uint32_t>(u_begin), up.template at<int32_t>(u_next),
+                         up.template at<uint32_t>(u_cursor), act_next, aslot_next, (uint32_t)S, nq,
+                         d_ccount.as<uint32_t>());
       HIPCHK(hipGetLastError());
       HIPCHK(hipEventRecord(e4.e, stream));
       {

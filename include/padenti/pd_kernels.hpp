@@ -1069,13 +1069,20 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_split(const uint32_t *__restr
 // Winner of each slot: res[slot] = {k, gain bits, left[0..nC)}.  A fused
 // slot takes the largest key over its tiles' candidates (larger gain, then
 // smaller k) and that tile's left counts; any other slot its searched key
-// and the counts of H block slot_hidx[slot].
+// and the counts of H block slot_hidx[slot].  With par / thr, also the winner's
+// feature parameters and threshold, re-derived from the sampler for the tree
+// arrays (f mapped through cand_map when given; the reference re-derives them
+// on the host, cl_tree_trainer_impl_learn_best_featthr.hpp:183-222).
+template <class F>
 __global__ void k_finalize(const uint32_t *__restrict__ H, const unsigned long long *__restrict__ best,
                            const uint8_t *__restrict__ slot_mode, const int32_t *__restrict__ slot_hidx,
                            const unsigned long long *__restrict__ cand_key, const uint32_t *__restrict__ cand_left,
                            uint32_t n_slots, uint32_t nC, uint32_t nT, uint32_t nF, uint32_t fpw,
-                           uint32_t *__restrict__ res)
+                           uint32_t *__restrict__ res, uint32_t tree, const int32_t *__restrict__ slot_node,
+                           const uint32_t *__restrict__ cand_map, Bounds<F> bnd,
+                           typename F::FeatType *__restrict__ par, typename F::FeatType *__restrict__ thr)
 {
+  using T = typename F::FeatType;
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t slot = i / (nC + 2), c = i % (nC + 2);
   if (slot >= n_slots) return;
@@ -1100,6 +1107,15 @@ __global__ void k_finalize(const uint32_t *__restrict__ H, const unsigned long l
   uint32_t *r = res + (size_t)slot * (nC + 2);
   if (c == 0) {
     r[0] = k;
+    if (par) {
+      const uint32_t f = k % nF;
+      const uint32_t fs = cand_map ? cand_map[(size_t)slot * nF + f] : f;
+      const uint32_t node = (uint32_t)slot_node[slot];
+      T p[F::FeatDim];
+      candidate_params<T, F::FeatDim>(tree, node, fs, bnd.lo, bnd.hi, p);
+      for (int j = 0; j < F::FeatDim; j++) par[(size_t)slot * F::FeatDim + j] = p[j];
+      thr[slot] = candidate_threshold<T>(tree, node, fs, k / nF, bnd.tlo, bnd.thi);
+    }
   } else if (c == 1) {
     const float g = key_gain(key);
     r[1] = __float_as_uint(g);
@@ -1123,10 +1139,9 @@ template <class F>
 __global__ __launch_bounds__(256) void k_route_flags(const typename F::ImgType *__restrict__ pixels,
                                                      const ImgDesc *__restrict__ imgs, const uint4 *__restrict__ recs,
                                                      const uint32_t *__restrict__ rec_slot, uint32_t n,
-                                                     const int32_t *__restrict__ slot_node,
-                                                     const int32_t *__restrict__ tree_left,
-                                                     const typename F::FeatType *__restrict__ tree_feat,
-                                                     const typename F::FeatType *__restrict__ tree_thr,
+                                                     const uint8_t *__restrict__ slot_split,
+                                                     const typename F::FeatType *__restrict__ slot_feat,
+                                                     const typename F::FeatType *__restrict__ slot_thr,
                                                      unsigned long long *__restrict__ flags, AcArgs ac)
 {
   using T = typename F::FeatType;
@@ -1135,16 +1150,15 @@ __global__ __launch_bounds__(256) void k_route_flags(const typename F::ImgType *
   unsigned long long fl = 0ull;   // (left) | (right << 32); entry n is the scan's total
   if (i < n) {
     const uint32_t slot = rec_slot[i];
-    const int32_t node = slot_node[slot];
-    if (tree_left[node] >= 0) {
+    if (slot_split[slot]) {
       const uint4 r = recs[i];
       const ImgDesc d = imgs[rec_img(r)];
       ImageView<typename F::ImgType, F::nChannels> view{pixels + d.off, (int)d.w, (int)d.h};
       T p[F::FeatDim];
 #pragma unroll
-      for (int j = 0; j < F::FeatDim; j++) p[j] = tree_feat[(size_t)node * F::FeatDim + j];
+      for (int j = 0; j < F::FeatDim; j++) p[j] = slot_feat[(size_t)slot * F::FeatDim + j];
       const T v = eval_hook<F>(view, rec_x(r), rec_y(r), unpack_prep<typename F::Prep>(r.z, r.w), p, ac, rec_img(r));
-      fl = (v <= tree_thr[node]) ? 1ull : (1ull << 32);
+      fl = (v <= slot_thr[slot]) ? 1ull : (1ull << 32);
     }
   }
   flags[i] = fl;
@@ -1159,9 +1173,15 @@ __global__ __launch_bounds__(256) void k_route_scatter(const uint4 *__restrict__
                                                        const uint32_t *__restrict__ slot_begin,
                                                        const int32_t *__restrict__ slot_next,
                                                        const uint32_t *__restrict__ next_begin, uint4 *__restrict__ out_recs,
-                                                       uint32_t *__restrict__ out_slot, uint32_t out_cap)
+                                                       uint32_t *__restrict__ out_slot, uint32_t out_cap,
+                                                       uint32_t n_slots, uint32_t *__restrict__ ccount)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_slots) {
+    const unsigned long long a = rank[slot_begin[i]], b = rank[slot_begin[i + 1]];
+    ccount[2 * i] = (uint32_t)b - (uint32_t)a;
+    ccount[2 * i + 1] = (uint32_t)(b >> 32) - (uint32_t)(a >> 32);
+  }
   if (i >= n) return;
   const unsigned long long fl = flags[i];
   if (!fl) return;
@@ -1178,17 +1198,6 @@ __global__ __launch_bounds__(256) void k_route_scatter(const uint4 *__restrict__
     out_recs[pos] = recs[i];
     out_slot[pos] = (uint32_t)ns;
   }
-}
-
-// Per-slot (left, right) totals of the routed samples from the scan.
-__global__ void k_route_counts(const unsigned long long *__restrict__ rank, const uint32_t *__restrict__ slot_begin,
-                               uint32_t n_slots, uint32_t *__restrict__ ccount)
-{
-  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n_slots) return;
-  const unsigned long long a = rank[slot_begin[q]], b = rank[slot_begin[q + 1]];
-  ccount[2 * q] = (uint32_t)b - (uint32_t)a;
-  ccount[2 * q + 1] = (uint32_t)(b >> 32) - (uint32_t)(a >> 32);
 }
 
 // ---------------------------------------------------------------------------
@@ -1412,30 +1421,6 @@ __global__ __launch_bounds__(256) void k_ac_post_finish(const int32_t *__restric
 __global__ __launch_bounds__(256) void k_fill_i32(int32_t *__restrict__ p, uint64_t n, int32_t v)
 {
   for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) p[i] = v;
-}
-
-// Parameters and threshold of each slot's winning pair (res rows
-// {k = t*nFe + f, ...}; f mapped through cand_map when given), re-derived
-// from the sampler for the tree arrays (the reference re-derives them on
-// the host, cl_tree_trainer_impl_learn_best_featthr.hpp:183-222).
-template <class F>
-__global__ __launch_bounds__(256) void k_winner_params(uint32_t tree, const int32_t *__restrict__ slot_node,
-                                                       const uint32_t *__restrict__ res, uint32_t ns, uint32_t nC,
-                                                       uint32_t nFe, const uint32_t *__restrict__ cand_map,
-                                                       Bounds<F> bnd, typename F::FeatType *__restrict__ par,
-                                                       typename F::FeatType *__restrict__ thr)
-{
-  using T = typename F::FeatType;
-  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= ns) return;
-  const uint32_t k = res[(size_t)q * (nC + 2)];
-  const uint32_t t = k / nFe, f = k % nFe;
-  const uint32_t fs = cand_map ? cand_map[(size_t)q * nFe + f] : f;
-  const uint32_t node = (uint32_t)slot_node[q];
-  T p[F::FeatDim];
-  candidate_params<T, F::FeatDim>(tree, node, fs, bnd.lo, bnd.hi, p);
-  for (int j = 0; j < F::FeatDim; j++) par[(size_t)q * F::FeatDim + j] = p[j];
-  thr[q] = candidate_threshold<T>(tree, node, fs, t, bnd.tlo, bnd.thi);
 }
 
 // Evenly spaced subsample of every slot's records (the refinement stage of

@@ -168,9 +168,6 @@ int pd_split_search(int device, uint32_t n_nodes, uint32_t n_classes, uint32_t n
     const size_t per = (size_t)n_classes * n_thresholds * n_features;
     const uint32_t ftiles = (n_features + 63) / 64;
     t.d_H.ensure(per * n_nodes * sizeof(uint32_t));
-    t.d_tot.ensure((size_t)n_nodes * n_classes * sizeof(uint32_t));
-    t.d_slot_mode.ensure(n_nodes);
-    t.d_slot_hidx.ensure(n_nodes * sizeof(int32_t));
     t.d_cand_key.ensure((size_t)n_nodes * ftiles * sizeof(unsigned long long));
     t.d_cand_left.ensure((size_t)n_nodes * ftiles * n_classes * sizeof(uint32_t));
     std::vector<uint8_t> mode(n_nodes, 0);
@@ -178,9 +175,20 @@ int pd_split_search(int device, uint32_t n_nodes, uint32_t n_classes, uint32_t n
     std::vector<uint32_t> hslots(n_nodes), res;
     for (uint32_t q = 0; q < n_nodes; q++) hidx[q] = (int32_t)(hslots[q] = q);
     HIPCHK(hipMemcpy(t.d_H.p, H, per * n_nodes * sizeof(uint32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(t.d_tot.p, tot, (size_t)n_nodes * n_classes * sizeof(uint32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(t.d_slot_mode.p, mode.data(), n_nodes, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(t.d_slot_hidx.p, hidx.data(), n_nodes * sizeof(int32_t), hipMemcpyHostToDevice));
+    const std::vector<uint64_t> no_key(n_nodes, 0ull);
+    Trainer<DepthU16Feature>::Upload up{t, t.d_slice};
+    const size_t u_tot = up.add(tot, (size_t)n_nodes * n_classes * sizeof(uint32_t));
+    const size_t u_mode = up.add(mode.data(), n_nodes);
+    const size_t u_hidx = up.add(hidx.data(), n_nodes * sizeof(int32_t));
+    const size_t u_list = up.add(hslots.data(), n_nodes * sizeof(uint32_t));
+    const size_t u_best = up.add(no_key.data(), n_nodes * sizeof(uint64_t));
+    up.stage();
+    up.commit();
+    t.sl.tot = up.at<uint32_t>(u_tot);
+    t.sl.slot_mode = up.at<uint8_t>(u_mode);
+    t.sl.slot_hidx = up.at<int32_t>(u_hidx);
+    t.sl.hlist = up.at<uint32_t>(u_list);
+    t.sl.best = up.at<unsigned long long>(u_best);
     DevBuf dg;
     if (all_gains) dg.ensure((size_t)n_nodes * n_thresholds * n_features * sizeof(float));
     t.split_slice(n_nodes, hslots, n_thresholds, n_features, PD_MODE_LEVEL_BATCHED, res,
