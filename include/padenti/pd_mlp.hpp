@@ -129,18 +129,28 @@ __device__ __forceinline__ f32x4 mma(uint4 a, uint4 b, f32x4 c)
 constexpr float GELU_C = 0.7978845608028654f;   // sqrt(2 / pi)
 constexpr float GELU_A = 0.044715f;
 
-// tanh-form GELU through 0.5 (1 + tanh u) = 1 / (1 + e^(-2u)): one exp and
-// one reciprocal instead of tanhf (the same function; FP32 rounding only)
-__device__ __forceinline__ float gelu_sig(float z)
+// tanh-form GELU through 0.5 (1 + tanh u) = 1 / (1 + 2^(-2u log2 e)), u =
+// GELU_C (z + GELU_A z^3): the constants folded into one polynomial of z^2, one
+// exp and one reciprocal, seven operations (the same function; FP32 rounding only)
+constexpr float GELU_K1 = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634);
+constexpr float GELU_K3 = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634 * 0.044715);
+__device__ __forceinline__ float gelu_sig(float z, float zz)
 {
-  const float u = GELU_C * (z + GELU_A * z * z * z);
-  return __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * u));
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * __builtin_fmaf(zz, GELU_K3, GELU_K1)));
 }
-__device__ __forceinline__ float gelu(float z) { return z * gelu_sig(z); }
-// d gelu / dz = s + 2 z s (1 - s) u',  s = sigmoid(2u) = gelu_sig(z), u' = c (1 + 3 a z^2)
-__device__ __forceinline__ float gelu_grad_s(float z, float s)
+// d gelu / dz = s + 2 z s (1 - s) u',  s = sigmoid(2u) = gelu_sig(z), h = z s, u' = c (1 + 3 a z^2)
+__device__ __forceinline__ float gelu_grad(float zz, float s, float h)
 {
-  return s + 2.0f * z * s * (1.0f - s) * (GELU_C * (1.0f + 3.0f * GELU_A * z * z));
+  const float du = __builtin_fmaf(zz, 6.0f * GELU_A * GELU_C, 2.0f * GELU_C);
+  return __builtin_fmaf(h * (1.0f - s), du, s);
+}
+
+// two floats to packed BF16, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t cvt2bf(float lo, float hi)
+{
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 
 // device view of the packed weights
@@ -185,26 +195,19 @@ struct RowsMem {
 
 __device__ __forceinline__ uint4 pack8(const float *v)
 {
-  uint4 r;
-  r.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-  r.y = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-  r.z = (uint32_t)f2bf(v[4]) | ((uint32_t)f2bf(v[5]) << 16);
-  r.w = (uint32_t)f2bf(v[6]) | ((uint32_t)f2bf(v[7]) << 16);
-  return r;
+  return uint4{cvt2bf(v[0], v[1]), cvt2bf(v[2], v[3]), cvt2bf(v[4], v[5]), cvt2bf(v[6], v[7])};
 }
 
-// Block GEMM of the tile: acc[rt][ct] = act[16 rt + i][:K] . W[64 wave + 16 ct + j][:K]
+// Block GEMM of the tile: acc[rt][ct] += act[16 rt + i][:K] . W[64 wave + 16 ct + j][:K]
 // MFMA fragments (16x16x32): lane l holds A[l % 16][8 (l / 16) .. +7],
 // B[8 (l / 16) .. +7][l % 16]; the result C[4 (l / 16) + jj][l % 16] in acc[jj].
-template <int K, int RT = 4>
+// The activations are operand A and the lane's four results are four rows of
+// one unit, or (UT) the weights are and they are four units of one row.
+template <int K, int RT = 4, bool UT = false>
 __device__ __forceinline__ void tile_gemm(const uint16_t *act, const uint16_t *__restrict__ W, uint32_t lane,
                                           uint32_t wave, f32x4 (&acc)[RT][4])
 {
   const uint32_t r16 = lane & 15u, kg = (lane >> 4) * 8u;
-#pragma unroll
-  for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-    for (int ct = 0; ct < 4; ct++) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 2
   for (int kk = 0; kk < K; kk += 32) {
     uint4 a[RT], b[4];
@@ -216,7 +219,7 @@ __device__ __forceinline__ void tile_gemm(const uint16_t *act, const uint16_t *_
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++) acc[rt][ct] = mma(a[rt], b[ct], acc[rt][ct]);
+      for (int ct = 0; ct < 4; ct++) acc[rt][ct] = UT ? mma(b[ct], a[rt], acc[rt][ct]) : mma(a[rt], b[ct], acc[rt][ct]);
   }
 }
 
@@ -262,48 +265,59 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
 #pragma unroll 1
   for (int layer = 0; layer < 3; layer++) {
     const float *bias = w.theta + (layer == 0 ? OFF_B1 : (layer == 1 ? OFF_B2 : OFF_B3));
-    if (layer == 0) tile_gemm<INP, RT>(act, w.W1, lane, wave, acc);
-    else tile_gemm<HID, RT>(act, layer == 1 ? w.W2 : w.W3, lane, wave, acc);
+    // the accumulators start from the bias; inference has a lane hold four
+    // units of a row (one 8-byte LDS store), training four rows of a unit (the
+    // order G and HT are stored in)
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) {
+      f32x4 b;
+      if constexpr (TRAIN) b = bias[64u * wave + 16u * ct + (lane & 15u)] * f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+      else b = *(const f32x4 *)(bias + 64u * wave + 16u * ct + 4u * (lane >> 4));
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++) acc[rt][ct] = b;
+    }
+    if (layer == 0) tile_gemm<INP, RT, !TRAIN>(act, w.W1, lane, wave, acc);
+    else tile_gemm<HID, RT, !TRAIN>(act, layer == 1 ? w.W2 : w.W3, lane, wave, acc);
     __syncthreads();   // every wave has read the layer input
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
       for (int ct = 0; ct < 4; ct++) {
-        const uint32_t col = 64u * wave + 16u * ct + (lane & 15u);
-        const uint32_t rb = 16u * rt + 4u * (lane >> 4);
-        const float b = bias[col];
-        uint16_t hb[4], gb[4];
+        float h[4], g[4];
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
-          const float z = acc[rt][ct][jj] + b;
-          const float sg = gelu_sig(z);
-          hb[jj] = f2bf(z * sg);
-          act[(rb + jj) * LDA + col] = hb[jj];
-          if (TRAIN) gb[jj] = f2bf(gelu_grad_s(z, sg));
+          const float z = acc[rt][ct][jj], zz = z * z, sg = gelu_sig(z, zz);
+          h[jj] = z * sg;
+          if (TRAIN) g[jj] = gelu_grad(zz, sg, h[jj]);
         }
-        if (TRAIN) {
-          uint2 pk;
-          pk.x = (uint32_t)hb[0] | ((uint32_t)hb[1] << 16);
-          pk.y = (uint32_t)hb[2] | ((uint32_t)hb[3] << 16);
-          *(uint2 *)(HT + tix((layer + 1) * HID + col, row0 + rb, ldb)) = pk;
-          pk.x = (uint32_t)gb[0] | ((uint32_t)gb[1] << 16);
-          pk.y = (uint32_t)gb[2] | ((uint32_t)gb[3] << 16);
-          *(uint2 *)(G + tix(layer * HID + col, row0 + rb, ldb)) = pk;
+        const uint2 hb{cvt2bf(h[0], h[1]), cvt2bf(h[2], h[3])};
+        if constexpr (TRAIN) {
+          const uint32_t col = 64u * wave + 16u * ct + (lane & 15u), rb = 16u * rt + 4u * (lane >> 4);
+          act[(rb + 0) * LDA + col] = (uint16_t)hb.x;
+          act[(rb + 1) * LDA + col] = (uint16_t)(hb.x >> 16);
+          act[(rb + 2) * LDA + col] = (uint16_t)hb.y;
+          act[(rb + 3) * LDA + col] = (uint16_t)(hb.y >> 16);
+          *(uint2 *)(HT + tix((layer + 1) * HID + col, row0 + rb, ldb)) = hb;
+          *(uint2 *)(G + tix(layer * HID + col, row0 + rb, ldb)) = uint2{cvt2bf(g[0], g[1]), cvt2bf(g[2], g[3])};
+        } else {
+          const uint32_t r = 16u * rt + (lane & 15u), ub = 64u * wave + 16u * ct + 4u * (lane >> 4);
+          *(uint2 *)(act + r * LDA + ub) = hb;
         }
       }
     __syncthreads();
   }
-  // output layer: y = h3 . w4 + b4 (FP32, fixed summation order)
+  // output layer: y = h3 . w4 + b4 on the matrix cores, w4 as every row of
+  // operand A: lane l < 16 receives the sum of row 16 rt + l
+  const float b4 = w.theta[OFF_B4];
 #pragma unroll
-  for (uint32_t rr = 0; rr < FR; rr += THREADS / 4) {
-    const uint32_t r = rr + (tid >> 2), part = tid & 3u;
-    if (FR < THREADS / 4 && r >= FR) break;   // a 32-row tile: the upper half of the block idles
-    float s = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < 64; k++) s += bf2f(act[r * LDA + part * 64 + k]) * bf2f(w.w4[part * 64 + k]);
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    if (part == 0 && row0 + r < (TRAIN ? ldb : n)) y[row0 + r] = s + w.theta[OFF_B4];
+  for (uint32_t rt = wave; rt < (uint32_t)RT; rt += THREADS / 64) {
+    f32x4 s{b4, b4, b4, b4};
+#pragma unroll
+    for (int kk = 0; kk < HID; kk += 32)
+      s = mma(*(const uint4 *)(w.w4 + kk + 8u * (lane >> 4)),
+              *(const uint4 *)(act + (16u * rt + (lane & 15u)) * LDA + kk + 8u * (lane >> 4)), s);
+    const uint32_t row = row0 + 16u * rt + lane;
+    if (lane < 16u && row < (TRAIN ? ldb : n)) y[row] = s[0];
   }
 }
 
@@ -372,6 +386,10 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
 #pragma unroll 1
   for (int layer = 2; layer >= 1; layer--) {
     // dH_{layer} = dZ_{layer+1} . W_{layer+1}: B[n][k] = W[n][k] = WT[k][n]
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     tile_gemm<HID, RT>(act, layer == 2 ? w.W3T : w.W2T, lane, wave, acc);
     __syncthreads();
 #pragma unroll
@@ -380,17 +398,18 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
       for (int ct = 0; ct < 4; ct++) {
         const uint32_t col = 64u * wave + 16u * ct + (lane & 15u);
         const uint32_t rb = 16u * rt + 4u * (lane >> 4);
-        uint16_t hb[4];
         const uint2 gq = *(const uint2 *)(G + tix((layer - 1) * HID + col, row0 + rb, ldb));   // rows rb .. rb + 3
-        const uint32_t gw[2] = {gq.x, gq.y};
+        float d[4];
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
-          hb[jj] = f2bf(acc[rt][ct][jj] * bf2f((uint16_t)(gw[jj >> 1] >> (16 * (jj & 1)))));
-          act[(rb + jj) * LDA + col] = hb[jj];
+          const uint32_t gw = jj < 2 ? gq.x : gq.y;
+          d[jj] = acc[rt][ct][jj] * __builtin_bit_cast(float, jj & 1 ? gw & 0xffff0000u : gw << 16);
         }
-        uint2 pk;
-        pk.x = (uint32_t)hb[0] | ((uint32_t)hb[1] << 16);
-        pk.y = (uint32_t)hb[2] | ((uint32_t)hb[3] << 16);
+        const uint2 pk{cvt2bf(d[0], d[1]), cvt2bf(d[2], d[3])};
+        act[(rb + 0) * LDA + col] = (uint16_t)pk.x;
+        act[(rb + 1) * LDA + col] = (uint16_t)(pk.x >> 16);
+        act[(rb + 2) * LDA + col] = (uint16_t)pk.y;
+        act[(rb + 3) * LDA + col] = (uint16_t)(pk.y >> 16);
         *(uint2 *)(DZT + tix((layer - 1) * HID + col, row0 + rb, ldb)) = pk;
       }
     __syncthreads();
