@@ -15,10 +15,18 @@
 // Kernels (256-thread blocks, 4 wave64s; 128-row tiles):
 //   k_mlp_fwd     all layers fused, 128 (or 64 / 32) rows per block; the
 //                 tile's activations stay in LDS.  A wave owns 64 output
-//                 columns: 8 x 4 MFMA 16x16 tiles, the A operand
-//                 (activations) from LDS, the B operand (weights, [out][in]
-//                 row-major) straight from L2; two waves per SIMD (registers
-//                 capped at 256), so one wave's epilogue overlaps another's
+//                 columns: 8 x 4 MFMA 16x16 tiles, one operand (activations)
+//                 from LDS, the other (weights, stored in MFMA fragment order,
+//                 tix()) from L2 through a register ring that runs ahead over
+//                 the layers; two waves per SIMD (registers capped at 256), so
+//                 one wave's epilogue overlaps another's MFMAs.  Bound by the
+//                 epilogue's VALU work: 2^20 rows 640 us (456 TFLOP/s) at first,
+//                 455 with the constants of the GELU folded, packed BF16
+//                 conversion, 8-byte LDS stores and the output layer on the
+//                 matrix cores, 380 (768 TFLOP/s) with the ring: VALU pipe 76%
+//                 busy (7.5 operations an activation), matrix cores 40%.
+//                 Batches of 4096 training rows: 17.4 -> 12.4 us, the backward
+//                 15.5 -> 10.0 us (waits for L2 loads).
 //                 MFMAs.  Training mode also stores the BF16 GELU
 //                 derivatives G = gelu'(z) of the pre-activations (the
 //                 backward multiplies by them) and the BF16 activations H in
@@ -36,7 +44,7 @@
 //                 from the weight-gradient blocks themselves).
 //   k_mlp_adam    sums the split partials in fixed order, applies Adam,
 //                 refreshes the BF16 weight copies and sums the step's loss.
-//   k_mlp_pack    FP32 master -> BF16 [out][in] and transposed copies.
+//   k_mlp_pack    FP32 master -> BF16 copies and transposed copies in fragment order.
 //   k_topk        per node, the `keep` best of K scores (radix select on the
 //                 orderable score bits, ties to the lower candidate index),
 //                 written in increasing candidate order.
@@ -98,6 +106,18 @@ __host__ __device__ __forceinline__ size_t tix(uint32_t n, uint32_t r, uint32_t 
   return ((size_t)(n >> 4) * (ldb >> 5) + (r >> 5)) * 512u + ((r & 31u) >> 3) * 128u + (n & 15u) * 8u + (r & 7u);
 }
 
+// tix() of the lane's four results of MFMA tile (units 16 n16 .. + 15, rows 16
+// r16 .. + 15, four rows of unit l % 16 a lane): the tile's part (uniform) and
+// the lane's
+__host__ __device__ __forceinline__ size_t tix_tile(uint32_t n16, uint32_t r16, uint32_t ldb)
+{
+  return ((size_t)n16 * (ldb >> 5) + (r16 >> 1)) * 512u + (r16 & 1u) * 256u;
+}
+__host__ __device__ __forceinline__ uint32_t tix_lane(uint32_t lane)
+{
+  return (lane >> 5) * 128u + (lane & 15u) * 8u + ((lane >> 4) & 1u) * 4u;
+}
+
 // Raw buffer resource word 3 of gfx9-family targets (32-bit data format,
 // no swizzle); loads past the resource's byte count return zero.
 constexpr int BUF_DWORD3 = 0x00020000;
@@ -155,10 +175,10 @@ __device__ __forceinline__ uint32_t cvt2bf(float lo, float hi)
 
 // device view of the packed weights
 struct Weights {
-  const uint16_t *W1;    // [256][32] bf16
-  const uint16_t *W2;    // [256][256]
-  const uint16_t *W3;    // [256][256]
-  const uint16_t *W2T;   // [256][256] transposed
+  const uint16_t *W1;    // bf16, element (unit, input) at tix(unit, input, 32)
+  const uint16_t *W2;    // at tix(unit, input, 256)
+  const uint16_t *W3;
+  const uint16_t *W2T;   // transposed: at tix(input, unit, 256)
   const uint16_t *W3T;
   const uint16_t *w4;    // [256]
   const float *theta;    // FP32 master (biases are read from it)
@@ -198,28 +218,60 @@ __device__ __forceinline__ uint4 pack8(const float *v)
   return uint4{cvt2bf(v[0], v[1]), cvt2bf(v[2], v[3]), cvt2bf(v[4], v[5]), cvt2bf(v[6], v[7])};
 }
 
-// Block GEMM of the tile: acc[rt][ct] += act[16 rt + i][:K] . W[64 wave + 16 ct + j][:K]
-// MFMA fragments (16x16x32): lane l holds A[l % 16][8 (l / 16) .. +7],
-// B[8 (l / 16) .. +7][l % 16]; the result C[4 (l / 16) + jj][l % 16] in acc[jj].
-// The activations are operand A and the lane's four results are four rows of
-// one unit, or (UT) the weights are and they are four units of one row.
-template <int K, int RT = 4, bool UT = false>
-__device__ __forceinline__ void tile_gemm(const uint16_t *act, const uint16_t *__restrict__ W, uint32_t lane,
-                                          uint32_t wave, f32x4 (&acc)[RT][4])
+// Matrix products of a tile of 16 RT rows: a wave owns 64 units (4 x RT MFMA
+// 16x16 tiles).  MFMA fragments (16x16x32): lane l holds A[l % 16][8 (l / 16)
+// .. +7], B[8 (l / 16) .. +7][l % 16]; the result C[4 (l / 16) + jj][l % 16] in
+// acc[jj].  The activations are operand A and the lane's four results are four
+// rows of one unit, or (UT) the weights are and they are four units of one row.
+//
+// The weights come from L2, a 32-deep step (4 fragments a wave) at a time and
+// through a ring of registers WD steps ahead that runs on over the layers: the
+// loads of a layer's first steps are in flight during the epilogue before it.
+// A block of few rows has little work to hide them behind (RT = 2: 128 cycles of
+// MFMA a step against ~1000 of latency) and the registers for a whole layer.
+// The activations' fragments come from LDS two products ahead.  Left to the
+// compiler, every step waited for its own loads.
+template <int RT>
+constexpr int weight_depth()
 {
-  const uint32_t r16 = lane & 15u, kg = (lane >> 4) * 8u;
-#pragma unroll 2
-  for (int kk = 0; kk < K; kk += 32) {
-    uint4 a[RT], b[4];
+  return RT >= 8 ? 2 : RT == 4 ? 4 : 8;
+}
+constexpr int KS = HID / 32;   // steps of a hidden layer
+
+// fragment of unit group cg (16 units), step s of a matrix with K columns (tix()
+// order), through a buffer resource: the address costs one register, not two a
+// fragment
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const void *p, uint32_t bytes)
+{
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)bytes, BUF_DWORD3);
+}
+__device__ __forceinline__ uint4 wfrag(__amdgpu_buffer_rsrc_t W, int K, uint32_t cg, int s, uint32_t lane)
+{
+  return buf_load16(W, lane * 16u, (int)((cg * (uint32_t)(K / 32) + (uint32_t)s) * 1024u));
+}
+
+// Steps [S0, S1) of the weight stream against the tile: acc = c0[ct] + ...;
+// load(s) fetches step s into ring slot s % WD (nothing past the last step).
+template <int S0, int S1, int RT, bool UT, int WD, class Load>
+__device__ __forceinline__ void tile_gemm(const uint16_t *act, uint32_t lane, uint4 (&wb)[WD][4], const Load &load,
+                                          const f32x4 (&c0)[4], f32x4 (&acc)[RT][4])
+{
+  constexpr int N = (S1 - S0) * RT, AD = N < 3 ? N : 3;
+  const uint16_t *base = act + (lane & 15u) * LDA + (lane >> 4) * 8u;
+  uint4 a[AD];
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++)
-      b[ct] = *(const uint4 *)(W + (size_t)(64u * wave + 16u * ct + r16) * K + kk + kg);
+  for (int i = 0; i < AD - 1; i++) a[i] = *(const uint4 *)(base + (i % RT) * 16 * LDA + (i / RT) * 32);
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) a[rt] = *(const uint4 *)(act + (16u * rt + r16) * LDA + kk + kg);
+  for (int i = 0; i < N; i++) {
+    const int s = S0 + i / RT, rt = i % RT, j = i + AD - 1;
+    if (j < N) a[j % AD] = *(const uint4 *)(base + (j % RT) * 16 * LDA + (j / RT) * 32);
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) acc[rt][ct] = UT ? mma(b[ct], a[rt], acc[rt][ct]) : mma(a[rt], b[ct], acc[rt][ct]);
+    for (int ct = 0; ct < 4; ct++) {
+      const f32x4 c = s == S0 ? c0[ct] : acc[rt][ct];
+      acc[rt][ct] = UT ? mma(wb[s % WD][ct], a[i % AD], c) : mma(a[i % AD], wb[s % WD][ct], c);
+    }
+    if (rt == RT - 1) load(s + WD);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -239,6 +291,34 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t row0 = blockIdx.x * FR;
+  constexpr int WD = weight_depth<RT>();
+  const __amdgpu_buffer_rsrc_t r1 = weight_rsrc(w.W1, HID * INP * 2), r2 = weight_rsrc(w.W2, HID * HID * 2),
+                               r3 = weight_rsrc(w.W3, HID * HID * 2), rth = weight_rsrc(w.theta, NPARAM * 4);
+  uint4 wb[WD][4];
+  const auto load = [&](int s) __attribute__((always_inline)) {
+    if (s >= 1 + 2 * KS) return;
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+      wb[s % WD][ct] = s == 0 ? wfrag(r1, INP, 4u * wave + ct, 0, lane)
+                              : wfrag(s <= KS ? r2 : r3, HID, 4u * wave + ct, (s - 1) % KS, lane);
+  };
+  // bias of a layer in accumulator form
+  f32x4 c0[4];
+  const auto load_bias = [&](int off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) {
+      if constexpr (TRAIN) {
+        const float b = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(rth, (lane & 15u) * 4u, (off + 64u * wave + 16u * ct) * 4u, 0));
+        c0[ct] = f32x4{b, b, b, b};
+      } else {
+        c0[ct] = __builtin_bit_cast(f32x4, buf_load16(rth, (lane >> 4) * 16u, (off + 64u * wave + 16u * ct) * 4u));
+      }
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < WD; s++) load(s);
+  load_bias(OFF_B1);
 #pragma unroll
   for (uint32_t i = tid; i < FR * 4u; i += THREADS) {
     const uint32_t r = i >> 2, q = i & 3u;
@@ -262,22 +342,24 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
     }
   }
   f32x4 acc[RT][4];
-#pragma unroll 1
+  uint4 w4f[KS];
+  const auto load_w4 = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < KS; s++) w4f[s] = *(const uint4 *)(w.w4 + 32 * s + 8u * (lane >> 4));
+  };
+  // the accumulators start from the bias; inference has a lane hold four units
+  // of a row (one 8-byte LDS store), training four rows of a unit (the order G
+  // and HT are stored in)
+#pragma unroll
   for (int layer = 0; layer < 3; layer++) {
-    const float *bias = w.theta + (layer == 0 ? OFF_B1 : (layer == 1 ? OFF_B2 : OFF_B3));
-    // the accumulators start from the bias; inference has a lane hold four
-    // units of a row (one 8-byte LDS store), training four rows of a unit (the
-    // order G and HT are stored in)
-#pragma unroll
-    for (int ct = 0; ct < 4; ct++) {
-      f32x4 b;
-      if constexpr (TRAIN) b = bias[64u * wave + 16u * ct + (lane & 15u)] * f32x4{1.0f, 1.0f, 1.0f, 1.0f};
-      else b = *(const f32x4 *)(bias + 64u * wave + 16u * ct + 4u * (lane >> 4));
-#pragma unroll
-      for (int rt = 0; rt < RT; rt++) acc[rt][ct] = b;
+    if (layer == 0) tile_gemm<0, 1, RT, !TRAIN, WD>(act, lane, wb, load, c0, acc);
+    else if (layer == 1) tile_gemm<1, 1 + KS, RT, !TRAIN, WD>(act, lane, wb, load, c0, acc);
+    else tile_gemm<1 + KS, 1 + 2 * KS, RT, !TRAIN, WD>(act, lane, wb, load, c0, acc);
+    if (layer < 2) {
+      load_bias(layer == 0 ? OFF_B2 : OFF_B3);
+    } else if (RT < 8) {
+      load_w4();
     }
-    if (layer == 0) tile_gemm<INP, RT, !TRAIN>(act, w.W1, lane, wave, acc);
-    else tile_gemm<HID, RT, !TRAIN>(act, layer == 1 ? w.W2 : w.W3, lane, wave, acc);
     __syncthreads();   // every wave has read the layer input
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
@@ -297,25 +379,28 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
           act[(rb + 1) * LDA + col] = (uint16_t)(hb.x >> 16);
           act[(rb + 2) * LDA + col] = (uint16_t)hb.y;
           act[(rb + 3) * LDA + col] = (uint16_t)(hb.y >> 16);
-          *(uint2 *)(HT + tix((layer + 1) * HID + col, row0 + rb, ldb)) = hb;
-          *(uint2 *)(G + tix(layer * HID + col, row0 + rb, ldb)) = uint2{cvt2bf(g[0], g[1]), cvt2bf(g[2], g[3])};
+          const uint32_t n16 = layer * (HID / 16) + 4u * wave + ct, r16 = row0 / 16u + rt;
+          *(uint2 *)(HT + tix_tile(n16 + HID / 16, r16, ldb) + tix_lane(lane)) = hb;
+          *(uint2 *)(G + tix_tile(n16, r16, ldb) + tix_lane(lane)) = uint2{cvt2bf(g[0], g[1]), cvt2bf(g[2], g[3])};
         } else {
           const uint32_t r = 16u * rt + (lane & 15u), ub = 64u * wave + 16u * ct + 4u * (lane >> 4);
           *(uint2 *)(act + r * LDA + ub) = hb;
         }
       }
+    if (RT >= 8 && layer == 2) load_w4();   // (no registers for them before)
     __syncthreads();
   }
   // output layer: y = h3 . w4 + b4 on the matrix cores, w4 as every row of
   // operand A: lane l < 16 receives the sum of row 16 rt + l
   const float b4 = w.theta[OFF_B4];
 #pragma unroll
-  for (uint32_t rt = wave; rt < (uint32_t)RT; rt += THREADS / 64) {
+  for (int i = 0; i < (RT + 3) / 4; i++) {
+    const uint32_t rt = wave + 4u * i;
+    if (RT % 4 != 0 && rt >= (uint32_t)RT) break;
     f32x4 s{b4, b4, b4, b4};
 #pragma unroll
-    for (int kk = 0; kk < HID; kk += 32)
-      s = mma(*(const uint4 *)(w.w4 + kk + 8u * (lane >> 4)),
-              *(const uint4 *)(act + (16u * rt + (lane & 15u)) * LDA + kk + 8u * (lane >> 4)), s);
+    for (int k = 0; k < KS; k++)
+      s = mma(w4f[k], *(const uint4 *)(act + (16u * rt + (lane & 15u)) * LDA + 32 * k + 8u * (lane >> 4)), s);
     const uint32_t row = row0 + 16u * rt + lane;
     if (lane < 16u && row < (TRAIN ? ldb : n)) y[row] = s[0];
   }
@@ -344,6 +429,22 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t row0 = blockIdx.x * ROWS;
+  constexpr int WD = weight_depth<RT>();
+  const __amdgpu_buffer_rsrc_t r3 = weight_rsrc(w.W3T, HID * HID * 2), r2 = weight_rsrc(w.W2T, HID * HID * 2);
+  uint4 wb[WD][4];
+  const auto load = [&](int s) __attribute__((always_inline)) {
+    if (s >= 2 * KS) return;
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) wb[s % WD][ct] = wfrag(s < KS ? r3 : r2, HID, 4u * wave + ct, s % KS, lane);
+  };
+  // gelu' of the last layer for 64 (or ROWS) rows of the thread's unit
+  constexpr int GB = ROWS < 64 ? ROWS / 8 : 8;
+  uint4 g3[GB];
+  const auto load_g3 = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < GB; i++) g3[i] = *(const uint4 *)(G + tix(2u * HID + tid, row0 + r0 + 8 * i, ldb));
+  };
+  load_g3(0);
   if (tid < 64u * LW) {
     const uint32_t row = row0 + tid;
     const bool live = tid < (uint32_t)ROWS && row < n;
@@ -365,32 +466,49 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
   {
     const uint32_t k = tid;
     const float wk = bf2f(w.w4[k]);
-#pragma unroll 1
-    for (int r8 = 0; r8 < ROWS; r8 += 8) {
-      float v[8];
-      const uint4 gq = *(const uint4 *)(G + tix(2u * HID + k, row0 + r8, ldb));   // rows r8 .. r8 + 7
-      const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        v[j] = dys[r8 + j] * wk * bf2f((uint16_t)(gw[j >> 1] >> (16 * (j & 1))));
+    for (int r0 = 0; r0 < ROWS; r0 += 8 * GB) {
+      if (r0) load_g3(r0);
+#pragma unroll
+      for (int i = 0; i < GB; i++) {
+        const int r8 = r0 + 8 * i;
+        float v[8];
+        const uint32_t gw[4] = {g3[i].x, g3[i].y, g3[i].z, g3[i].w};   // rows r8 .. r8 + 7
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          v[j] = dys[r8 + j] * wk * bf2f((uint16_t)(gw[j >> 1] >> (16 * (j & 1))));
+        }
+        const uint4 pk = pack8(v);
+        *(uint4 *)(DZT + tix(2u * HID + k, row0 + r8, ldb)) = pk;
+        const uint32_t pw[4] = {pk.x, pk.y, pk.z, pk.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) act[(r8 + j) * LDA + k] = (uint16_t)(pw[j >> 1] >> (16 * (j & 1)));
       }
-      const uint4 pk = pack8(v);
-      *(uint4 *)(DZT + tix(2u * HID + k, row0 + r8, ldb)) = pk;
-      const uint16_t *e = (const uint16_t *)&pk;
-#pragma unroll
-      for (int j = 0; j < 8; j++) act[(r8 + j) * LDA + k] = e[j];
     }
   }
+#pragma unroll
+  for (int s = 0; s < WD; s++) load(s);
   __syncthreads();
   f32x4 acc[RT][4];
-#pragma unroll 1
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f}, c0[4] = {zero, zero, zero, zero};
+  // gelu' of the tile's elements: fetched ahead of the product where registers are left
+  constexpr bool G_AHEAD = RT <= 4;
+  uint2 gp[G_AHEAD ? RT : 1][4];
+#pragma unroll
   for (int layer = 2; layer >= 1; layer--) {
+    const auto load_g = [&](int rt, int ct) __attribute__((always_inline)) {   // rows rb .. rb + 3
+      return *(const uint2 *)(G + tix_tile((layer - 1) * (HID / 16) + 4u * wave + ct, row0 / 16u + rt, ldb) +
+                              tix_lane(lane));
+    };
+    if constexpr (G_AHEAD) {
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) gp[rt][ct] = load_g(rt, ct);
+    }
     // dH_{layer} = dZ_{layer+1} . W_{layer+1}: B[n][k] = W[n][k] = WT[k][n]
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    tile_gemm<HID, RT>(act, layer == 2 ? w.W3T : w.W2T, lane, wave, acc);
+    if (layer == 2) tile_gemm<0, KS, RT, false, WD>(act, lane, wb, load, c0, acc);
+    else tile_gemm<KS, 2 * KS, RT, false, WD>(act, lane, wb, load, c0, acc);
     __syncthreads();
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
@@ -398,7 +516,9 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
       for (int ct = 0; ct < 4; ct++) {
         const uint32_t col = 64u * wave + 16u * ct + (lane & 15u);
         const uint32_t rb = 16u * rt + 4u * (lane >> 4);
-        const uint2 gq = *(const uint2 *)(G + tix((layer - 1) * HID + col, row0 + rb, ldb));   // rows rb .. rb + 3
+        uint2 gq;
+        if constexpr (G_AHEAD) gq = gp[rt][ct];
+        else gq = load_g(rt, ct);
         float d[4];
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
@@ -410,7 +530,7 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
         act[(rb + 1) * LDA + col] = (uint16_t)(pk.x >> 16);
         act[(rb + 2) * LDA + col] = (uint16_t)pk.y;
         act[(rb + 3) * LDA + col] = (uint16_t)(pk.y >> 16);
-        *(uint2 *)(DZT + tix((layer - 1) * HID + col, row0 + rb, ldb)) = pk;
+        *(uint2 *)(DZT + tix_tile((layer - 1) * (HID / 16) + 4u * wave + ct, row0 / 16u + rt, ldb) + tix_lane(lane)) = pk;
       }
     __syncthreads();
   }
@@ -737,15 +857,15 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ theta, flo
   theta[i] = th;
   const uint16_t hb = f2bf(th);
   if (i < (uint32_t)OFF_B1) {
-    pk.W1[i - OFF_W1] = hb;
+    pk.W1[tix((i - OFF_W1) / INP, (i - OFF_W1) % INP, INP)] = hb;
   } else if (i >= (uint32_t)OFF_W2 && i < (uint32_t)OFF_B2) {
     const uint32_t j = i - OFF_W2;
-    pk.W2[j] = hb;
-    pk.W2T[(j % HID) * HID + j / HID] = hb;
+    pk.W2[tix(j / HID, j % HID, HID)] = hb;
+    pk.W2T[tix(j % HID, j / HID, HID)] = hb;
   } else if (i >= (uint32_t)OFF_W3 && i < (uint32_t)OFF_B3) {
     const uint32_t j = i - OFF_W3;
-    pk.W3[j] = hb;
-    pk.W3T[(j % HID) * HID + j / HID] = hb;
+    pk.W3[tix(j / HID, j % HID, HID)] = hb;
+    pk.W3T[tix(j % HID, j / HID, HID)] = hb;
   } else if (i >= (uint32_t)OFF_W4 && i < (uint32_t)OFF_B4) {
     pk.w4[i - OFF_W4] = hb;
   }
@@ -760,14 +880,14 @@ __global__ void k_mlp_pack(const float *__restrict__ theta, uint16_t *__restrict
   if (i < (uint32_t)(HID * HID)) {
     const uint32_t nn = i / HID, k = i % HID;
     const uint16_t a = f2bf(theta[OFF_W2 + i]), b = f2bf(theta[OFF_W3 + i]);
-    W2[i] = a;
-    W3[i] = b;
-    W2T[k * HID + nn] = a;
-    W3T[k * HID + nn] = b;
+    W2[tix(nn, k, HID)] = a;
+    W3[tix(nn, k, HID)] = b;
+    W2T[tix(k, nn, HID)] = a;
+    W3T[tix(k, nn, HID)] = b;
   }
   if (i < (uint32_t)(HID * INP)) {
     const uint32_t nn = i / INP, k = i % INP;
-    W1[i] = k < (uint32_t)IN ? f2bf(theta[OFF_W1 + nn * IN + k]) : (uint16_t)0;
+    W1[tix(nn, k, INP)] = k < (uint32_t)IN ? f2bf(theta[OFF_W1 + nn * IN + k]) : (uint16_t)0;
   }
   if (i < (uint32_t)HID) w4[i] = f2bf(theta[OFF_W4 + i]);
 }
