@@ -411,6 +411,24 @@ __global__ __launch_bounds__(256) void k_sample_uniform(const SampleJob *__restr
 }
 
 // ---- class-weighted reservoir --------------------------------------------
+// The serial loop walks the pixels in scan order: pixel p of class c with class
+// ordinal k goes to slot k while k < B_c, afterwards it draws from the image's
+// MT19937 stream and may replace a slot.  Neither the ordinals nor the draw
+// indices depend on what was drawn, so the loop is three parallel steps:
+//   k_weighted_count  class counts of every segment (seg_len pixels, one wave
+//                     each) and, in its first blocks, the tempered outputs of
+//                     every image's stream;
+//   k_weighted_scan   per image: class ordinals and draw index at the start of
+//                     every segment;
+//   k_weighted_draw   the segments' pixels, one wave a segment.
+// Only the stream is serial (454 words a step, below).  150 images of 321 x 243,
+// 16 classes: 846 us with one wave an image walking all of it, 102 us now.
+//
+// The streams are generated for draws [w0, w0 + win) of every image at a time
+// (win * n_images words of workspace); larger images take several windows.
+constexpr uint32_t MT_LAG = MT_N - MT_M;     // 227
+constexpr uint32_t MT_STEP = 2 * MT_LAG;     // words a step computes from the last 624
+
 // Ordering inside one wave: LDS operations of a wave execute in issue order,
 // so a fence + wave barrier is all the synchronisation lanes of one wave need.
 __device__ __forceinline__ void wave_sync()
@@ -420,139 +438,246 @@ __device__ __forceinline__ void wave_sync()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One twist of a state by one wave (no tempering: outputs are tempered when
-// drawn).  Same three dependent ranges as mt_twist.
-__device__ inline void mt_twist_wave(uint32_t *mt, uint32_t lane)
+// LDS of the block is in order for its waves (no wait for global memory)
+__device__ __forceinline__ void lds_sync()
 {
-  uint32_t a1[4], a2[4], a3[3];
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const uint32_t i = lane + 64u * r;
-    a1[r] = a2[r] = 0;
-    if (i < 227) {
-      a1[r] = mt[i + MT_M] ^ mt_mix(mt[i], mt[i + 1]);
-      a2[r] = mt_mix(mt[227 + i], mt[228 + i]);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 3; r++) {
-    const uint32_t i = lane + 64u * r;
-    a3[r] = (i < 169) ? mt_mix(mt[454 + i], mt[455 + i]) : 0u;
-  }
-  const uint32_t last_old = mt[623];
-  wave_sync();
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    if (lane + 64u * r < 227) mt[lane + 64u * r] = a1[r];
-  wave_sync();
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    if (lane + 64u * r < 227) mt[227 + lane + 64u * r] = mt[lane + 64u * r] ^ a2[r];
-  wave_sync();
-#pragma unroll
-  for (int r = 0; r < 3; r++)
-    if (lane + 64u * r < 169) mt[454 + lane + 64u * r] = mt[227 + lane + 64u * r] ^ a3[r];
-  if (lane == 0) mt[623] = mt[396] ^ mt_mix(last_old, mt[0]);
-  wave_sync();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One wave per image (four images per block), 64 pixels per step in scan
-// order (lane l: pixel t0 + 64 s + l); the label bytes of the next 16 steps
-// are prefetched from global memory.  A pixel's class ordinal k is the class
-// count so far (LDS) plus its rank among the wave's lanes of that class (one
-// ballot per distinct class, the class read with readlane); it draws iff
-// k >= B_c, and its draw index is the wave prefix of those flags, so the MT
-// stream is consumed in the serial loop's order.  bucket: zero-initialised
-// slots [image][sum B] (class c at boff[c]) filled with atomicMax (the last
-// writer in scan order has the largest pixel index).  Labels above
-// n_classes set *bad.
-//
-// Bound by VALU issue: about 85 VALU + 43 SALU instructions per 64-pixel step
-// (class ranks, the draw's FP64 product and roundf, tempering, a twist per
-// 624 draws).  Keeping the slots in LDS instead of global atomics cut the
-// occupancy and ran slower.
-__global__ __launch_bounds__(256) void k_sample_weighted(const uint8_t *__restrict__ labels,
-                                                         const SampleJob *__restrict__ jobs, uint32_t n_images,
-                                                         const uint32_t *__restrict__ crc, uint32_t seed,
-                                                         uint32_t n_classes, const uint32_t *__restrict__ B,
-                                                         const uint32_t *__restrict__ boff, uint32_t *bucket,
-                                                         uint32_t *class_count, uint32_t *bad)
+// Ordinals of the wave's 64 labels: calls f(class, mask of its lanes) for every
+// distinct class of the lanes with l != 0.
+template <class Fn>
+__device__ __forceinline__ void each_class(uint32_t l, const Fn &f)
 {
-  __shared__ uint32_t sB[256], sO[256];
-  __shared__ uint32_t mt_all[4][MT_N], cnt_all[4][256];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  sB[threadIdx.x] = threadIdx.x < n_classes ? B[threadIdx.x] : 0u;
-  sO[threadIdx.x] = threadIdx.x < n_classes ? boff[threadIdx.x] : 0u;
-  __syncthreads();  // the only block-wide barrier: from here on the waves are independent
-  const uint32_t im = blockIdx.x * 4u + wave;
-  if (im >= n_images) return;
-  uint32_t *mt = mt_all[wave], *cnt = cnt_all[wave];
+  uint64_t pending = __ballot(l != 0u);
+  while (pending) {
+    const uint32_t lead = (uint32_t)__builtin_ctzll(pending);
+    const uint32_t cl = __builtin_amdgcn_readlane(l, lead);
+    const uint64_t mm = __ballot(l == cl);
+    f(cl - 1u, mm);
+    pending &= ~mm;
+  }
+}
+
+// Blocks [0, n_images): the stream of image blockIdx.x, draws [w0, w0 + win)
+// into draws[image * win ..]; `state` carries the last 624 words to the next
+// window.  The other blocks (w0 = 0 only): class counts of four segments.
+// Labels above n_classes set *bad and count as unlabelled.
+//
+// x[k + 624] = x[k + 397] ^ mix(x[k], x[k + 1]): thread i computes words k + 624
+// + i and k + 851 + i of a step of 454; the x[k + 397] of each is the word it
+// computed before, so only old words come from LDS, a ring of 2048 (a step writes
+// words k + 624 .. k + 1077 and reads k .. k + 454; its barrier keeps later writes
+// to their slots behind the reads).  Bound by a step's latency: 227 words a step
+// and x[k + 397] from LDS took the kernel 72 us for 78003 draws an image, this
+// one 56 us.
+__global__ __launch_bounds__(256) void k_weighted_count(const uint8_t *__restrict__ labels,
+                                                        const SampleJob *__restrict__ jobs, uint32_t n_images,
+                                                        const uint32_t *__restrict__ seg0, uint32_t n_segs,
+                                                        uint32_t seg_len, const uint32_t *__restrict__ crc,
+                                                        uint32_t seed, uint32_t n_classes, uint32_t w0, uint32_t win,
+                                                        uint32_t *__restrict__ draws, uint32_t *__restrict__ state,
+                                                        uint32_t *__restrict__ counts, uint32_t *bad)
+{
+  __shared__ uint32_t sh[2048];
+  const uint32_t tid = threadIdx.x;
+  if (blockIdx.x < n_images) {
+    const uint32_t im = blockIdx.x, n_px = jobs[im].n_px;
+    if (n_px <= w0) return;
+    if (w0 == 0u) {
+      if (tid == 0) mt_seed(sh, crc[im] ^ seed);
+    } else {
+      for (uint32_t i = tid; i < MT_N; i += 256u) sh[i] = state[(size_t)im * MT_N + i];
+    }
+    lds_sync();
+    const uint32_t n = n_px - w0 < win ? n_px - w0 : win;   // (an image draws at most once a pixel)
+    uint32_t *o = draws + (size_t)im * win;
+    uint32_t k = 0, x = tid < MT_LAG ? sh[MT_M + tid] : 0u;
+    for (; k < n; k += MT_STEP) {
+      if (tid < MT_LAG) {
+        const uint32_t i = k + tid;
+        const uint32_t m0 = mt_mix(sh[i & 2047u], sh[(i + 1u) & 2047u]);
+        const uint32_t m1 = mt_mix(sh[(i + MT_LAG) & 2047u], sh[(i + MT_LAG + 1u) & 2047u]);
+        const uint32_t y = x ^ m0;
+        x = y ^ m1;
+        sh[(i + MT_N) & 2047u] = y;
+        sh[(i + MT_N + MT_LAG) & 2047u] = x;
+        if (i < n) o[i] = mt_temper(y);
+        if (i + MT_LAG < n) o[i + MT_LAG] = mt_temper(x);
+      }
+      lds_sync();
+    }
+    if (n_px - w0 > win)   // (win is a multiple of MT_STEP)
+      for (uint32_t i = tid; i < MT_N; i += 256u) state[(size_t)im * MT_N + i] = sh[(k + i) & 2047u];
+    return;
+  }
+  const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t seg = (blockIdx.x - n_images) * 4u + wave;
+  if (seg >= n_segs) return;
+  uint32_t *cnt = sh + 256u * wave;
   for (uint32_t c = lane; c < 256u; c += 64u) cnt[c] = 0;
+  wave_sync();
+  const uint32_t im = find_owner(seg0, n_images, seg);
   const SampleJob J = jobs[im];
   const uint8_t *lab = labels + J.lab_off;
-  uint32_t *bk = bucket + J.out_base;
-  if (lane == 0) mt_seed(mt, crc[im] ^ seed);
-  wave_sync();
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
-  uint32_t D = 0, gen = 0;  // draws consumed; outputs generated ([gen - 624, gen) are in mt)
-  uint32_t nx[16];
-#pragma unroll
-  for (int s = 0; s < 16; s++) nx[s] = (64u * s + lane < J.n_px) ? lab[64u * s + lane] : 0u;
-  for (uint32_t t0 = 0; t0 < J.n_px; t0 += 1024u) {
+  const uint32_t p0 = (seg - seg0[im]) * seg_len, p1 = J.n_px - p0 < seg_len ? J.n_px : p0 + seg_len;
+  for (uint32_t t = p0; t < p1; t += 1024u) {
     uint32_t cur[16];
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-      cur[s] = nx[s];
-      const uint32_t q = t0 + 1024u + 64u * s + lane;
-      nx[s] = (q < J.n_px) ? lab[q] : 0u;  // prefetch the next tile
-    }
+    for (uint32_t s = 0; s < 16u; s++) cur[s] = t + 64u * s + lane < p1 ? lab[t + 64u * s + lane] : 0u;
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-      if (t0 + 64u * s >= J.n_px) break;
-      const uint32_t p = t0 + 64u * s + lane;
+    for (uint32_t s = 0; s < 16u; s++) {
+      if (t + 64u * s >= p1) break;
       uint32_t l = cur[s];
-      if (l > n_classes) { atomicOr(bad, 1u); l = 0; }
-      const bool valid = l != 0u;
-      const uint32_t c = l - 1u;
+      if (l > n_classes) {
+        atomicOr(bad, 1u);
+        l = 0;
+      }
+      each_class(l, [&](uint32_t c, uint64_t mm) {
+        if (lane == 0) cnt[c] += (uint32_t)__popcll(mm);
+      });
+    }
+  }
+  wave_sync();
+  for (uint32_t c = lane; c < n_classes; c += 64u) counts[(size_t)seg * n_classes + c] = cnt[c];
+}
+
+// One block of 1024 threads per image.  counts[seg][c]: class counts of a
+// segment in, class ordinal at its start out; seg_draw[seg] = (draw index at its
+// start, number of draws); class_count[image][c] the totals.
+__global__ __launch_bounds__(1024) void k_weighted_scan(const uint32_t *__restrict__ seg0, uint32_t n_images,
+                                                        uint32_t n_segs, uint32_t n_classes,
+                                                        const uint32_t *__restrict__ B, uint32_t *counts,
+                                                        uint2 *__restrict__ seg_draw,
+                                                        uint32_t *__restrict__ class_count)
+{
+  __shared__ uint32_t sB[256], tot[256], ws[16];
+  const uint32_t im = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t s0 = seg0[im], ns = (im + 1u < n_images ? seg0[im + 1u] : n_segs) - s0;
+  uint32_t *ct = counts + (size_t)s0 * n_classes;
+  if (tid < n_classes) sB[tid] = B[tid];
+  for (uint32_t c = wave; c < n_classes; c += 16u) {
+    uint32_t run = 0;
+    for (uint32_t s = 0; s < ns; s += 64u) {
+      const uint32_t v = s + lane < ns ? ct[(size_t)(s + lane) * n_classes + c] : 0u;
+      uint32_t x = v;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(x, o);
+        if (lane >= (uint32_t)o) x += t;
+      }
+      if (s + lane < ns) ct[(size_t)(s + lane) * n_classes + c] = run + x - v;
+      run += __shfl(x, 63);
+    }
+    if (lane == 0) {
+      tot[c] = run;
+      class_count[(size_t)im * n_classes + c] = run;
+    }
+  }
+  __syncthreads();
+  uint32_t carry = 0;
+  for (uint32_t s1 = 0; s1 < ns; s1 += 1024u) {
+    const uint32_t s = s1 + tid;
+    uint32_t d = 0;
+    if (s < ns)
+      for (uint32_t c = 0; c < n_classes; c++) {
+        const uint32_t st = ct[(size_t)s * n_classes + c];
+        const uint32_t en = s + 1u < ns ? ct[(size_t)(s + 1u) * n_classes + c] : tot[c];
+        const uint32_t from = st > sB[c] ? st : sB[c];
+        d += en > from ? en - from : 0u;
+      }
+    uint32_t x = d;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t t = __shfl_up(x, o);
+      if (lane >= (uint32_t)o) x += t;
+    }
+    if (lane == 63u) ws[wave] = x;
+    __syncthreads();
+    uint32_t before = carry;
+    for (uint32_t w = 0; w < 16u; w++) {
+      const uint32_t t = ws[w];
+      if (w < wave) before += t;
+      carry += t;
+    }
+    if (s < ns) seg_draw[s0 + s] = uint2{before + x - d, d};
+    __syncthreads();
+  }
+}
+
+// One wave per segment, 64 pixels per step in scan order.  A pixel's class
+// ordinal is the count so far (LDS, from the segment's start) plus its rank
+// among the wave's lanes of that class; it draws iff the ordinal is at least
+// B_c, and its draw index is the wave prefix of those flags.  bucket:
+// zero-initialised slots [image][sum B] (class c at boff[c]) filled with
+// atomicMax (the last writer in scan order has the largest pixel index).  Draws
+// outside the window [w0, w0 + win) are another launch's; pixels that do not
+// draw belong to the first one's.  Bound by VALU issue (about 90 operations a
+// step).
+__global__ __launch_bounds__(256) void k_weighted_draw(const uint8_t *__restrict__ labels,
+                                                       const SampleJob *__restrict__ jobs, uint32_t n_images,
+                                                       const uint32_t *__restrict__ seg0, uint32_t n_segs,
+                                                       uint32_t seg_len, uint32_t n_classes,
+                                                       const uint32_t *__restrict__ B,
+                                                       const uint32_t *__restrict__ boff, uint32_t w0, uint32_t win,
+                                                       const uint32_t *__restrict__ draws,
+                                                       const uint32_t *__restrict__ counts,
+                                                       const uint2 *__restrict__ seg_draw, uint32_t *bucket)
+{
+  __shared__ uint32_t sB[256], sO[256], cnt_all[4][256];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  sB[tid] = tid < n_classes ? B[tid] : 0u;
+  sO[tid] = tid < n_classes ? boff[tid] : 0u;
+  __syncthreads();  // the only block-wide barrier: from here on the waves are independent
+  const uint32_t seg = blockIdx.x * 4u + wave;
+  if (seg >= n_segs) return;
+  const uint2 sd = seg_draw[seg];
+  if (w0 != 0u && (sd.x + sd.y <= w0 || sd.x - w0 >= win)) return;
+  uint32_t *cnt = cnt_all[wave];
+  for (uint32_t c = lane; c < n_classes; c += 64u) cnt[c] = counts[(size_t)seg * n_classes + c];
+  const uint32_t im = find_owner(seg0, n_images, seg);
+  const SampleJob J = jobs[im];
+  const uint8_t *lab = labels + J.lab_off;
+  const uint32_t *x = draws + (size_t)im * win;
+  uint32_t *bk = bucket + J.out_base;
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
+  const uint32_t p0 = (seg - seg0[im]) * seg_len, p1 = J.n_px - p0 < seg_len ? J.n_px : p0 + seg_len;
+  uint32_t D = sd.x;
+  wave_sync();
+  for (uint32_t t = p0; t < p1; t += 1024u) {
+    uint32_t cur[16];
+#pragma unroll
+    for (uint32_t s = 0; s < 16u; s++) cur[s] = t + 64u * s + lane < p1 ? lab[t + 64u * s + lane] : 0u;
+#pragma unroll
+    for (uint32_t s = 0; s < 16u; s++) {
+      if (t + 64u * s >= p1) break;
+      const uint32_t p = t + 64u * s + lane;
+      const uint32_t l = cur[s] <= n_classes ? cur[s] : 0u;
       uint32_t k = 0, Bc = 0, Oc = 0;
-      uint64_t pending = __ballot(valid);
-      while (pending) {
-        const uint32_t lead = (uint32_t)__builtin_ctzll(pending);
-        const uint32_t cl = __builtin_amdgcn_readlane(c, lead);
-        const uint64_t mm = __ballot(valid && c == cl);
-        const uint32_t before = cnt[cl], bcl = sB[cl], ocl = sO[cl];
-        if (valid && c == cl) {
+      each_class(l, [&](uint32_t c, uint64_t mm) {
+        const uint32_t before = cnt[c], b = sB[c], o = sO[c];
+        if (l == c + 1u) {
           k = before + (uint32_t)__popcll(mm & lt);
-          Bc = bcl;
-          Oc = ocl;
+          Bc = b;
+          Oc = o;
         }
-        if (lane == lead) cnt[cl] = before + (uint32_t)__popcll(mm);
-        pending &= ~mm;
-      }
-      const bool draw = valid && k >= Bc;
+        if (lane == 0) cnt[c] = before + (uint32_t)__popcll(mm);
+      });
+      const bool draw = l != 0u && k >= Bc;
       const uint64_t dm = __ballot(draw);
-      const uint32_t d = D + (uint32_t)__popcll(dm & lt);
+      const uint32_t d = D + (uint32_t)__popcll(dm & lt) - w0;   // (wraps below the window)
       D += (uint32_t)__popcll(dm);
-      uint32_t x = 0;
-      if (D > gen) {  // wave-uniform: this step crosses into the next twist
-        if (draw && d < gen) x = mt[d + MT_N - gen];
-        mt_twist_wave(mt, lane);
-        gen += MT_N;
-        if (draw && d + MT_N >= gen) x = mt[d + MT_N - gen];
-      } else if (draw) {
-        x = mt[d + MT_N - gen];
-      }
       if (draw) {
-        const double u = (double)mt_temper(x) * 2.3283064365386962890625e-10;  // x / 2^32
-        const uint32_t j = (uint32_t)roundf((float)(u * (double)k));
-        if (j < Bc) atomicMax(&bk[Oc + j], p);
-      } else if (valid) {
+        if (d < win) {
+          const double u = (double)x[d] * 2.3283064365386962890625e-10;  // x / 2^32
+          const uint32_t j = (uint32_t)roundf((float)(u * (double)k));
+          if (j < Bc) atomicMax(&bk[Oc + j], p);
+        }
+      } else if (l != 0u && w0 == 0u) {
         atomicMax(&bk[Oc + k], p);
       }
     }
   }
-  wave_sync();
-  for (uint32_t c = lane; c < n_classes; c += 64u) class_count[(uint64_t)im * n_classes + c] = cnt[c];
 }
 
 // filled slots of every class -> contiguous unsorted samples; segment end

@@ -27,6 +27,7 @@ namespace {
 struct IngestDev {
   std::recursive_mutex mu;
   hipStream_t stream = nullptr;
+  DevBuf draws, mt_state, seg_counts, seg_draw;   // class-weighted sampler
   DevBuf jobs, blk0, P, gap, acc, crc, sjobs, tile0, bits, cnt, pre, scan_tmp, unsorted, bucket, class_count, B,
       boff, seg_begin, seg_end, sort_tmp, bad, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
   std::vector<uint32_t> hP;  // x^(8 * 4096 j) mod P
@@ -38,6 +39,7 @@ struct IngestDev {
 };
 
 constexpr CrcTables HT = make_crc_tables();
+constexpr uint64_t WEIGHTED_WORDS = 16ull << 20;   // stream words of the class-weighted sampler at a time (64 MiB)
 using Lock = std::lock_guard<std::recursive_mutex>;
 
 IngestDev &ctx(int device)
@@ -250,9 +252,39 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
                        X.bucket.as<uint32_t>(), (uint64_t)n * cap, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, X.bad.as<uint32_t>(), 1ull, 0u);
     tm.mark(2);
-    hipLaunchKernelGGL(k_sample_weighted, dim3((n + 3) / 4), dim3(256), 0, st, d_labels, X.sjobs.as<SampleJob>(), n,
-                       crc, s.seed, s.n_classes, X.B.as<uint32_t>(), X.boff.as<uint32_t>(), X.bucket.as<uint32_t>(),
-                       X.class_count.as<uint32_t>(), X.bad.as<uint32_t>());
+    // segments of whole 1024-pixel steps, about 16384 in the batch (64 waves a
+    // CU); the streams' windows share WEIGHTED_WORDS words
+    const uint32_t seg_len = (uint32_t)((std::max<uint64_t>(label_bytes / 16384u, 1) + 1023u) / 1024u * 1024u);
+    std::vector<uint32_t> &seg0 = X.h_tile0;   // (the uniform sampler's tiles are not used here)
+    uint64_t segs = 0;
+    for (uint32_t i = 0; i < n; i++) {
+      seg0[i] = (uint32_t)segs;
+      segs += (jobs[i].n_px + (uint64_t)seg_len - 1) / seg_len;
+    }
+    upload(X.tile0, seg0, st);
+    const uint32_t n_segs = (uint32_t)segs;
+    const uint64_t share = std::min<uint64_t>(std::max<uint64_t>(max_px, 1), std::max<uint64_t>(WEIGHTED_WORDS / n, 1));
+    const uint32_t win = (uint32_t)((share + MT_STEP - 1) / MT_STEP * MT_STEP);
+    X.draws.ensure((size_t)n * win * 4u);
+    if (max_px > win) X.mt_state.ensure((size_t)n * MT_N * 4u);
+    X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
+    X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
+    for (uint64_t w0 = 0; w0 == 0 || w0 < max_px; w0 += win) {
+      const uint32_t cb = w0 == 0 ? (n_segs + 3) / 4 : 0u;
+      hipLaunchKernelGGL(k_weighted_count, dim3(n + cb), dim3(256), 0, st, d_labels, X.sjobs.as<SampleJob>(), n,
+                         X.tile0.as<uint32_t>(), n_segs, seg_len, crc, s.seed, s.n_classes, (uint32_t)w0, win,
+                         X.draws.as<uint32_t>(), X.mt_state.as<uint32_t>(), X.seg_counts.as<uint32_t>(),
+                         X.bad.as<uint32_t>());
+      if (w0 == 0)
+        hipLaunchKernelGGL(k_weighted_scan, dim3(n), dim3(1024), 0, st, X.tile0.as<uint32_t>(), n, n_segs,
+                           s.n_classes, X.B.as<uint32_t>(), X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
+                           X.class_count.as<uint32_t>());
+      if (n_segs)
+        hipLaunchKernelGGL(k_weighted_draw, dim3((n_segs + 3) / 4), dim3(256), 0, st, d_labels,
+                           X.sjobs.as<SampleJob>(), n, X.tile0.as<uint32_t>(), n_segs, seg_len, s.n_classes,
+                           X.B.as<uint32_t>(), X.boff.as<uint32_t>(), (uint32_t)w0, win, X.draws.as<uint32_t>(),
+                           X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(), X.bucket.as<uint32_t>());
+    }
     hipLaunchKernelGGL(k_compact_buckets, dim3(n), dim3(256), 0, st, X.sjobs.as<SampleJob>(), s.n_classes,
                        X.B.as<uint32_t>(), X.boff.as<uint32_t>(), X.class_count.as<uint32_t>(),
                        X.bucket.as<uint32_t>(), uns, d_n_out, X.seg_end.as<uint32_t>());

@@ -123,6 +123,21 @@ def test_weighted_sampler_matches_oracle(gpu, n_classes, weights, n_samples):
         assert np.array_equal(g, w), i
 
 
+@pytest.mark.parametrize("shapes,n_samples", [
+    ([(32, 32), (1, 1025), (1, 1023), (48, 64), (1, 1)], 40),   # whole segments, one pixel more and less
+    ([(4100, 4100), (37, 61), (227, 4)], 500),                         # several windows of the draw streams
+])
+def test_weighted_sampler_segments_and_windows(gpu, shapes, n_samples):
+    rng = np.random.default_rng(n_samples)
+    labs = [rng.integers(0, 6, s).astype(np.uint8) for s in shapes]
+    datas = [rng.integers(0, 65536, s, dtype=np.uint16) for s in shapes]
+    smp = ds.ClassWeightedImageSampler(n_samples, 5, None, seed=9)
+    got = smp.sample_batch(datas, labs)
+    want, _ = oi.sample_images(1, datas, labs, n_samples, 5, None, seed=9)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert np.array_equal(g, w), i
+
+
 def test_weighted_sampler_rejects_label_above_classes(gpu):
     lab = np.array([[1, 2, 5]], np.uint8)
     with pytest.raises(pa.PdError, match="exceeds n_classes"):
