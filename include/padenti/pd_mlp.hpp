@@ -20,14 +20,14 @@
 //                 tix()) from L2 through a register ring that runs ahead over
 //                 the layers; two waves per SIMD (registers capped at 256), so
 //                 one wave's epilogue overlaps another's MFMAs.  Bound by the
-//                 epilogue's VALU work: 2^20 rows 640 us (456 TFLOP/s) at first,
-//                 455 with the constants of the GELU folded, packed BF16
+//                 epilogue's VALU work: 2^20 rows 560 us (520 TFLOP/s) at first,
+//                 400 with the constants of the GELU folded, packed BF16
 //                 conversion, 8-byte LDS stores and the output layer on the
-//                 matrix cores, 380 (768 TFLOP/s) with the ring: VALU pipe 76%
+//                 matrix cores, 340 (860 TFLOP/s) with the ring: VALU pipe 76%
 //                 busy (7.5 operations an activation), matrix cores 40%.
 //                 Batches of 4096 training rows: 17.4 -> 12.4 us, the backward
 //                 15.5 -> 10.0 us (waits for L2 loads).
-//                 MFMAs.  Training mode also stores the BF16 GELU
+//                 Training mode also stores the BF16 GELU
 //                 derivatives G = gelu'(z) of the pre-activations (the
 //                 backward multiplies by them) and the BF16 activations H in
 //                 MFMA fragment blocks

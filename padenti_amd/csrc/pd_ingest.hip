@@ -28,14 +28,16 @@ struct IngestDev {
   std::recursive_mutex mu;
   hipStream_t stream = nullptr;
   DevBuf draws, mt_state, seg_counts, seg_draw;   // class-weighted sampler
-  DevBuf jobs, blk0, P, gap, acc, crc, sjobs, tile0, bits, cnt, pre, scan_tmp, unsorted, bucket, class_count, B,
-      boff, seg_begin, seg_end, sort_tmp, bad, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
+  DevBuf tables, P, gap, crc, bits, cnt, pre, scan_tmp, unsorted, bucket, class_count, seg_end, sort_tmp, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
   std::vector<uint32_t> hP;  // x^(8 * 4096 j) mod P
   std::vector<uint32_t> hgap;  // [4][256]: byte k of a register times x^(8 * CRC_GAP)
   std::vector<CrcJob> h_jobs;
   std::vector<SampleJob> h_sjobs;
   std::vector<uint32_t> h_blk0, h_tile0, h_seg_begin, h_B, h_boff, h_keys;
-  std::vector<uint8_t> h_cls, h_stage;
+  std::vector<uint8_t> h_cls, h_stage, h_tables;
+  std::vector<Event> ev{5};   // stage times (Timer)
+  size_t n_P = 0;   // entries of P and whether gap are on the device (constants)
+  bool have_gap = false;
 };
 
 constexpr CrcTables HT = make_crc_tables();
@@ -61,6 +63,37 @@ void upload(DevBuf &b, const std::vector<T> &v, hipStream_t s)
   b.ensure(std::max<size_t>(v.size(), 1) * sizeof(T));
   if (!v.empty()) HIPCHK(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
 }
+
+// The host tables of a call in one buffer and one copy (a copy costs about 3 us
+// of the GPU's time and as much of the host's).
+struct Tables {
+  IngestDev &X;
+  explicit Tables(IngestDev &x) : X(x) { X.h_tables.clear(); }
+  size_t reserve(size_t bytes)   // zeros
+  {
+    const size_t o = X.h_tables.size();
+    X.h_tables.resize(o + ((bytes + 15) & ~(size_t)15), 0);
+    return o;
+  }
+  template <class T>
+  size_t add(const std::vector<T> &v)
+  {
+    const size_t o = reserve(v.size() * sizeof(T));
+    if (!v.empty()) std::memcpy(X.h_tables.data() + o, v.data(), v.size() * sizeof(T));
+    return o;
+  }
+  void commit()
+  {
+    X.tables.ensure(std::max<size_t>(X.h_tables.size(), 16));
+    if (!X.h_tables.empty())
+      HIPCHK(hipMemcpyAsync(X.tables.p, X.h_tables.data(), X.h_tables.size(), hipMemcpyHostToDevice, X.stream));
+  }
+  template <class T>
+  T *at(size_t o) const
+  {
+    return (T *)((char *)X.tables.p + o);
+  }
+};
 
 uint32_t grid_for(uint64_t n, uint32_t per_block, uint32_t cap = 65535u * 16u)
 {
@@ -102,60 +135,75 @@ void check_ranges(uint32_t n, const uint64_t *off, const uint64_t *bytes, uint64
             std::string(what) + " range " + std::to_string(i) + " lies outside its buffer");
 }
 
-// CRC jobs of n byte ranges of `base` (checked by the caller); launches
-// zero-fill, the block kernel and the finalisation on the context stream,
-// crc -> d_crc.
-void launch_crc(IngestDev &X, uint32_t n, const uint8_t *base, const uint64_t *off, const uint64_t *bytes,
-                uint32_t *d_crc)
-{
-  std::vector<CrcJob> &jobs = X.h_jobs;
-  std::vector<uint32_t> &chunk0 = X.h_blk0;
-  jobs.assign(n, CrcJob{});
-  chunk0.assign(n, 0u);
-  uint64_t total = 0;  // chunks
-  uint32_t max_nb = 0;
-  for (uint32_t i = 0; i < n; i++) {
-    CrcJob &J = jobs[i];
-    J.start = (uint64_t)(uintptr_t)base + off[i];
-    J.end = J.start + bytes[i];
-    J.a0 = J.start & ~63ull;
-    const uint64_t nb = bytes[i] ? (J.end - J.a0 + 4095u) / 4096u : 0u;
-    require(nb < (1ull << 32) && total + nb < (1ull << 32), "too many bytes in one CRC batch");
-    J.first_chunk = chunk0[i] = (uint32_t)total;
-    J.n_blocks = (uint32_t)nb;
-    total += (nb + CRC_CHUNK - 1) / CRC_CHUNK;
-    max_nb = std::max<uint32_t>(max_nb, (uint32_t)nb);
+// CRC of n byte ranges of `base` (checked by the caller): add() puts its tables
+// into t, launch() runs the block kernel and the finalisation on the context
+// stream, crc -> d_crc.
+struct CrcBatch {
+  IngestDev &X;
+  Tables &t;
+  uint32_t n = 0, total = 0;
+  size_t jobs_o = 0, chunk0_o = 0, acc_o = 0;
+  void add(uint32_t n_, const uint8_t *base, const uint64_t *off, const uint64_t *bytes)
+  {
+    n = n_;
+    std::vector<CrcJob> &jobs = X.h_jobs;
+    std::vector<uint32_t> &chunk0 = X.h_blk0;
+    jobs.assign(n, CrcJob{});
+    chunk0.assign(n, 0u);
+    uint64_t chunks = 0;
+    uint32_t max_nb = 0;
+    for (uint32_t i = 0; i < n; i++) {
+      CrcJob &J = jobs[i];
+      J.start = (uint64_t)(uintptr_t)base + off[i];
+      J.end = J.start + bytes[i];
+      J.a0 = J.start & ~63ull;
+      const uint64_t nb = bytes[i] ? (J.end - J.a0 + 4095u) / 4096u : 0u;
+      require(nb < (1ull << 32) && chunks + nb < (1ull << 32), "too many bytes in one CRC batch");
+      J.first_chunk = chunk0[i] = (uint32_t)chunks;
+      J.n_blocks = (uint32_t)nb;
+      chunks += (nb + CRC_CHUNK - 1) / CRC_CHUNK;
+      max_nb = std::max<uint32_t>(max_nb, (uint32_t)nb);
+    }
+    total = (uint32_t)chunks;
+    if (X.hP.empty()) X.hP.push_back(CRC_ONE);
+    while (X.hP.size() < max_nb) X.hP.push_back(gf2_mul(X.hP.back(), HT.x2k[15]));  // * x^(8 * 4096)
+    if (X.hgap.empty()) {
+      const uint32_t C = crc_x8n(HT, CRC_GAP);
+      X.hgap.resize(1024);
+      for (uint32_t k = 0; k < 4; k++)
+        for (uint32_t v = 0; v < 256; v++) X.hgap[k * 256 + v] = gf2_mul(v << (8 * k), C);
+    }
+    jobs_o = t.add(jobs);
+    chunk0_o = t.add(chunk0);
+    acc_o = t.reserve(2ull * n * 4u);   // the two accumulators, zero
   }
-  if (X.hP.empty()) X.hP.push_back(CRC_ONE);
-  while (X.hP.size() < max_nb) X.hP.push_back(gf2_mul(X.hP.back(), HT.x2k[15]));  // * x^(8 * 4096)
-  if (X.hgap.empty()) {
-    const uint32_t C = crc_x8n(HT, CRC_GAP);
-    X.hgap.resize(1024);
-    for (uint32_t k = 0; k < 4; k++)
-      for (uint32_t v = 0; v < 256; v++) X.hgap[k * 256 + v] = gf2_mul(v << (8 * k), C);
+  void launch(uint32_t *d_crc)
+  {
+    if (X.n_P < X.hP.size()) {
+      upload(X.P, X.hP, X.stream);
+      X.n_P = X.hP.size();
+    }
+    if (!X.have_gap) {
+      upload(X.gap, X.hgap, X.stream);
+      X.have_gap = true;
+    }
+    uint32_t *acc = t.at<uint32_t>(acc_o);
+    if (total)
+      hipLaunchKernelGGL(k_crc32, dim3(grid_for(total, 4, 1u << 20)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o),
+                         t.at<uint32_t>(chunk0_o), n, total, X.P.as<uint32_t>(), X.gap.as<uint32_t>(), acc, acc + n);
+    hipLaunchKernelGGL(k_crc_final, dim3(grid_for(n, 4)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o), n, acc, acc + n,
+                       d_crc);
+    HIPCHK(hipGetLastError());
   }
-  upload(X.jobs, jobs, X.stream);
-  upload(X.blk0, chunk0, X.stream);
-  upload(X.P, X.hP, X.stream);
-  upload(X.gap, X.hgap, X.stream);
-  X.acc.ensure(2ull * std::max<uint32_t>(n, 1) * 4u);
-  uint32_t *acc = X.acc.as<uint32_t>();
-  hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2ull * n, 256)), dim3(256), 0, X.stream, acc, 2ull * n, 0u);
-  if (total)
-    hipLaunchKernelGGL(k_crc32, dim3(grid_for(total, 4, 1u << 20)), dim3(256), 0, X.stream, X.jobs.as<CrcJob>(),
-                       X.blk0.as<uint32_t>(), n, (uint32_t)total, X.P.as<uint32_t>(), X.gap.as<uint32_t>(), acc,
-                       acc + n);
-  hipLaunchKernelGGL(k_crc_final, dim3(grid_for(n, 64)), dim3(64), 0, X.stream, X.jobs.as<CrcJob>(), n, acc,
-                     acc + n, d_crc);
-  HIPCHK(hipGetLastError());
-}
+};
 
+// Stage times from the context's events (creating five a call cost the host more
+// than recording them)
 struct Timer {
-  hipStream_t s;
-  std::vector<Event> ev;
-  explicit Timer(hipStream_t st, int n) : s(st), ev(n) {}
-  void mark(int i) { HIPCHK(hipEventRecord(ev[i].e, s)); }
-  float ms(int a, int b) const { return (float)elapsed_ms(ev[a], ev[b]); }
+  IngestDev &X;
+  explicit Timer(IngestDev &x) : X(x) {}
+  void mark(int i) { HIPCHK(hipEventRecord(X.ev[i].e, X.stream)); }
+  float ms(int a, int b) const { return (float)elapsed_ms(X.ev[a], X.ev[b]); }
 };
 
 void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data, uint64_t data_size,
@@ -207,62 +255,69 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
   }
   require(n_words < (1ull << 31) && n_tiles < (1ull << 31), "too many pixels in one batch");
 
-  Timer tm(st, 5);
+  Timer tm(X);
   tm.mark(0);
   X.crc.ensure((size_t)n * 4u);
   uint32_t *crc = d_crc ? d_crc : X.crc.as<uint32_t>();
-  launch_crc(X, n, (const uint8_t *)d_data, data_off, data_bytes, crc);
+  Tables tab(X);
+  CrcBatch cb{X, tab};
+  cb.add(n, (const uint8_t *)d_data, data_off, data_bytes);
+  const bool weighted = s.kind == PD_SAMPLER_CLASS_WEIGHTED;
+  // class-weighted: segments of whole 1024-pixel steps, about 16384 in the batch
+  // (64 waves a CU)
+  const uint32_t seg_len = (uint32_t)((std::max<uint64_t>(label_bytes / 16384u, 1) + 1023u) / 1024u * 1024u);
+  uint32_t n_segs = 0;
+  if (weighted) {
+    uint64_t segs = 0;
+    for (uint32_t i = 0; i < n; i++) {
+      tile0[i] = (uint32_t)segs;
+      segs += (jobs[i].n_px + (uint64_t)seg_len - 1) / seg_len;
+    }
+    n_segs = (uint32_t)segs;
+    std::vector<uint32_t> &B = X.h_B, &boff = X.h_boff;
+    B = bucket_sizes(s);
+    boff.assign(s.n_classes, 0u);
+    uint32_t o = 0;
+    for (uint32_t c = 0; c < s.n_classes; c++) { boff[c] = o; o += B[c]; }
+  }
+  const size_t o_jobs = tab.add(jobs), o_begin = tab.add(seg_begin), o_first = tab.add(tile0);
+  const size_t o_B = weighted ? tab.add(X.h_B) : 0, o_boff = weighted ? tab.add(X.h_boff) : 0;
+  const size_t o_bad = tab.reserve(4);
+  tab.commit();
+  const SampleJob *d_jobs = tab.at<SampleJob>(o_jobs);
+  const uint32_t *d_begin = tab.at<uint32_t>(o_begin), *d_first = tab.at<uint32_t>(o_first);
+  const uint32_t *d_B = tab.at<uint32_t>(o_B), *d_boff = tab.at<uint32_t>(o_boff);
+  uint32_t *d_bad = tab.at<uint32_t>(o_bad);
+  cb.launch(crc);
   tm.mark(1);
-  upload(X.sjobs, jobs, st);
-  upload(X.seg_begin, seg_begin, st);
   X.seg_end.ensure((size_t)n * 4u);
   X.unsorted.ensure((size_t)n * cap * 4u + 4u);
   uint32_t *uns = X.unsorted.as<uint32_t>();
   if (s.kind == PD_SAMPLER_UNIFORM) {
     const uint32_t nw = (uint32_t)n_words;
-    upload(X.tile0, tile0, st);
     X.bits.ensure((size_t)nw * 4u + 4u);
     X.cnt.ensure(((size_t)nw + 1) * 4u);
     X.pre.ensure(((size_t)nw + 1) * 4u);
     uint32_t *cnt = X.cnt.as<uint32_t>();
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, cnt + nw, 1ull, 0u);
     if (n_tiles)
-      hipLaunchKernelGGL(k_label_bits, dim3((uint32_t)n_tiles), dim3(256), 0, st, d_labels, X.sjobs.as<SampleJob>(),
-                         X.tile0.as<uint32_t>(), n, X.bits.as<uint32_t>(), cnt);
+      hipLaunchKernelGGL(k_label_bits, dim3((uint32_t)n_tiles), dim3(256), 0, st, d_labels, d_jobs,
+                         d_first, n, X.bits.as<uint32_t>(), cnt);
     size_t tb = 0;
     HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt, X.pre.as<uint32_t>(), (int)nw + 1, st));
     X.scan_tmp.ensure(tb);
     HIPCHK(hipcub::DeviceScan::ExclusiveSum(X.scan_tmp.p, tb, cnt, X.pre.as<uint32_t>(), (int)nw + 1, st));
     tm.mark(2);
-    hipLaunchKernelGGL(k_sample_uniform, dim3(n), dim3(256), 0, st, X.sjobs.as<SampleJob>(), X.bits.as<uint32_t>(),
+    hipLaunchKernelGGL(k_sample_uniform, dim3(n), dim3(256), 0, st, d_jobs, X.bits.as<uint32_t>(),
                        X.pre.as<uint32_t>(), crc, s.seed, s.n_samples, uns, d_n_out, X.seg_end.as<uint32_t>());
     HIPCHK(hipGetLastError());
   } else {
-    std::vector<uint32_t> &B = X.h_B, &boff = X.h_boff;
-    B = bucket_sizes(s);
-    boff.assign(s.n_classes, 0u);
-    uint32_t o = 0;
-    for (uint32_t c = 0; c < s.n_classes; c++) { boff[c] = o; o += B[c]; }
-    upload(X.B, B, st);
-    upload(X.boff, boff, st);
     X.bucket.ensure((size_t)n * cap * 4u + 4u);
     X.class_count.ensure((size_t)n * s.n_classes * 4u);
-    X.bad.ensure(4);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for((uint64_t)n * cap, 256)), dim3(256), 0, st,
                        X.bucket.as<uint32_t>(), (uint64_t)n * cap, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, X.bad.as<uint32_t>(), 1ull, 0u);
     tm.mark(2);
-    // segments of whole 1024-pixel steps, about 16384 in the batch (64 waves a
-    // CU); the streams' windows share WEIGHTED_WORDS words
-    const uint32_t seg_len = (uint32_t)((std::max<uint64_t>(label_bytes / 16384u, 1) + 1023u) / 1024u * 1024u);
-    std::vector<uint32_t> &seg0 = X.h_tile0;   // (the uniform sampler's tiles are not used here)
-    uint64_t segs = 0;
-    for (uint32_t i = 0; i < n; i++) {
-      seg0[i] = (uint32_t)segs;
-      segs += (jobs[i].n_px + (uint64_t)seg_len - 1) / seg_len;
-    }
-    upload(X.tile0, seg0, st);
-    const uint32_t n_segs = (uint32_t)segs;
+    // the streams' windows share WEIGHTED_WORDS words
     const uint64_t share = std::min<uint64_t>(std::max<uint64_t>(max_px, 1), std::max<uint64_t>(WEIGHTED_WORDS / n, 1));
     const uint32_t win = (uint32_t)((share + MT_STEP - 1) / MT_STEP * MT_STEP);
     X.draws.ensure((size_t)n * win * 4u);
@@ -270,23 +325,23 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
     X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
     X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
     for (uint64_t w0 = 0; w0 == 0 || w0 < max_px; w0 += win) {
-      const uint32_t cb = w0 == 0 ? (n_segs + 3) / 4 : 0u;
-      hipLaunchKernelGGL(k_weighted_count, dim3(n + cb), dim3(256), 0, st, d_labels, X.sjobs.as<SampleJob>(), n,
-                         X.tile0.as<uint32_t>(), n_segs, seg_len, crc, s.seed, s.n_classes, (uint32_t)w0, win,
+      const uint32_t count_blocks = w0 == 0 ? (n_segs + 3) / 4 : 0u;
+      hipLaunchKernelGGL(k_weighted_count, dim3(n + count_blocks), dim3(256), 0, st, d_labels, d_jobs, n,
+                         d_first, n_segs, seg_len, crc, s.seed, s.n_classes, (uint32_t)w0, win,
                          X.draws.as<uint32_t>(), X.mt_state.as<uint32_t>(), X.seg_counts.as<uint32_t>(),
-                         X.bad.as<uint32_t>());
+                         d_bad);
       if (w0 == 0)
-        hipLaunchKernelGGL(k_weighted_scan, dim3(n), dim3(1024), 0, st, X.tile0.as<uint32_t>(), n, n_segs,
-                           s.n_classes, X.B.as<uint32_t>(), X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
+        hipLaunchKernelGGL(k_weighted_scan, dim3(n), dim3(1024), 0, st, d_first, n, n_segs,
+                           s.n_classes, d_B, X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
                            X.class_count.as<uint32_t>());
       if (n_segs)
         hipLaunchKernelGGL(k_weighted_draw, dim3((n_segs + 3) / 4), dim3(256), 0, st, d_labels,
-                           X.sjobs.as<SampleJob>(), n, X.tile0.as<uint32_t>(), n_segs, seg_len, s.n_classes,
-                           X.B.as<uint32_t>(), X.boff.as<uint32_t>(), (uint32_t)w0, win, X.draws.as<uint32_t>(),
+                           d_jobs, n, d_first, n_segs, seg_len, s.n_classes,
+                           d_B, d_boff, (uint32_t)w0, win, X.draws.as<uint32_t>(),
                            X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(), X.bucket.as<uint32_t>());
     }
-    hipLaunchKernelGGL(k_compact_buckets, dim3(n), dim3(256), 0, st, X.sjobs.as<SampleJob>(), s.n_classes,
-                       X.B.as<uint32_t>(), X.boff.as<uint32_t>(), X.class_count.as<uint32_t>(),
+    hipLaunchKernelGGL(k_compact_buckets, dim3(n), dim3(256), 0, st, d_jobs, s.n_classes,
+                       d_B, d_boff, X.class_count.as<uint32_t>(),
                        X.bucket.as<uint32_t>(), uns, d_n_out, X.seg_end.as<uint32_t>());
     HIPCHK(hipGetLastError());
   }
@@ -295,19 +350,17 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
   while (end_bit < 32 && (1ull << end_bit) < max_px) end_bit++;
   size_t sb = 0;
   HIPCHK(hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, sb, uns, d_samples, (int)((uint64_t)n * cap), (int)n,
-                                                     X.seg_begin.as<uint32_t>(), X.seg_end.as<uint32_t>(), 0,
+                                                     d_begin, X.seg_end.as<const uint32_t>(), 0,
                                                      end_bit, st));
   X.sort_tmp.ensure(sb);
   HIPCHK(hipcub::DeviceSegmentedRadixSort::SortKeys(X.sort_tmp.p, sb, uns, d_samples, (int)((uint64_t)n * cap),
-                                                     (int)n, X.seg_begin.as<uint32_t>(), X.seg_end.as<uint32_t>(),
+                                                     (int)n, d_begin, X.seg_end.as<const uint32_t>(),
                                                      0, end_bit, st));
   tm.mark(4);
+  uint32_t bad = 0;
+  if (weighted) HIPCHK(hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (s.kind == PD_SAMPLER_CLASS_WEIGHTED) {
-    uint32_t bad = 0;
-    HIPCHK(hipMemcpy(&bad, X.bad.p, 4, hipMemcpyDeviceToHost));
-    require(bad == 0, "a label exceeds n_classes");
-  }
+  require(bad == 0, "a label exceeds n_classes");
   if (stats) {
     stats->crc_ms = tm.ms(0, 1);
     stats->index_ms = s.kind == PD_SAMPLER_UNIFORM ? tm.ms(1, 2) : 0.f;
@@ -418,9 +471,13 @@ int pd_crc32_images_dev(int device, uint32_t n, const void *d_data, uint64_t dat
     set_device(device);
     IngestDev &X = ctx(device);
     Lock g(X.mu);
-    Timer tm(X.stream, 2);
+    Timer tm(X);
     tm.mark(0);
-    launch_crc(X, n, (const uint8_t *)d_data, offsets, bytes, d_crc);
+    Tables tab(X);
+    CrcBatch cb{X, tab};
+    cb.add(n, (const uint8_t *)d_data, offsets, bytes);
+    tab.commit();
+    cb.launch(d_crc);
     tm.mark(1);
     HIPCHK(hipStreamSynchronize(X.stream));
     if (kernel_ms) *kernel_ms = tm.ms(0, 1);
@@ -441,7 +498,7 @@ int pd_rgb_to_labels_dev(int device, uint64_t n_pixels, uint32_t channels, const
     rgb_keys(rgb2label, n_classes, keys, cls);
     upload(X.keys, keys, X.stream);
     upload(X.cls, cls, X.stream);
-    Timer tm(X.stream, 2);
+    Timer tm(X);
     tm.mark(0);
     if (n_pixels)
       hipLaunchKernelGGL(k_rgb_labels, dim3(grid_for(n_pixels, 256, 1u << 16)), dim3(256), 0, X.stream, d_rgb,
