@@ -28,7 +28,7 @@ struct IngestDev {
   std::recursive_mutex mu;
   hipStream_t stream = nullptr;
   DevBuf draws, mt_state, seg_counts, seg_draw;   // class-weighted sampler
-  DevBuf tables, P, gap, crc, bits, cnt, pre, scan_tmp, unsorted, bucket, class_count, seg_end, sort_tmp, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
+  DevBuf tables, P, gap, crc, bits, cnt, pre, unsorted, bucket, class_count, seg_end, sort_tmp, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
   std::vector<uint32_t> hP;  // x^(8 * 4096 j) mod P
   std::vector<uint32_t> hgap;  // [4][256]: byte k of a register times x^(8 * CRC_GAP)
   std::vector<CrcJob> h_jobs;
@@ -296,20 +296,15 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
   if (s.kind == PD_SAMPLER_UNIFORM) {
     const uint32_t nw = (uint32_t)n_words;
     X.bits.ensure((size_t)nw * 4u + 4u);
-    X.cnt.ensure(((size_t)nw + 1) * 4u);
-    X.pre.ensure(((size_t)nw + 1) * 4u);
-    uint32_t *cnt = X.cnt.as<uint32_t>();
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, cnt + nw, 1ull, 0u);
+    X.cnt.ensure((size_t)n_tiles * 4u + 4u);
+    X.pre.ensure((size_t)nw * 2u + 4u);
     if (n_tiles)
-      hipLaunchKernelGGL(k_label_bits, dim3((uint32_t)n_tiles), dim3(256), 0, st, d_labels, d_jobs,
-                         d_first, n, X.bits.as<uint32_t>(), cnt);
-    size_t tb = 0;
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt, X.pre.as<uint32_t>(), (int)nw + 1, st));
-    X.scan_tmp.ensure(tb);
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(X.scan_tmp.p, tb, cnt, X.pre.as<uint32_t>(), (int)nw + 1, st));
+      hipLaunchKernelGGL(k_label_bits, dim3((uint32_t)n_tiles), dim3(256), 0, st, d_labels, d_jobs, d_first, n,
+                         X.bits.as<uint32_t>(), X.pre.as<uint16_t>(), X.cnt.as<uint32_t>());
     tm.mark(2);
-    hipLaunchKernelGGL(k_sample_uniform, dim3(n), dim3(256), 0, st, d_jobs, X.bits.as<uint32_t>(),
-                       X.pre.as<uint32_t>(), crc, s.seed, s.n_samples, uns, d_n_out, X.seg_end.as<uint32_t>());
+    hipLaunchKernelGGL(k_sample_uniform, dim3(n), dim3(256), 0, st, d_jobs, d_first, n, (uint32_t)n_tiles,
+                       X.bits.as<uint32_t>(), X.pre.as<uint16_t>(), X.cnt.as<uint32_t>(), crc, s.seed, s.n_samples,
+                       uns, d_n_out, X.seg_end.as<uint32_t>());
     HIPCHK(hipGetLastError());
   } else {
     X.bucket.ensure((size_t)n * cap * 4u + 4u);
