@@ -155,6 +155,7 @@ struct MlpNet {
   uint32_t ldb = 0;   // batch stride of the training buffers (multiple of SPLIT)
   uint64_t t_step = 0;
   uint32_t n_xcc = 1;   // XCDs of the device (weight-gradient tiles are grouped per XCD)
+  PinnedStage stage;    // parameter transfers
 
   MlpNet(int dev, uint64_t seed)
   {
@@ -208,25 +209,29 @@ struct MlpNet {
   {
     hipLaunchKernelGGL(mlp::k_mlp_pack, dim3(mlp::HID * mlp::HID / 256), dim3(256), 0, stream, theta.as<float>(),
                        W1.as<uint16_t>(), W2.as<uint16_t>(), W2T.as<uint16_t>(), W3.as<uint16_t>(),
-                       W3T.as<uint16_t>(), w4.as<uint16_t>());
+                       W3T.as<uint16_t>(), w4.as<uint16_t>(), m.as<float>(), v.as<float>());
     HIPCHK(hipGetLastError());
   }
-  // new parameters; the Adam state restarts
+  // new parameters; the Adam state restarts (through pinned memory)
   void set_params(const float *h)
   {
     set_device(device);
-    HIPCHK(hipMemcpyAsync(theta.p, h, mlp::NPARAM * sizeof(float), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemsetAsync(m.p, 0, mlp::NPARAM * sizeof(float), stream));
-    HIPCHK(hipMemsetAsync(v.p, 0, mlp::NPARAM * sizeof(float), stream));
+    const size_t bytes = mlp::NPARAM * sizeof(float);
+    HIPCHK(hipMemcpyAsync(theta.p, stage.put(h, bytes), bytes, hipMemcpyHostToDevice, stream));
     t_step = 0;
     pack();
     HIPCHK(hipStreamSynchronize(stream));
+    stage.reset();
   }
   void get_params(float *h)
   {
     set_device(device);
-    HIPCHK(hipMemcpyAsync(h, theta.p, mlp::NPARAM * sizeof(float), hipMemcpyDeviceToHost, stream));
+    const size_t bytes = mlp::NPARAM * sizeof(float);
+    const char *pin = (const char *)stage.alloc(bytes);
+    HIPCHK(hipMemcpyAsync((void *)pin, theta.p, bytes, hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
+    std::copy(pin, pin + bytes, (char *)h);
+    stage.reset();
   }
   void ensure_batch(uint32_t B)
   {
@@ -260,6 +265,12 @@ struct MlpNet {
   // the step's mean squared error into loss_out (device pointers, may be null)
   void step(uint32_t n, bool update, const pd_adam &opt, float *grad_out, float *loss_out)
   {
+    step(Xb.as<uint16_t>(), tb.as<float>(), nullptr, n, update, opt, grad_out, loss_out);
+  }
+  // the same on the rows perm[0 .. n) of X / t
+  void step(const uint16_t *X, const float *t, const uint32_t *rows, uint32_t n, bool update, const pd_adam &opt,
+            float *grad_out, float *loss_out)
+  {
     require(n >= 1 && n <= ldb, "batch larger than the staged buffers");
     const uint32_t lrow = (n + mlp::SPLIT - 1) / mlp::SPLIT * mlp::SPLIT;
     // rows per weight-gradient partial: SPLIT doubled while it divides the
@@ -279,28 +290,28 @@ struct MlpNet {
     // forward row tile: 128 rows (half the weight re-reads of 64) once the
     // batch fills the chip with them, else 64 or 32 rows for more blocks
     const uint32_t fr = big ? 128u : (mid ? 64u : 32u);
-    const mlp::RowsMem src{Xb.as<uint16_t>(), n};
+    const mlp::RowsPerm src{X, rows, n};
     if (fr == 128u)
-      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsMem, true, 128>), dim3(lrow / 128u), dim3(mlp::THREADS), 0, stream,
+      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsPerm, true, 128>), dim3(lrow / 128u), dim3(mlp::THREADS), 0, stream,
                          src, n, w, yb.as<float>(), G.as<uint16_t>(), ht, ldb);
     else if (fr == 64u)
-      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsMem, true, 64>), dim3(lrow / 64u), dim3(mlp::THREADS), 0, stream,
+      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsPerm, true, 64>), dim3(lrow / 64u), dim3(mlp::THREADS), 0, stream,
                          src, n, w, yb.as<float>(), G.as<uint16_t>(), ht, ldb);
     else
-      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsMem, true, 32>), dim3(lrow / 32u), dim3(mlp::THREADS), 0, stream,
+      hipLaunchKernelGGL((mlp::k_mlp_fwd<mlp::RowsPerm, true, 32>), dim3(lrow / 32u), dim3(mlp::THREADS), 0, stream,
                          src, n, w, yb.as<float>(), G.as<uint16_t>(), ht, ldb);
     HIPCHK(hipGetLastError());
     if (big)
       hipLaunchKernelGGL(mlp::k_mlp_bwd<mlp::ROWS_BIG>, dim3(nblk), dim3(mlp::THREADS), 0, stream, yb.as<float>(),
-                         tb.as<float>(), n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
+                         t, rows, n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
                          lossp.as<float>(), ldb);
     else if (mid)
       hipLaunchKernelGGL(mlp::k_mlp_bwd<mlp::ROWS>, dim3(nblk), dim3(mlp::THREADS), 0, stream, yb.as<float>(),
-                         tb.as<float>(), n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
+                         t, rows, n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
                          lossp.as<float>(), ldb);
     else
       hipLaunchKernelGGL(mlp::k_mlp_bwd<mlp::ROWS_SMALL>, dim3(nblk), dim3(mlp::THREADS), 0, stream, yb.as<float>(),
-                         tb.as<float>(), n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
+                         t, rows, n, 1.0f / (float)n, G.as<uint16_t>(), w, dz, dy.as<float>(),
                          lossp.as<float>(), ldb);
     HIPCHK(hipGetLastError());
     float *pt = part.as<float>();
@@ -383,10 +394,7 @@ struct MlpNet {
       for (uint64_t sidx = 0; sidx < steps; sidx++) {
         const uint64_t base = sidx * B;
         const uint32_t cnt = (uint32_t)std::min<uint64_t>(B, N - base);
-        hipLaunchKernelGGL(mlp::k_mlp_gather, dim3((ldb * 4 + 255) / 256), dim3(256), 0, stream, X, t,
-                           perm.as<uint32_t>(), base, cnt, ldb, Xb.as<uint16_t>(), tb.as<float>());
-        HIPCHK(hipGetLastError());
-        step(cnt, true, opt, nullptr, lsteps.as<float>() + sidx);
+        step(X, t, perm.as<uint32_t>() + base, cnt, true, opt, nullptr, lsteps.as<float>() + sidx);
       }
       HIPCHK(hipEventRecord(e1.e, stream));
       HIPCHK(hipMemcpyAsync(ls.data(), lsteps.p, steps * sizeof(float), hipMemcpyDeviceToHost, stream));

@@ -44,7 +44,8 @@
 //                 from the weight-gradient blocks themselves).
 //   k_mlp_adam    sums the split partials in fixed order, applies Adam,
 //                 refreshes the BF16 weight copies and sums the step's loss.
-//   k_mlp_pack    FP32 master -> BF16 copies and transposed copies in fragment order.
+//   k_mlp_pack    FP32 master -> BF16 copies and transposed copies in fragment
+//                 order; clears the Adam state.
 //   k_topk        per node, the `keep` best of K scores (radix select on the
 //                 orderable score bits, ties to the lower candidate index),
 //                 written in increasing candidate order.
@@ -210,6 +211,18 @@ struct RowsMem {
   {
     if (row >= n) return make_uint4(0u, 0u, 0u, 0u);
     return *(const uint4 *)(X + (size_t)row * INP + q * 8);
+  }
+};
+
+// training rows: row r of the batch is row perm[r] of X (perm null: row r)
+struct RowsPerm {
+  const uint16_t *X;
+  const uint32_t *perm;
+  uint32_t n;
+  __device__ __forceinline__ uint4 fill(uint32_t row, uint32_t q) const
+  {
+    if (row >= n) return make_uint4(0u, 0u, 0u, 0u);
+    return *(const uint4 *)(X + (size_t)(perm ? perm[row] : row) * INP + q * 8);
   }
 };
 
@@ -407,7 +420,8 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
 }
 
 // Backward of the mean squared error L = 1/n sum_r (y_r - t_r)^2 over the
-// first n rows of the batch (rows n..ldb-1 are padding, dL/dy = 0 there).
+// first n rows of the batch (rows n..ldb-1 are padding, dL/dy = 0 there), the
+// target of row r being t[perm[r]] (perm null: t[r]).
 // DZT receives dL/dZ_{l+1} (BF16, element (256 l + unit, row) at tix()),
 // dy[ldb] FP32,
 // lossp[block] the block's sum of squared errors.  TR rows per block (64 or
@@ -415,7 +429,7 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_fwd(Src src, uint32_t n, Wei
 // first half of wave 0, the rest adding zeros).
 template <int TR>
 __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict__ y, const float *__restrict__ t,
-                                                     uint32_t n, float inv_n, const uint16_t *__restrict__ G,
+                                                     const uint32_t *__restrict__ perm, uint32_t n, float inv_n, const uint16_t *__restrict__ G,
                                                      Weights w, uint16_t *__restrict__ DZT, float *__restrict__ dy,
                                                      float *__restrict__ lossp, uint32_t ldb)
 {
@@ -448,7 +462,7 @@ __global__ __launch_bounds__(THREADS, 2) void k_mlp_bwd(const float *__restrict_
   if (tid < 64u * LW) {
     const uint32_t row = row0 + tid;
     const bool live = tid < (uint32_t)ROWS && row < n;
-    const float e = live ? y[row] - t[row] : 0.0f;
+    const float e = live ? y[row] - t[perm ? perm[row] : row] : 0.0f;
     const float d = live ? 2.0f * e * inv_n : 0.0f;
     if (tid < (uint32_t)ROWS) {
       dys[tid] = d;
@@ -874,9 +888,10 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ theta, flo
 // FP32 master -> BF16 working copies
 __global__ void k_mlp_pack(const float *__restrict__ theta, uint16_t *__restrict__ W1, uint16_t *__restrict__ W2,
                            uint16_t *__restrict__ W2T, uint16_t *__restrict__ W3, uint16_t *__restrict__ W3T,
-                           uint16_t *__restrict__ w4)
+                           uint16_t *__restrict__ w4, float *__restrict__ m, float *__restrict__ v)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t j = i; j < (uint32_t)NPARAM; j += gridDim.x * blockDim.x) m[j] = v[j] = 0.0f;
   if (i < (uint32_t)(HID * HID)) {
     const uint32_t nn = i / HID, k = i % HID;
     const uint16_t a = f2bf(theta[OFF_W2 + i]), b = f2bf(theta[OFF_W3 + i]);
@@ -890,25 +905,6 @@ __global__ void k_mlp_pack(const float *__restrict__ theta, uint16_t *__restrict
     W1[tix(nn, k, INP)] = k < (uint32_t)IN ? f2bf(theta[OFF_W1 + nn * IN + k]) : (uint16_t)0;
   }
   if (i < (uint32_t)HID) w4[i] = f2bf(theta[OFF_W4 + i]);
-}
-
-// batch gather: rows perm[base + i] of X / t into Xb / tb, zero padding to ldb
-__global__ void k_mlp_gather(const uint16_t *__restrict__ X, const float *__restrict__ t,
-                             const uint32_t *__restrict__ perm, uint64_t base, uint32_t count, uint32_t ldb,
-                             uint16_t *__restrict__ Xb, float *__restrict__ tb)
-{
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // (row, quarter)
-  const uint32_t r = i >> 2, q = i & 3u;
-  if (r >= ldb) return;
-  uint4 v = make_uint4(0u, 0u, 0u, 0u);
-  float tv = 0.0f;
-  if (r < count) {
-    const uint32_t src = perm[base + r];
-    v = *(const uint4 *)(X + (size_t)src * INP + q * 8);
-    tv = t[src];
-  }
-  *(uint4 *)(Xb + (size_t)r * INP + q * 8) = v;
-  if (q == 0) tb[r] = tv;
 }
 
 // ---------------------------------------------------------------------------

@@ -566,7 +566,10 @@ int pd_mlp_set_params(pd_mlp *m, const float *theta)
 {
   return guarded([&] {
     require(m && theta, "null argument");
-    for (int i = 0; i < mlp::NPARAM; i++) require(std::isfinite(theta[i]), "non-finite parameter");
+    // (one verdict for all: a message string per parameter took 870 us)
+    bool finite = true;
+    for (int i = 0; i < mlp::NPARAM; i++) finite = finite && std::isfinite(theta[i]);
+    require(finite, "non-finite parameter");
     m->impl->set_params(theta);
   });
 }
