@@ -510,10 +510,15 @@ __global__ __launch_bounds__(256) void k_sample_uniform(const SampleJob *__restr
 //                     every segment;
 //   k_weighted_draw   the segments' pixels, one wave a segment.
 // Only the stream is serial (454 words a step, below).  150 images of 321 x 243,
-// 16 classes: 846 us with one wave an image walking all of it, 102 us now.
+// 16 classes: 846 us with one wave an image walking all of it, 102 us now.  The
+// labels are read and ranked twice, so a batch that gives every SIMD a wave of
+// its own (1024 images) keeps the walk, k_sample_weighted (images of 640 x 480, walk
+// -> segments: 250 images 2.75 -> 0.70 ms, 500 2.81 -> 1.23, 1000 2.82 -> 2.71; 5000
+// 4.3 -> 8.8).
 //
-// The streams are generated for draws [w0, w0 + win) of every image at a time
-// (win * n_images words of workspace); larger images take several windows.
+// The streams are generated for draws [w0, w0 + win) of every image of a group
+// at a time (win * n_images words of workspace, which bounds the group); an image
+// larger than the workspace takes several windows.
 constexpr uint32_t MT_LAG = MT_N - MT_M;     // 227
 constexpr uint32_t MT_STEP = 2 * MT_LAG;     // words a step computes from the last 624
 
@@ -550,7 +555,8 @@ __device__ __forceinline__ void each_class(uint32_t l, const Fn &f)
 }
 
 // Blocks [0, n_images): the stream of image blockIdx.x, draws [w0, w0 + win)
-// into draws[image * win ..]; `state` carries the last 624 words to the next
+// into draws[image * win ..] (images and seg0 are a group's, segments [seg_base,
+// seg_end)); `state` carries the last 624 words to the next
 // window.  The other blocks (w0 = 0 only): class counts of four segments.
 // Labels above n_classes set *bad and count as unlabelled.
 //
@@ -563,7 +569,8 @@ __device__ __forceinline__ void each_class(uint32_t l, const Fn &f)
 // one 56 us.
 __global__ __launch_bounds__(256) void k_weighted_count(const uint8_t *__restrict__ labels,
                                                         const SampleJob *__restrict__ jobs, uint32_t n_images,
-                                                        const uint32_t *__restrict__ seg0, uint32_t n_segs,
+                                                        const uint32_t *__restrict__ seg0, uint32_t seg_base,
+                                                        uint32_t seg_end,
                                                         uint32_t seg_len, const uint32_t *__restrict__ crc,
                                                         uint32_t seed, uint32_t n_classes, uint32_t w0, uint32_t win,
                                                         uint32_t *__restrict__ draws, uint32_t *__restrict__ state,
@@ -602,8 +609,8 @@ __global__ __launch_bounds__(256) void k_weighted_count(const uint8_t *__restric
     return;
   }
   const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t seg = (blockIdx.x - n_images) * 4u + wave;
-  if (seg >= n_segs) return;
+  const uint32_t seg = seg_base + (blockIdx.x - n_images) * 4u + wave;
+  if (seg >= seg_end) return;
   uint32_t *cnt = sh + 256u * wave;
   for (uint32_t c = lane; c < 256u; c += 64u) cnt[c] = 0;
   wave_sync();
@@ -636,14 +643,14 @@ __global__ __launch_bounds__(256) void k_weighted_count(const uint8_t *__restric
 // segment in, class ordinal at its start out; seg_draw[seg] = (draw index at its
 // start, number of draws); class_count[image][c] the totals.
 __global__ __launch_bounds__(1024) void k_weighted_scan(const uint32_t *__restrict__ seg0, uint32_t n_images,
-                                                        uint32_t n_segs, uint32_t n_classes,
+                                                        uint32_t seg_end, uint32_t n_classes,
                                                         const uint32_t *__restrict__ B, uint32_t *counts,
                                                         uint2 *__restrict__ seg_draw,
                                                         uint32_t *__restrict__ class_count)
 {
   __shared__ uint32_t sB[256], tot[256], ws[16];
   const uint32_t im = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t s0 = seg0[im], ns = (im + 1u < n_images ? seg0[im + 1u] : n_segs) - s0;
+  const uint32_t s0 = seg0[im], ns = (im + 1u < n_images ? seg0[im + 1u] : seg_end) - s0;
   uint32_t *ct = counts + (size_t)s0 * n_classes;
   if (tid < n_classes) sB[tid] = B[tid];
   for (uint32_t c = wave; c < n_classes; c += 16u) {
@@ -704,8 +711,8 @@ __global__ __launch_bounds__(1024) void k_weighted_scan(const uint32_t *__restri
 // step).
 __global__ __launch_bounds__(256) void k_weighted_draw(const uint8_t *__restrict__ labels,
                                                        const SampleJob *__restrict__ jobs, uint32_t n_images,
-                                                       const uint32_t *__restrict__ seg0, uint32_t n_segs,
-                                                       uint32_t seg_len, uint32_t n_classes,
+                                                       const uint32_t *__restrict__ seg0, uint32_t seg_base,
+                                                       uint32_t seg_end, uint32_t seg_len, uint32_t n_classes,
                                                        const uint32_t *__restrict__ B,
                                                        const uint32_t *__restrict__ boff, uint32_t w0, uint32_t win,
                                                        const uint32_t *__restrict__ draws,
@@ -717,8 +724,8 @@ __global__ __launch_bounds__(256) void k_weighted_draw(const uint8_t *__restrict
   sB[tid] = tid < n_classes ? B[tid] : 0u;
   sO[tid] = tid < n_classes ? boff[tid] : 0u;
   __syncthreads();  // the only block-wide barrier: from here on the waves are independent
-  const uint32_t seg = blockIdx.x * 4u + wave;
-  if (seg >= n_segs) return;
+  const uint32_t seg = seg_base + blockIdx.x * 4u + wave;
+  if (seg >= seg_end) return;
   const uint2 sd = seg_draw[seg];
   if (w0 != 0u && (sd.x + sd.y <= w0 || sd.x - w0 >= win)) return;
   uint32_t *cnt = cnt_all[wave];
@@ -766,6 +773,142 @@ __global__ __launch_bounds__(256) void k_weighted_draw(const uint8_t *__restrict
       }
     }
   }
+}
+
+// One twist of a state by one wave (no tempering: outputs are tempered when
+// drawn).  Same three dependent ranges as mt_twist.
+__device__ inline void mt_twist_wave(uint32_t *mt, uint32_t lane)
+{
+  uint32_t a1[4], a2[4], a3[3];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const uint32_t i = lane + 64u * r;
+    a1[r] = a2[r] = 0;
+    if (i < 227) {
+      a1[r] = mt[i + MT_M] ^ mt_mix(mt[i], mt[i + 1]);
+      a2[r] = mt_mix(mt[227 + i], mt[228 + i]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    const uint32_t i = lane + 64u * r;
+    a3[r] = (i < 169) ? mt_mix(mt[454 + i], mt[455 + i]) : 0u;
+  }
+  const uint32_t last_old = mt[623];
+  wave_sync();
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if (lane + 64u * r < 227) mt[lane + 64u * r] = a1[r];
+  wave_sync();
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if (lane + 64u * r < 227) mt[227 + lane + 64u * r] = mt[lane + 64u * r] ^ a2[r];
+  wave_sync();
+#pragma unroll
+  for (int r = 0; r < 3; r++)
+    if (lane + 64u * r < 169) mt[454 + lane + 64u * r] = mt[227 + lane + 64u * r] ^ a3[r];
+  if (lane == 0) mt[623] = mt[396] ^ mt_mix(last_old, mt[0]);
+  wave_sync();
+}
+
+// Batches of WEIGHTED_BATCH images and more: one wave per image (four images per
+// block), 64 pixels per step in scan
+// order (lane l: pixel t0 + 64 s + l); the label bytes of the next 16 steps
+// are prefetched from global memory.  A pixel's class ordinal k is the class
+// count so far (LDS) plus its rank among the wave's lanes of that class (one
+// ballot per distinct class, the class read with readlane); it draws iff
+// k >= B_c, and its draw index is the wave prefix of those flags, so the MT
+// stream is consumed in the serial loop's order.  bucket: zero-initialised
+// slots [image][sum B] (class c at boff[c]) filled with atomicMax (the last
+// writer in scan order has the largest pixel index).  Labels above
+// n_classes set *bad.
+//
+// Bound by VALU issue: about 85 VALU + 43 SALU instructions per 64-pixel step
+// (class ranks, the draw's FP64 product and roundf, tempering, a twist per
+// 624 draws).  Keeping the slots in LDS instead of global atomics cut the
+// occupancy and ran slower.
+__global__ __launch_bounds__(256) void k_sample_weighted(const uint8_t *__restrict__ labels,
+                                                         const SampleJob *__restrict__ jobs, uint32_t n_images,
+                                                         const uint32_t *__restrict__ crc, uint32_t seed,
+                                                         uint32_t n_classes, const uint32_t *__restrict__ B,
+                                                         const uint32_t *__restrict__ boff, uint32_t *bucket,
+                                                         uint32_t *class_count, uint32_t *bad)
+{
+  __shared__ uint32_t sB[256], sO[256];
+  __shared__ uint32_t mt_all[4][MT_N], cnt_all[4][256];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  sB[threadIdx.x] = threadIdx.x < n_classes ? B[threadIdx.x] : 0u;
+  sO[threadIdx.x] = threadIdx.x < n_classes ? boff[threadIdx.x] : 0u;
+  __syncthreads();  // the only block-wide barrier: from here on the waves are independent
+  const uint32_t im = blockIdx.x * 4u + wave;
+  if (im >= n_images) return;
+  uint32_t *mt = mt_all[wave], *cnt = cnt_all[wave];
+  for (uint32_t c = lane; c < 256u; c += 64u) cnt[c] = 0;
+  const SampleJob J = jobs[im];
+  const uint8_t *lab = labels + J.lab_off;
+  uint32_t *bk = bucket + J.out_base;
+  if (lane == 0) mt_seed(mt, crc[im] ^ seed);
+  wave_sync();
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
+  uint32_t D = 0, gen = 0;  // draws consumed; outputs generated ([gen - 624, gen) are in mt)
+  uint32_t nx[16];
+#pragma unroll
+  for (int s = 0; s < 16; s++) nx[s] = (64u * s + lane < J.n_px) ? lab[64u * s + lane] : 0u;
+  for (uint32_t t0 = 0; t0 < J.n_px; t0 += 1024u) {
+    uint32_t cur[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      cur[s] = nx[s];
+      const uint32_t q = t0 + 1024u + 64u * s + lane;
+      nx[s] = (q < J.n_px) ? lab[q] : 0u;  // prefetch the next tile
+    }
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      if (t0 + 64u * s >= J.n_px) break;
+      const uint32_t p = t0 + 64u * s + lane;
+      uint32_t l = cur[s];
+      if (l > n_classes) { atomicOr(bad, 1u); l = 0; }
+      const bool valid = l != 0u;
+      const uint32_t c = l - 1u;
+      uint32_t k = 0, Bc = 0, Oc = 0;
+      uint64_t pending = __ballot(valid);
+      while (pending) {
+        const uint32_t lead = (uint32_t)__builtin_ctzll(pending);
+        const uint32_t cl = __builtin_amdgcn_readlane(c, lead);
+        const uint64_t mm = __ballot(valid && c == cl);
+        const uint32_t before = cnt[cl], bcl = sB[cl], ocl = sO[cl];
+        if (valid && c == cl) {
+          k = before + (uint32_t)__popcll(mm & lt);
+          Bc = bcl;
+          Oc = ocl;
+        }
+        if (lane == lead) cnt[cl] = before + (uint32_t)__popcll(mm);
+        pending &= ~mm;
+      }
+      const bool draw = valid && k >= Bc;
+      const uint64_t dm = __ballot(draw);
+      const uint32_t d = D + (uint32_t)__popcll(dm & lt);
+      D += (uint32_t)__popcll(dm);
+      uint32_t x = 0;
+      if (D > gen) {  // wave-uniform: this step crosses into the next twist
+        if (draw && d < gen) x = mt[d + MT_N - gen];
+        mt_twist_wave(mt, lane);
+        gen += MT_N;
+        if (draw && d + MT_N >= gen) x = mt[d + MT_N - gen];
+      } else if (draw) {
+        x = mt[d + MT_N - gen];
+      }
+      if (draw) {
+        const double u = (double)mt_temper(x) * 2.3283064365386962890625e-10;  // x / 2^32
+        const uint32_t j = (uint32_t)roundf((float)(u * (double)k));
+        if (j < Bc) atomicMax(&bk[Oc + j], p);
+      } else if (valid) {
+        atomicMax(&bk[Oc + k], p);
+      }
+    }
+  }
+  wave_sync();
+  for (uint32_t c = lane; c < n_classes; c += 64u) class_count[(uint64_t)im * n_classes + c] = cnt[c];
 }
 
 // filled slots of every class -> contiguous unsorted samples; segment end

@@ -41,7 +41,8 @@ struct IngestDev {
 };
 
 constexpr CrcTables HT = make_crc_tables();
-constexpr uint64_t WEIGHTED_WORDS = 16ull << 20;   // stream words of the class-weighted sampler at a time (64 MiB)
+constexpr uint64_t WEIGHTED_WORDS = 64ull << 20;   // stream words of the class-weighted sampler at a time (256 MiB)
+constexpr uint32_t WEIGHTED_BATCH = 1024;           // images from which every one is walked by a wave of its own
 using Lock = std::lock_guard<std::recursive_mutex>;
 
 IngestDev &ctx(int device)
@@ -312,28 +313,39 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for((uint64_t)n * cap, 256)), dim3(256), 0, st,
                        X.bucket.as<uint32_t>(), (uint64_t)n * cap, 0u);
     tm.mark(2);
-    // the streams' windows share WEIGHTED_WORDS words
-    const uint64_t share = std::min<uint64_t>(std::max<uint64_t>(max_px, 1), std::max<uint64_t>(WEIGHTED_WORDS / n, 1));
-    const uint32_t win = (uint32_t)((share + MT_STEP - 1) / MT_STEP * MT_STEP);
-    X.draws.ensure((size_t)n * win * 4u);
-    if (max_px > win) X.mt_state.ensure((size_t)n * MT_N * 4u);
-    X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
-    X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
-    for (uint64_t w0 = 0; w0 == 0 || w0 < max_px; w0 += win) {
-      const uint32_t count_blocks = w0 == 0 ? (n_segs + 3) / 4 : 0u;
-      hipLaunchKernelGGL(k_weighted_count, dim3(n + count_blocks), dim3(256), 0, st, d_labels, d_jobs, n,
-                         d_first, n_segs, seg_len, crc, s.seed, s.n_classes, (uint32_t)w0, win,
-                         X.draws.as<uint32_t>(), X.mt_state.as<uint32_t>(), X.seg_counts.as<uint32_t>(),
-                         d_bad);
-      if (w0 == 0)
-        hipLaunchKernelGGL(k_weighted_scan, dim3(n), dim3(1024), 0, st, d_first, n, n_segs,
-                           s.n_classes, d_B, X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
-                           X.class_count.as<uint32_t>());
-      if (n_segs)
-        hipLaunchKernelGGL(k_weighted_draw, dim3((n_segs + 3) / 4), dim3(256), 0, st, d_labels,
-                           d_jobs, n, d_first, n_segs, seg_len, s.n_classes,
-                           d_B, d_boff, (uint32_t)w0, win, X.draws.as<uint32_t>(),
-                           X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(), X.bucket.as<uint32_t>());
+    if (n >= WEIGHTED_BATCH) {
+      hipLaunchKernelGGL(k_sample_weighted, dim3((n + 3) / 4), dim3(256), 0, st, d_labels, d_jobs, n, crc, s.seed,
+                         s.n_classes, d_B, d_boff, X.bucket.as<uint32_t>(), X.class_count.as<uint32_t>(), d_bad);
+    } else {
+      // groups of about equal size whose streams fit WEIGHTED_WORDS (an image
+      // that does not fit alone: windows of it)
+      const uint64_t px = std::max<uint64_t>(max_px, 1);
+      const uint32_t fit = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, WEIGHTED_WORDS / px));
+      const uint32_t n_groups = (n + fit - 1) / fit, per = (n + n_groups - 1) / n_groups;
+      const uint32_t win = (uint32_t)((std::min(px, WEIGHTED_WORDS) + MT_STEP - 1) / MT_STEP * MT_STEP);
+      X.draws.ensure((size_t)per * win * 4u);
+      if (max_px > win) X.mt_state.ensure((size_t)per * MT_N * 4u);
+      X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
+      X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
+      for (uint32_t g = 0; g < n; g += per) {
+        const uint32_t gn = std::min(per, n - g);
+        const uint32_t sb = tile0[g], se = g + gn < n ? tile0[g + gn] : n_segs, seg_blocks = (se - sb + 3) / 4;
+        for (uint64_t w0 = 0; w0 == 0 || w0 < max_px; w0 += win) {
+          hipLaunchKernelGGL(k_weighted_count, dim3(gn + (w0 == 0 ? seg_blocks : 0u)), dim3(256), 0, st, d_labels,
+                             d_jobs + g, gn, d_first + g, sb, se, seg_len, crc + g, s.seed, s.n_classes, (uint32_t)w0,
+                             win, X.draws.as<uint32_t>(), X.mt_state.as<uint32_t>(), X.seg_counts.as<uint32_t>(),
+                             d_bad);
+          if (w0 == 0)
+            hipLaunchKernelGGL(k_weighted_scan, dim3(gn), dim3(1024), 0, st, d_first + g, gn, se, s.n_classes, d_B,
+                               X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
+                               X.class_count.as<uint32_t>() + (size_t)g * s.n_classes);
+          if (seg_blocks)
+            hipLaunchKernelGGL(k_weighted_draw, dim3(seg_blocks), dim3(256), 0, st, d_labels, d_jobs + g, gn,
+                               d_first + g, sb, se, seg_len, s.n_classes, d_B, d_boff, (uint32_t)w0, win,
+                               X.draws.as<uint32_t>(), X.seg_counts.as<uint32_t>(), X.seg_draw.as<uint2>(),
+                               X.bucket.as<uint32_t>());
+        }
+      }
     }
     hipLaunchKernelGGL(k_compact_buckets, dim3(n), dim3(256), 0, st, d_jobs, s.n_classes,
                        d_B, d_boff, X.class_count.as<uint32_t>(),

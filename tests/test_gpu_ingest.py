@@ -125,12 +125,13 @@ def test_weighted_sampler_matches_oracle(gpu, n_classes, weights, n_samples):
 
 @pytest.mark.parametrize("shapes,n_samples", [
     ([(32, 32), (1, 1025), (1, 1023), (48, 64), (1, 1)], 40),   # whole segments, one pixel more and less
-    ([(4100, 4100), (37, 61), (227, 4)], 500),                         # several windows of the draw streams
+    ([(37, 61), (8200, 8200), (227, 4)], 500),                  # groups of images, windows of a draw stream
+    ([(3, 17), (9, 8), (1, 1)] * 342, 10),                      # 1026 images: a wave walks each
 ])
-def test_weighted_sampler_segments_and_windows(gpu, shapes, n_samples):
+def test_weighted_sampler_segments_groups_and_windows(gpu, shapes, n_samples):
     rng = np.random.default_rng(n_samples)
-    labs = [rng.integers(0, 6, s).astype(np.uint8) for s in shapes]
-    datas = [rng.integers(0, 65536, s, dtype=np.uint16) for s in shapes]
+    labs = [rng.integers(0, 6, s, dtype=np.uint8) for s in shapes]
+    datas = [rng.integers(0, 256, s, dtype=np.uint8) for s in shapes]
     smp = ds.ClassWeightedImageSampler(n_samples, 5, None, seed=9)
     got = smp.sample_batch(datas, labs)
     want, _ = oi.sample_images(1, datas, labs, n_samples, 5, None, seed=9)
