@@ -876,11 +876,11 @@ struct Trainer final : TrainerBase {
     std::vector<uint8_t> smode(ns, 0);
     std::vector<uint32_t> zero, group_start;
     std::vector<float> group_pos;
-    // level-batched launches with round-robin XCD placement: the (node,
-    // chunk) groups are collected first and their items written straight
-    // into the interleaved order xcd_order() builds (group g on XCD g % X at
-    // lane row g / X, its ftiles items in tile order, NULL_SLOT padding), so
-    // the host does not build, copy and re-interleave the item list per level
+    // level-batched launches with balanced XCD placement: the (node, chunk)
+    // groups are collected first and their items written straight into the
+    // interleaved order of the launch (below; ftiles items a group in tile
+    // order, NULL_SLOT padding), so the host does not build, copy and
+    // re-interleave the item list per level
     const bool direct = mode == PD_MODE_LEVEL_BATCHED && n_xcc > 1 && !xcd_by_position;
     std::vector<uint4> groups;   // (slot, begin, count) of each group, in order
     hslots.clear();
