@@ -517,8 +517,9 @@ __global__ __launch_bounds__(256) void k_sample_uniform(const SampleJob *__restr
 // 4.3 -> 8.8).
 //
 // The streams are generated for draws [w0, w0 + win) of every image of a group
-// at a time (win * n_images words of workspace, which bounds the group); an image
-// larger than the workspace takes several windows.
+// at a time (win * n_images words of scratch, which bounds the group); an image
+// larger than the scratch takes several windows, and a segment's draws may lie in
+// two of them and more.
 constexpr uint32_t MT_LAG = MT_N - MT_M;     // 227
 constexpr uint32_t MT_STEP = 2 * MT_LAG;     // words a step computes from the last 624
 
@@ -727,7 +728,9 @@ __global__ __launch_bounds__(256) void k_weighted_draw(const uint8_t *__restrict
   const uint32_t seg = seg_base + blockIdx.x * 4u + wave;
   if (seg >= seg_end) return;
   const uint2 sd = seg_draw[seg];
-  if (w0 != 0u && (sd.x + sd.y <= w0 || sd.x - w0 >= win)) return;
+  // no draw of the segment is in the window: it ends before it or begins behind it
+  // (one that begins before it and ends inside draws its last ones here)
+  if (w0 != 0u && (sd.x + sd.y <= w0 || (sd.x >= w0 && sd.x - w0 >= win))) return;
   uint32_t *cnt = cnt_all[wave];
   for (uint32_t c = lane; c < n_classes; c += 64u) cnt[c] = counts[(size_t)seg * n_classes + c];
   const uint32_t im = find_owner(seg0, n_images, seg);

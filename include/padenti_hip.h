@@ -447,6 +447,16 @@ PD_API int pd_sample_images_dev(int device, const pd_sampler *s, uint32_t n_imag
                                 const uint8_t *d_labels, uint64_t labels_size, const uint64_t *label_offsets,
                                 const uint32_t *widths, const uint32_t *heights, uint32_t *d_samples,
                                 uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats);
+/* The same with at most scratch_bytes (rounded up to one step of a stream, 1816
+ * bytes an image; pd_sample_images_dev: 256 MiB) of device memory for the
+ * random streams of the class-weighted sampler.  Longer streams are generated
+ * in parts, larger batches in groups of images; the samples do not depend on it. */
+PD_API int pd_sample_images_dev_scratch(int device, const pd_sampler *s, uint32_t n_images, const void *d_data,
+                                        uint64_t data_size, const uint64_t *data_offsets, const uint64_t *data_bytes,
+                                        const uint8_t *d_labels, uint64_t labels_size, const uint64_t *label_offsets,
+                                        const uint32_t *widths, const uint32_t *heights, uint32_t *d_samples,
+                                        uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats,
+                                        uint64_t scratch_bytes);
 /* crc32 (zlib's) of n byte ranges of device memory d_data (data_size bytes;
  * every range is checked against it); kernel_ms optional */
 PD_API int pd_crc32_images_dev(int device, uint32_t n, const void *d_data, uint64_t data_size,

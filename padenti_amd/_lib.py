@@ -203,6 +203,8 @@ def lib():
         "pd_sample_images": (I32, [I32, C.POINTER(Sampler), U32, VP, VP, VP, VP, VP, VP, VP, VP, VP, VP]),
         "pd_sample_images_dev": (I32, [I32, C.POINTER(Sampler), U32, VP, U64, VP, VP, VP, U64, VP, VP, VP, VP, VP,
                                        VP, C.POINTER(IngestStats)]),
+        "pd_sample_images_dev_scratch": (I32, [I32, C.POINTER(Sampler), U32, VP, U64, VP, VP, VP, U64, VP, VP, VP, VP,
+                                               VP, VP, C.POINTER(IngestStats), U64]),
         "pd_crc32_images_dev": (I32, [I32, U32, VP, U64, VP, VP, VP, C.POINTER(C.c_float)]),
         "pd_rgb_to_labels": (I32, [I32, U64, U32, VP, VP, U32, VP]),
         "pd_rgb_to_labels_dev": (I32, [I32, U64, U32, VP, VP, U32, VP, C.POINTER(C.c_float)]),

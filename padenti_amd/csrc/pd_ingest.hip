@@ -41,7 +41,7 @@ struct IngestDev {
 };
 
 constexpr CrcTables HT = make_crc_tables();
-constexpr uint64_t WEIGHTED_WORDS = 64ull << 20;   // stream words of the class-weighted sampler at a time (256 MiB)
+constexpr uint64_t WEIGHTED_SCRATCH = 256ull << 20;   // random streams of the class-weighted sampler at a time
 constexpr uint32_t WEIGHTED_BATCH = 1024;           // images from which every one is walked by a wave of its own
 using Lock = std::lock_guard<std::recursive_mutex>;
 
@@ -210,7 +210,7 @@ struct Timer {
 void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data, uint64_t data_size,
                 const uint64_t *data_off, const uint64_t *data_bytes, const uint8_t *d_labels, uint64_t labels_size,
                 const uint64_t *lab_off, const uint32_t *widths, const uint32_t *heights, uint32_t *d_samples,
-                uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats)
+                uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats, uint64_t scratch_bytes = WEIGHTED_SCRATCH)
 {
   require(n >= 1, "n_images must be >= 1");
   require(d_data && data_off && data_bytes && d_labels && lab_off && widths && heights && d_samples && d_n_out,
@@ -317,12 +317,12 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
       hipLaunchKernelGGL(k_sample_weighted, dim3((n + 3) / 4), dim3(256), 0, st, d_labels, d_jobs, n, crc, s.seed,
                          s.n_classes, d_B, d_boff, X.bucket.as<uint32_t>(), X.class_count.as<uint32_t>(), d_bad);
     } else {
-      // groups of about equal size whose streams fit WEIGHTED_WORDS (an image
+      // groups of about equal size whose streams fit the scratch (an image
       // that does not fit alone: windows of it)
-      const uint64_t px = std::max<uint64_t>(max_px, 1);
-      const uint32_t fit = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, WEIGHTED_WORDS / px));
+      const uint64_t px = std::max<uint64_t>(max_px, 1), words = std::max<uint64_t>(scratch_bytes / 4u, 1);
+      const uint32_t fit = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, words / px));
       const uint32_t n_groups = (n + fit - 1) / fit, per = (n + n_groups - 1) / n_groups;
-      const uint32_t win = (uint32_t)((std::min(px, WEIGHTED_WORDS) + MT_STEP - 1) / MT_STEP * MT_STEP);
+      const uint32_t win = (uint32_t)((std::min(px, words) + MT_STEP - 1) / MT_STEP * MT_STEP);
       X.draws.ensure((size_t)per * win * 4u);
       if (max_px > win) X.mt_state.ensure((size_t)per * MT_N * 4u);
       X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
@@ -435,6 +435,19 @@ int pd_sample_images_dev(int device, const pd_sampler *s, uint32_t n_images, con
     require(s != nullptr, "null sampler");
     sample_dev(device, *s, n_images, d_data, data_size, data_offsets, data_bytes, d_labels, labels_size,
                label_offsets, widths, heights, d_samples, d_n_out, d_crc, stats);
+  });
+}
+
+int pd_sample_images_dev_scratch(int device, const pd_sampler *s, uint32_t n_images, const void *d_data,
+                                 uint64_t data_size, const uint64_t *data_offsets, const uint64_t *data_bytes,
+                                 const uint8_t *d_labels, uint64_t labels_size, const uint64_t *label_offsets,
+                                 const uint32_t *widths, const uint32_t *heights, uint32_t *d_samples,
+                                 uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats, uint64_t scratch_bytes)
+{
+  return guarded([&] {
+    require(s != nullptr, "null sampler");
+    sample_dev(device, *s, n_images, d_data, data_size, data_offsets, data_bytes, d_labels, labels_size,
+               label_offsets, widths, heights, d_samples, d_n_out, d_crc, stats, scratch_bytes);
   });
 }
 

@@ -152,11 +152,12 @@ class _Sampler:
         return (res, crcs) if crc else res
 
     def sample_dev(self, n, d_data, data_size, data_off, data_bytes, d_labels, labels_size, lab_off, widths, heights,
-                   d_samples, d_n_out, d_crc=None):
+                   d_samples, d_n_out, d_crc=None, scratch_bytes=None):
         """Device-resident form (pd_sample_images_dev): d_* are device
         pointers, data_size / labels_size the bytes of those buffers, the
         rest host arrays (uint64 offsets and byte counts, uint32 sizes).
-        Returns the stage timings."""
+        scratch_bytes bounds the class-weighted sampler's random streams
+        (pd_sample_images_dev_scratch).  Returns the stage timings."""
         st = IngestStats()
         desc = self._desc()
         arrs = [np.ascontiguousarray(a, dtype=t) for a, t in ((data_off, np.uint64), (data_bytes, np.uint64),
@@ -165,9 +166,12 @@ class _Sampler:
         for a in arrs:
             if a.size != n:
                 raise ValueError("one offset / size per image")
-        check(lib().pd_sample_images_dev(self.device, C.byref(desc), n, d_data, int(data_size), ptr(arrs[0]),
-                                         ptr(arrs[1]), d_labels, int(labels_size), ptr(arrs[2]), ptr(arrs[3]),
-                                         ptr(arrs[4]), d_samples, d_n_out, d_crc, C.byref(st)))
+        args = (self.device, C.byref(desc), n, d_data, int(data_size), ptr(arrs[0]), ptr(arrs[1]), d_labels,
+                int(labels_size), ptr(arrs[2]), ptr(arrs[3]), ptr(arrs[4]), d_samples, d_n_out, d_crc, C.byref(st))
+        if scratch_bytes is None:
+            check(lib().pd_sample_images_dev(*args))
+        else:
+            check(lib().pd_sample_images_dev_scratch(*args, int(scratch_bytes)))
         self.last_stats = {f: getattr(st, f) for f, _ in IngestStats._fields_}
         return self.last_stats
 

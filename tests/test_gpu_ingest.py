@@ -125,7 +125,7 @@ def test_weighted_sampler_matches_oracle(gpu, n_classes, weights, n_samples):
 
 @pytest.mark.parametrize("shapes,n_samples", [
     ([(32, 32), (1, 1025), (1, 1023), (48, 64), (1, 1)], 40),   # whole segments, one pixel more and less
-    ([(37, 61), (8200, 8200), (227, 4)], 500),                  # groups of images, windows of a draw stream
+    ([(37, 61), (8200, 8200), (227, 4)], 500),                  # one image more than the scratch: groups of one
     ([(3, 17), (9, 8), (1, 1)] * 342, 10),                      # 1026 images: a wave walks each
 ])
 def test_weighted_sampler_segments_groups_and_windows(gpu, shapes, n_samples):
@@ -135,6 +135,47 @@ def test_weighted_sampler_segments_groups_and_windows(gpu, shapes, n_samples):
     smp = ds.ClassWeightedImageSampler(n_samples, 5, None, seed=9)
     got = smp.sample_batch(datas, labs)
     want, _ = oi.sample_images(1, datas, labs, n_samples, 5, None, seed=9)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert np.array_equal(g, w), i
+
+
+def _sample_dev(smp, datas, labs, scratch_bytes):
+    """sample_dev of a host batch with the given scratch, one array per image."""
+    n, off, loff = len(labs), [], []
+    buf, lbuf = b"", b""
+    for d, l in zip(datas, labs):
+        off.append(len(buf))
+        buf += d.tobytes()
+        loff.append(len(lbuf))
+        lbuf += l.tobytes()
+        lbuf += bytes(-len(lbuf) % 16)
+    dd, dl = DevArray(len(buf)), DevArray(len(lbuf))
+    dd.put(np.frombuffer(buf, np.uint8))
+    dl.put(np.frombuffer(lbuf, np.uint8))
+    cap = smp.capacity()
+    ds_, dn = DevArray(4 * n * cap), DevArray(4 * n)
+    smp.sample_dev(n, dd.p, len(buf), off, [d.nbytes for d in datas], dl.p, len(lbuf), loff,
+                   [l.shape[1] for l in labs], [l.shape[0] for l in labs], ds_.p, dn.p, scratch_bytes=scratch_bytes)
+    out, n_out = ds_.get(n * cap, np.uint32), dn.get(n, np.uint32)
+    for a in (dd, dl, ds_, dn):
+        a.free()
+    return [out[i * cap:i * cap + n_out[i]] for i in range(n)]
+
+
+# words of the random streams at a time: one step of a stream (a segment of 1024
+# pixels meets several windows), windows that end inside segments, whole images
+# in groups of one and two, everything at once
+@pytest.mark.parametrize("words", [1, 3 * 454, 5000, 30000, 61000, 1 << 20])
+@pytest.mark.parametrize("n_samples", [900, 24000])   # few slots replaced often; as many slots as pixels
+def test_weighted_sampler_scratch_bounds(gpu, words, n_samples):
+    rng = np.random.default_rng(words + n_samples)
+    shapes = [(64, 64), (37, 61), (1, 455), (200, 150), (1, 1), (31, 33)]
+    labs = [rng.integers(1, 4, s, dtype=np.uint8) for s in shapes]   # every pixel labelled
+    labs[5][rng.random(shapes[5]) < 0.5] = 0
+    datas = [rng.integers(0, 256, s, dtype=np.uint8) for s in shapes]
+    smp = ds.ClassWeightedImageSampler(n_samples, 3, None, seed=21)
+    got = _sample_dev(smp, datas, labs, 4 * words)
+    want, _ = oi.sample_images(1, datas, labs, n_samples, 3, None, seed=21)
     for i, (g, w) in enumerate(zip(got, want)):
         assert np.array_equal(g, w), i
 
