@@ -213,26 +213,28 @@ __global__ __launch_bounds__(256) void k_crc32(const CrcJob *__restrict__ jobs, 
 // with q the length of the last block from a0 (at most 4096).  One wave per
 // image: lane k < 16 holds the factor of bit k of q, lane 16 + k that of bit k of
 // len (below 2^44), multiplied in a tree (one thread walking the bits: 11.5 us
-// for 150 images, now 8.2).
+// for 150 images, now 8.2).  The grid is bounded; its waves go on by its size.
 __global__ __launch_bounds__(256) void k_crc_final(const CrcJob *__restrict__ jobs, uint32_t n_images,
                                                    const uint32_t *__restrict__ acc_a,
                                                    const uint32_t *__restrict__ acc_b, uint32_t *crc_out)
 {
-  const uint32_t lane = threadIdx.x & 63u, i = blockIdx.x * 4u + (threadIdx.x >> 6);
-  if (i >= n_images) return;
-  const CrcJob J = jobs[i];
-  const uint64_t q = J.n_blocks ? J.end - J.a0 - 4096ull * (J.n_blocks - 1u) : 0ull;
-  const uint64_t n = lane < 16u ? q : J.end - J.start;
-  const uint32_t bit = lane < 16u ? lane : lane - 16u;
-  uint32_t f = (n >> bit) & 1u ? c_crc.x2k[bit + 3u] : CRC_ONE;
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint64_t i = blockIdx.x * 4u + (threadIdx.x >> 6); i < n_images; i += gridDim.x * 4u) {
+    const CrcJob J = jobs[i];
+    const uint64_t q = J.n_blocks ? J.end - J.a0 - 4096ull * (J.n_blocks - 1u) : 0ull;
+    const uint64_t n = lane < 16u ? q : J.end - J.start;
+    const uint32_t bit = lane < 16u ? lane : lane - 16u;
+    uint32_t f = (n >> bit) & 1u ? c_crc.x2k[bit + 3u] : CRC_ONE;
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) f = gf2_mul(f, __shfl_xor(f, o));
-  const uint32_t a = gf2_mul(f, __shfl_xor(f, 16));   // lanes 32..: bits 16..47 of len
-  const uint32_t l = gf2_mul(__shfl(a, 32), __shfl(f, 16));
-  const uint32_t fq = __shfl(f, 0);
-  if (lane != 0u) return;
-  const uint32_t pure = J.n_blocks ? gf2_mul(acc_a[i], fq) ^ acc_b[i] : 0u;
-  crc_out[i] = pure ^ gf2_mul(0xFFFFFFFFu, l) ^ 0xFFFFFFFFu;
+    for (int o = 1; o < 16; o <<= 1) f = gf2_mul(f, __shfl_xor(f, o));
+    const uint32_t a = gf2_mul(f, __shfl_xor(f, 16));   // lanes 32..: bits 16..47 of len
+    const uint32_t l = gf2_mul(__shfl(a, 32), __shfl(f, 16));
+    const uint32_t fq = __shfl(f, 0);
+    if (lane == 0u) {
+      const uint32_t pure = J.n_blocks ? gf2_mul(acc_a[i], fq) ^ acc_b[i] : 0u;
+      crc_out[i] = pure ^ gf2_mul(0xFFFFFFFFu, l) ^ 0xFFFFFFFFu;
+    }
+  }
 }
 
 // ---- MT19937 (Matsumoto & Nishimura 1998), 256 threads share one state ----

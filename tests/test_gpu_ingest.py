@@ -60,6 +60,24 @@ def test_crc32_ragged_ranges(gpu):
     crc.free()
 
 
+def test_crc32_more_images_than_one_grid_holds(gpu):
+    rng = np.random.default_rng(2)
+    buf = rng.integers(0, 256, 1 << 16, dtype=np.uint8)
+    n = 4 * 65535 * 16 + 65   # a wave per image, four a block: past a grid of 65535 x 16 blocks
+    off = rng.integers(0, buf.size - 300, 4096).astype(np.uint64)
+    size = rng.integers(0, 300, 4096).astype(np.uint64)
+    want = np.array([zlib.crc32(buf[int(o):int(o + k)].tobytes()) for o, k in zip(off, size)], np.uint32)
+    reps = -(-n // 4096)
+    off, size, want = (np.tile(a, reps)[:n] for a in (off, size, want))
+    d, crc = DevArray(buf.size), DevArray(4 * n)
+    d.put(buf)
+    ms = C.c_float()
+    check(lib().pd_crc32_images_dev(0, n, d.p, buf.size, ptr(off), ptr(size), crc.p, C.byref(ms)))
+    assert np.array_equal(crc.get(n, np.uint32), want)
+    d.free()
+    crc.free()
+
+
 def _batch(seed, n=24):
     """Ragged images: sizes from 1x1 to 640x480, label densities from none to all."""
     rng = np.random.default_rng(seed)
