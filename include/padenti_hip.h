@@ -448,9 +448,11 @@ PD_API int pd_sample_images_dev(int device, const pd_sampler *s, uint32_t n_imag
                                 const uint32_t *widths, const uint32_t *heights, uint32_t *d_samples,
                                 uint32_t *d_n_out, uint32_t *d_crc, pd_ingest_stats *stats);
 /* The same with at most scratch_bytes (rounded up to one step of a stream, 1816
- * bytes an image; pd_sample_images_dev: 256 MiB) of device memory for the
- * random streams of the class-weighted sampler.  Longer streams are generated
- * in parts, larger batches in groups of images; the samples do not depend on it. */
+ * bytes; pd_sample_images_dev: 256 MiB) of device memory for the random streams
+ * of the class-weighted sampler.  Longer streams are generated in parts, larger
+ * batches in groups of images; without any (0, or where the allocation fails)
+ * every image is walked by one wave.  The samples do not depend on it.  What is
+ * held beyond the bound from earlier calls on the device is freed. */
 PD_API int pd_sample_images_dev_scratch(int device, const pd_sampler *s, uint32_t n_images, const void *d_data,
                                         uint64_t data_size, const uint64_t *data_offsets, const uint64_t *data_bytes,
                                         const uint8_t *d_labels, uint64_t labels_size, const uint64_t *label_offsets,

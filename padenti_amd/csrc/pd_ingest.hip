@@ -313,20 +313,31 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for((uint64_t)n * cap, 256)), dim3(256), 0, st,
                        X.bucket.as<uint32_t>(), (uint64_t)n * cap, 0u);
     tm.mark(2);
-    if (n >= WEIGHTED_BATCH) {
+    // groups of about equal size whose streams fit the scratch (an image
+    // that does not fit alone: windows of it)
+    const uint64_t px = std::max<uint64_t>(max_px, 1), words = std::max<uint64_t>(scratch_bytes / 4u, 1);
+    const uint32_t fit = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, words / px));
+    const uint32_t n_groups = (n + fit - 1) / fit, per = (n + n_groups - 1) / n_groups;
+    const uint32_t win = (uint32_t)((std::min(px, words) + MT_STEP - 1) / MT_STEP * MT_STEP);
+    bool segments = n < WEIGHTED_BATCH && scratch_bytes != 0;
+    // (held from a call with a larger bound)
+    if (X.draws.cap > std::max<uint64_t>(scratch_bytes, (uint64_t)per * win * 4u)) X.draws.release();
+    if (segments) {
+      // device memory short: the walk needs none of it
+      try {
+        X.draws.ensure((size_t)per * win * 4u);
+        if (max_px > win) X.mt_state.ensure((size_t)per * MT_N * 4u);
+        X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
+        X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
+      } catch (const NoMem &) {
+        X.draws.release();
+        segments = false;
+      }
+    }
+    if (!segments) {
       hipLaunchKernelGGL(k_sample_weighted, dim3((n + 3) / 4), dim3(256), 0, st, d_labels, d_jobs, n, crc, s.seed,
                          s.n_classes, d_B, d_boff, X.bucket.as<uint32_t>(), X.class_count.as<uint32_t>(), d_bad);
     } else {
-      // groups of about equal size whose streams fit the scratch (an image
-      // that does not fit alone: windows of it)
-      const uint64_t px = std::max<uint64_t>(max_px, 1), words = std::max<uint64_t>(scratch_bytes / 4u, 1);
-      const uint32_t fit = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, words / px));
-      const uint32_t n_groups = (n + fit - 1) / fit, per = (n + n_groups - 1) / n_groups;
-      const uint32_t win = (uint32_t)((std::min(px, words) + MT_STEP - 1) / MT_STEP * MT_STEP);
-      X.draws.ensure((size_t)per * win * 4u);
-      if (max_px > win) X.mt_state.ensure((size_t)per * MT_N * 4u);
-      X.seg_counts.ensure(std::max<size_t>((size_t)n_segs * s.n_classes, 1) * 4u);
-      X.seg_draw.ensure(std::max<size_t>(n_segs, 1) * sizeof(uint2));
       for (uint32_t g = 0; g < n; g += per) {
         const uint32_t gn = std::min(per, n - g);
         const uint32_t sb = tile0[g], se = g + gn < n ? tile0[g + gn] : n_segs, seg_blocks = (se - sb + 3) / 4;

@@ -180,10 +180,10 @@ def _sample_dev(smp, datas, labs, scratch_bytes):
     return [out[i * cap:i * cap + n_out[i]] for i in range(n)]
 
 
-# words of the random streams at a time: one step of a stream (a segment of 1024
-# pixels meets several windows), windows that end inside segments, whole images
-# in groups of one and two, everything at once
-@pytest.mark.parametrize("words", [1, 3 * 454, 5000, 30000, 61000, 1 << 20])
+# words of the random streams at a time: none (every image walked by a wave), one
+# step of a stream (a segment of 1024 pixels meets several windows), windows that
+# end inside segments, whole images in groups of one and two, everything at once
+@pytest.mark.parametrize("words", [0, 1, 3 * 454, 5000, 30000, 61000, 1 << 20])
 @pytest.mark.parametrize("n_samples", [900, 24000])   # few slots replaced often; as many slots as pixels
 def test_weighted_sampler_scratch_bounds(gpu, words, n_samples):
     rng = np.random.default_rng(words + n_samples)
@@ -196,6 +196,26 @@ def test_weighted_sampler_scratch_bounds(gpu, words, n_samples):
     want, _ = oi.sample_images(1, datas, labs, n_samples, 3, None, seed=21)
     for i, (g, w) in enumerate(zip(got, want)):
         assert np.array_equal(g, w), i
+
+
+def test_weighted_sampler_gives_its_scratch_back(gpu):
+    """A call with a smaller bound frees the streams held from a larger one:
+    the device has that much more free memory afterwards."""
+    def free_bytes():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert lib().hipMemGetInfo(C.byref(a), C.byref(b)) == 0   # of the runtime the library is linked to
+        return a.value
+
+    labs = [np.full((2048, 4096), 1 + i, np.uint8) for i in range(2)]   # 64 MiB of streams
+    datas = [np.zeros(16, np.uint8)] * 2
+    smp = ds.ClassWeightedImageSampler(100, 2, None, seed=1)
+    _sample_dev(smp, datas, labs, 0)
+    free = [free_bytes()]
+    for scratch in (64 << 20, 1 << 20, 64 << 20, 0):
+        _sample_dev(smp, datas, labs, scratch)
+        free.append(free_bytes())
+    held = [free[0] - f for f in free[1:]]
+    assert held[0] - held[1] >= 48 << 20 and held[2] - held[3] >= 48 << 20, held
 
 
 def test_weighted_sampler_rejects_label_above_classes(gpu):
