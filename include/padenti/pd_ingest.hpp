@@ -513,8 +513,9 @@ __global__ __launch_bounds__(256) void k_sample_uniform(const SampleJob *__restr
 //   k_weighted_draw   the segments' pixels, one wave a segment.
 // Only the stream is serial (454 words a step, below).  150 images of 321 x 243,
 // 16 classes: 846 us with one wave an image walking all of it, 102 us now.  The
-// labels are read and ranked twice, so a batch that gives every SIMD a wave of
-// its own (1024 images) keeps the walk, k_sample_weighted (images of 640 x 480, walk
+// labels are read and ranked twice, so a batch that keeps a wave on every SIMD for
+// as long as its largest image takes (1024 images of one size) keeps the walk,
+// k_sample_weighted (images of 640 x 480, walk
 // -> segments: 250 images 2.75 -> 0.70 ms, 500 2.81 -> 1.23, 1000 2.82 -> 2.71; 5000
 // 4.3 -> 8.8).
 //
@@ -816,8 +817,8 @@ __device__ inline void mt_twist_wave(uint32_t *mt, uint32_t lane)
   wave_sync();
 }
 
-// Batches of WEIGHTED_BATCH images and more: one wave per image (four images per
-// block), 64 pixels per step in scan
+// Large batches, and batches without scratch: one wave per image (four images
+// per block), 64 pixels per step in scan
 // order (lane l: pixel t0 + 64 s + l); the label bytes of the next 16 steps
 // are prefetched from global memory.  A pixel's class ordinal k is the class
 // count so far (LDS) plus its rank among the wave's lanes of that class (one

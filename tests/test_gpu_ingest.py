@@ -144,7 +144,10 @@ def test_weighted_sampler_matches_oracle(gpu, n_classes, weights, n_samples):
 @pytest.mark.parametrize("shapes,n_samples", [
     ([(32, 32), (1, 1025), (1, 1023), (48, 64), (1, 1)], 40),   # whole segments, one pixel more and less
     ([(37, 61), (8200, 8200), (227, 4)], 500),                  # one image more than the scratch: groups of one
-    ([(3, 17), (9, 8), (1, 1)] * 342, 10),                      # 1026 images: a wave walks each
+    ([(3, 17), (9, 8), (1, 1)] * 342, 10),                      # 1026 images, 42408 pixels
+    ([(9, 8)] * 1023 + [(1, 72)], 10),                          # 1024 times the largest image: a wave walks each
+    ([(9, 8)] * 1024 + [(1, 73)], 10),                          # a little less: segments
+    ([(3, 5)] * 1100 + [(150, 200)], 2000),                     # one large image among many small ones
 ])
 def test_weighted_sampler_segments_groups_and_windows(gpu, shapes, n_samples):
     rng = np.random.default_rng(n_samples)
