@@ -260,24 +260,26 @@ PD_HD int probe_at(const ImageView<ImgT, NCH> &im, uint32_t ox, uint32_t oy, int
   return v;
 }
 
-// Offset parameters of a hook with a fast form (kFastParams below), converted
+// Offset parameters of a hook with a fast form (FastForm below), converted
 // once per candidate or visited node.
 struct FastParams {
   double p[4];
   int ca, cb;
 };
 
-// A functor with
-//   static constexpr bool kFastParams = true;
+// A functor F with
+//   using FastForm = F;
 //   static FastParams fast_params(const FeatType *p);
 //   static FeatType eval_fast(view, x, y, Prep, const FastParams &);
 // gives eval_prep's result through eval_fast for parameters whose first four
 // entries are at most RECIP_MAX in magnitude; callers check that bound once per
-// launch (feature bounds) or per forest.
+// launch (feature bounds) or per forest.  FastForm names the functor itself: one
+// derived from it has its own eval_prep, which the inherited fast form knows
+// nothing of, and is evaluated through that.
 template <class F, class = void>
 struct has_fast : std::false_type {};
 template <class F>
-struct has_fast<F, std::void_t<decltype(F::kFastParams)>> : std::integral_constant<bool, F::kFastParams> {};
+struct has_fast<F, std::void_t<typename F::FastForm>> : std::is_same<typename F::FastForm, F> {};
 
 // C2/C3: uint16 depth in millimetres, float response; p in pixel*mm,
 // out-of-image reads 10000 mm, d(x) == 0 -> 0.
@@ -289,7 +291,7 @@ struct DepthU16Feature {
   static constexpr int FeatDim = 4;
   static constexpr int kind = 1;
   static constexpr int kProbeRowA = 1, kProbeRowB = 3;   // row offsets of the two probes
-  static constexpr bool kFastParams = true;
+  using FastForm = DepthU16Feature;
   PD_HD static Prep prepare(const ImageView<uint16_t, 1> &im, int x, int y) { return recip_prep(im.at(x, y, 0)); }
   // (a zero depth makes both offsets 0: the two probes read the same texel)
   PD_HD static float eval_prep(const ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const float *p)
@@ -332,7 +334,7 @@ struct RGBDFeature {
     if (c >= 3.0f) return 3;
     return (int)c;
   }
-  static constexpr bool kFastParams = true;
+  using FastForm = RGBDFeature;
   PD_HD static Prep prepare(const ImageView<uint16_t, 4> &im, int x, int y) { return recip_prep(im.at(x, y, 3)); }
   PD_HD static float eval_prep(const ImageView<uint16_t, 4> &im, int x, int y, Prep dp, const float *p)
   {
