@@ -293,9 +293,9 @@ struct DepthU16Feature {
   static constexpr int kProbeRowA = 1, kProbeRowB = 3;   // row offsets of the two probes
   using FastForm = DepthU16Feature;
   PD_HD static Prep prepare(const ImageView<uint16_t, 1> &im, int x, int y) { return recip_prep(im.at(x, y, 0)); }
-  // (a zero depth makes both offsets 0: the two probes read the same texel)
   PD_HD static float eval_prep(const ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const float *p)
   {
+    if (!(dp.y > 0.0)) return 0.0f;   // (an infinite offset times 0 is no coordinate)
     const int a = probe_at(im, recip_coord_any(x, p[0], dp), recip_coord_any(y, p[1], dp), 0, 10000);
     const int b = probe_at(im, recip_coord_any(x, p[2], dp), recip_coord_any(y, p[3], dp), 0, 10000);
     return (float)(a - b);
@@ -304,6 +304,7 @@ struct DepthU16Feature {
   {
     return FastParams{{(double)p[0], (double)p[1], (double)p[2], (double)p[3]}, 0, 0};
   }
+  // (a zero depth makes both offsets 0: the two probes read the same texel)
   PD_HD static float eval_fast(const ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const FastParams &f)
   {
     const int a = probe_at(im, recip_coord(x, f.p[0], dp), recip_coord(y, f.p[1], dp), 0, 10000);
