@@ -260,6 +260,16 @@ PD_HD int probe_at(const ImageView<ImgT, NCH> &im, uint32_t ox, uint32_t oy, int
   return v;
 }
 
+// The same at x + round(px/d), y + round(py/d) with an integer depth d > 0
+// (IntDivPrep).
+template <typename ImgT, int NCH>
+PD_HD int probe_int(const ImageView<ImgT, NCH> &im, int x, int y, const IntDivPrep &dp, float px, float py, int ch,
+                    int bg)
+{
+  return probe_at(im, (uint32_t)x + (uint32_t)offset_of_num(int_div(px, dp), px),
+                  (uint32_t)y + (uint32_t)offset_of_num(int_div(py, dp), py), ch, bg);
+}
+
 // Offset parameters of a hook with a fast form (FastForm below), converted
 // once per candidate or visited node.
 struct FastParams {

@@ -21,6 +21,26 @@ struct NegatedDepth : pd::DepthU16Feature {
   }
 };
 
+// a user's hook on the header's integer-depth probe
+struct UserDepth {
+  using ImgType = uint16_t;
+  using FeatType = float;
+  using Prep = pd::IntDivPrep;
+  static constexpr int nChannels = 1;
+  static constexpr int FeatDim = 4;
+  static Prep prepare(const pd::ImageView<uint16_t, 1> &im, int x, int y)
+  {
+    return pd::int_div_prep((float)im.at(x, y, 0));
+  }
+  static float eval_prep(const pd::ImageView<uint16_t, 1> &im, int x, int y, Prep dp, const float *p)
+  {
+    if (!(dp.d > 0.0f)) return 0.0f;
+    const int a = pd::probe_int(im, x, y, dp, p[0], p[1], 0, 10000);
+    const int b = pd::probe_int(im, x, y, dp, p[2], p[3], 0, 10000);
+    return (float)(a - b);
+  }
+};
+
 extern "C" {
 int has_fast_depth(void) { return pd::has_fast<pd::DepthU16Feature>::value; }
 int has_fast_rgbd(void) { return pd::has_fast<pd::RGBDFeature>::value; }
@@ -29,6 +49,17 @@ int has_fast_derived(void) { return pd::has_fast<NegatedDepth>::value; }
 float depth_u16(const uint16_t *im, int w, int h, int x, int y, const float *p)
 {
   return pd::DepthU16Feature::eval(pd::ImageView<uint16_t, 1>{im, w, h}, x, y, p);
+}
+float depth_u16_fast(const uint16_t *im, int w, int h, int x, int y, const float *p)
+{
+  using F = pd::DepthU16Feature;
+  const pd::ImageView<uint16_t, 1> v{im, w, h};
+  return F::eval_fast(v, x, y, F::prepare(v, x, y), F::fast_params(p));
+}
+float user_depth(const uint16_t *im, int w, int h, int x, int y, const float *p)
+{
+  const pd::ImageView<uint16_t, 1> v{im, w, h};
+  return UserDepth::eval_prep(v, x, y, UserDepth::prepare(v, x, y), p);
 }
 }
 """
@@ -42,7 +73,8 @@ def host(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-Wno-unknown-pragmas", "-fPIC", "-shared", "-I",
                     os.path.join(ROOT, "include"), str(src), "-o", str(lib)], check=True)
     so = C.CDLL(str(lib))
-    so.depth_u16.restype = C.c_float
+    for f in (so.depth_u16, so.depth_u16_fast, so.user_depth):
+        f.restype = C.c_float
     return so
 
 
@@ -60,3 +92,21 @@ def test_zero_depth_gives_zero_for_every_offset(host, p):
     im[2, 2] = 0
     a = np.array(p, np.float32)
     assert host.depth_u16(im.ctypes.data_as(C.c_void_p), 5, 5, 2, 2, a.ctypes.data_as(C.c_void_p)) == 0.0
+
+
+def test_integer_depth_probe_for_user_hooks(host):
+    """A hook written with int_div_prep / probe_int compiles and gives the
+    shipped depth hook's response, in its general and its fast form."""
+    rng = np.random.default_rng(8)
+    im = rng.choice(np.array([0, 1, 2, 3, 64, 1000, 4096, 65535], np.uint16), (17, 23))
+    pi = im.ctypes.data_as(C.c_void_p)
+    for _ in range(3000):
+        x, y = int(rng.integers(23)), int(rng.integers(17))
+        d = max(int(im[y, x]), 1)
+        # offsets of a few pixels, every other one on a half
+        p = np.array([(int(k) / 2) * d for k in rng.integers(-30, 31, 4)], np.float32)
+        p = np.clip(p, -4194304, 4194304) * (1 if rng.random() < 0.5 else np.float32(rng.uniform(0.9, 1.0)))
+        pp = p.ctypes.data_as(C.c_void_p)
+        want = host.user_depth(pi, 23, 17, x, y, pp)
+        assert host.depth_u16(pi, 23, 17, x, y, pp) == want, (x, y, p)
+        assert host.depth_u16_fast(pi, 23, 17, x, y, pp) == want, (x, y, p)
