@@ -46,6 +46,36 @@ int has_fast_depth(void) { return pd::has_fast<pd::DepthU16Feature>::value; }
 int has_fast_rgbd(void) { return pd::has_fast<pd::RGBDFeature>::value; }
 int has_fast_f32(void) { return pd::has_fast<pd::DepthF32Feature>::value; }
 int has_fast_derived(void) { return pd::has_fast<NegatedDepth>::value; }
+// mismatches of the coordinate rules with x + roundf(p / d) at the quotients that
+// are exactly halves, (n + 1/2) d <= 2^22 of every n for d in [d0, d1), and at the
+// floats next to them, both signs
+static uint64_t bad_at(uint32_t x, float p, uint32_t d, bool any)
+{
+  const pd::RecipPrep y = pd::recip_prep(d);
+  const uint32_t want = x + (uint32_t)(int)roundf(p / (float)d);
+  uint64_t bad = 0;
+  if (fabsf(p) <= pd::RECIP_MAX) bad += pd::recip_coord(x, (double)p, y) != want;
+  // (the general form takes every quotient from 2^20 on as outside)
+  if (any && fabsf(p / (float)d) < 1048576.0f) bad += pd::recip_coord_any(x, p, y) != want;
+  return bad;
+}
+uint64_t bad_halves(uint32_t d0, uint32_t d1)
+{
+  uint64_t bad = 0;
+  for (uint32_t d = d0; d < d1; d++)
+    for (uint64_t h = d; h <= 2ull << 22; h += 2ull * d) {   // h / 2 = (n + 1/2) d, a float
+      const float p = (float)h * 0.5f, c[3] = {p, nextafterf(p, 0.0f), nextafterf(p, INFINITY)};
+      const uint32_t x = (uint32_t)(h * 2654435761u) >> 16;
+      for (float q : c) bad += bad_at(x, q, d, true) + bad_at(x, -q, d, true);
+    }
+  return bad;
+}
+uint64_t bad_of(uint64_t n, const uint32_t *x, const float *p, const uint32_t *d)
+{
+  uint64_t bad = 0;
+  for (uint64_t i = 0; i < n; i++) bad += bad_at(x[i], p[i], d[i], true);
+  return bad;
+}
 float depth_u16(const uint16_t *im, int w, int h, int x, int y, const float *p)
 {
   return pd::DepthU16Feature::eval(pd::ImageView<uint16_t, 1>{im, w, h}, x, y, p);
@@ -75,6 +105,7 @@ def host(tmp_path_factory):
     so = C.CDLL(str(lib))
     for f in (so.depth_u16, so.depth_u16_fast, so.user_depth):
         f.restype = C.c_float
+    so.bad_halves.restype = so.bad_of.restype = C.c_uint64
     return so
 
 
@@ -110,3 +141,26 @@ def test_integer_depth_probe_for_user_hooks(host):
         want = host.user_depth(pi, 23, 17, x, y, pp)
         assert host.depth_u16(pi, 23, 17, x, y, pp) == want, (x, y, p)
         assert host.depth_u16_fast(pi, 23, 17, x, y, pp) == want, (x, y, p)
+
+
+@pytest.mark.parametrize("d0,d1", [(1, 2), (2, 3), (3, 16), (16, 256), (256, 4096), (4096, 65536)])
+def test_coordinate_of_every_half(host, d0, d1):
+    """recip_coord and recip_coord_any against x + roundf(p / d) at every
+    half-integer quotient of the fast form's range and the floats beside it."""
+    assert host.bad_halves(d0, d1) == 0
+
+
+def test_coordinate_of_random_offsets(host):
+    rng = np.random.default_rng(6)
+    n = 4_000_000
+    d = rng.integers(1, 65536, n).astype(np.uint32)
+    d[: n // 4] = rng.integers(1, 64, n // 4)
+    x = rng.integers(0, 65536, n).astype(np.uint32)
+    x[::3] = 0                                        # sums below zero
+    p = rng.uniform(-4194304, 4194304, n)
+    p[1::4] = np.exp(rng.uniform(-30, 26, n)[1::4]) * rng.choice([-1, 1], n)[1::4]   # every magnitude
+    p[2::4] = rng.integers(-4194304, 4194305, n)[2::4]                                # whole numbers
+    p[:8] = [4194304, -4194304, 4194303.5, -4194303.5, 0.0, -0.0, 1e-40, -1e-40]
+    p = p.astype(np.float32)
+    assert host.bad_of(C.c_uint64(n), x.ctypes.data_as(C.c_void_p), p.ctypes.data_as(C.c_void_p),
+                       d.ctypes.data_as(C.c_void_p)) == 0
