@@ -11,6 +11,7 @@
 // cl_classifier_impl.hpp:41-557 (classifier).
 #pragma once
 #include "../padenti_hip.h"
+#include "pd_placement.hpp"
 #include "pd_kernels.hpp"
 #include "pd_runtime.hpp"
 
@@ -753,20 +754,12 @@ struct Trainer final : TrainerBase {
   // candidates per histogram tile
   uint32_t hist_fpw(uint32_t nT) const { return 64u / hist_spw(nT); }
 
-  uint32_t pick_chunk(uint64_t level_samples, uint32_t ftiles) const
+  uint32_t pick_chunk(uint64_t level_samples, uint32_t nF, uint32_t nT, uint32_t launches = 1) const
   {
     if (chunk) return std::max<uint32_t>(64u, std::min<uint32_t>(chunk, 32768u));
-    const uint64_t target_blocks = (uint64_t)cu_count * tune.blocks_per_cu;
-    uint64_t c = (level_samples * ftiles + target_blocks - 1) / target_blocks;
-    // at least 1024 samples an item (shorter ones pay for the candidate set-up
-    // and the histogram flush), down to 64 where the level would otherwise
-    // leave CUs without two items: a wave walks its samples one after the
-    // other, so a level of few items lasts as long as one of them (8192 samples
-    // x 100 candidates: 92 us a level in 16 items of 1024, 17 us in 256 of 64)
-    const uint64_t two_per_cu = level_samples * ftiles / (2u * (uint64_t)cu_count);
-    c = std::max<uint64_t>(c, std::min<uint64_t>(std::max<uint64_t>(two_per_cu, 64u), 1024u));
-    c = std::min<uint64_t>(c, 32768u);
-    return (uint32_t)c;
+    const uint32_t fpw = hist_fpw(nT);
+    return item_chunk(level_samples, nF, (nF + fpw - 1) / fpw, nT, nC, (uint32_t)cu_count, tune.blocks_per_cu,
+                      launches);
   }
 
   template <int NTP>
@@ -1312,7 +1305,7 @@ struct Trainer final : TrainerBase {
     Pe.n_thresholds = 1;
     d_map_cur = rows.map;
     hist_slice(full, 0, ns, act, Pe, bnd, tree, PD_MODE_LEVEL_BATCHED,
-               pick_chunk(cnt, (screen + hist_fpw(1) - 1) / hist_fpw(1)), T, true, hslots);
+               pick_chunk(cnt, screen, 1), T, true, hslots);
     d_map_cur = nullptr;
     const uint32_t nh = (uint32_t)hslots.size();
     d_full.ensure((size_t)ns * screen * sizeof(float));
@@ -1467,7 +1460,7 @@ struct Trainer final : TrainerBase {
     pd_train_params Pe = P;
     Pe.n_features = screen;
     Pe.n_thresholds = 1;
-    const uint32_t ch = pick_chunk(total, (screen + hist_fpw(1) - 1) / hist_fpw(1));
+    const uint32_t ch = pick_chunk(total, screen, 1);
     const size_t per_bytes = (size_t)nC * screen * sizeof(uint32_t);
     const size_t h_per_slice = std::max<size_t>(
         1, std::min<size_t>(hist_budget / per_bytes, (1ull << 30) / ((size_t)screen * 4)));
@@ -1662,14 +1655,14 @@ struct Trainer final : TrainerBase {
         dmap = d_map2.as<uint32_t>();
       }
       evaluate(slots, gidx, act, P, keep, dmap, &hmap, bnd, tree, PD_MODE_LEVEL_BATCHED,
-               pick_chunk(gact, (keep + hist_fpw(1) - 1) / hist_fpw(1)), classTot, level, false, res_all, st);
+               pick_chunk(gact, keep, 1), classTot, level, false, res_all, st);
       if (prop_judge) {
         std::vector<uint32_t> res_j(slots.size() * (nC + 2), 0u);
         pd_level_stats js{};
         std::vector<T> *keep_par = lvl_par, *keep_thr = lvl_thr;
         lvl_par = lvl_thr = nullptr;   // the judge's winners are not the tree's
         evaluate(slots, gidx, act, P, K, nullptr, nullptr, bnd, tree, PD_MODE_LEVEL_BATCHED,
-                 pick_chunk(gact, (K + hist_fpw(1) - 1) / hist_fpw(1)), classTot, level, false, res_j, js);
+                 pick_chunk(gact, K, 1), classTot, level, false, res_j, js);
         lvl_par = keep_par;
         lvl_thr = keep_thr;
         st.judge_ms += js.hist_ms + js.split_ms;
@@ -1819,7 +1812,8 @@ struct Trainer final : TrainerBase {
       for (const SlotInfo &s : slots) n_trainable += s.trainable ? 1u : 0u;
       const pd_tuning keep_tune = tune;
       tune = level_tuning(active, n_trainable);
-      uint32_t ch = pick_chunk(active, (nF + hist_fpw(nT) - 1) / hist_fpw(nT));
+      uint32_t ch = pick_chunk(active, nF, nT,
+                               mode == PD_MODE_PER_NODE ? std::max<uint32_t>(n_trainable, 1u) : 1u);
       std::vector<uint8_t> split_flag(slots.size(), 0);
       // per-slot result: k = t * nF + f (sampler index f), FP32 gain bits, left counts
       std::vector<uint32_t> res_all(slots.size() * (nC + 2), 0u);
@@ -2017,7 +2011,7 @@ struct Trainer final : TrainerBase {
     const Bounds<F> bnd = make_bounds<F>(P);
     std::vector<uint32_t> idx(n_nodes), res_all((size_t)n_nodes * (nC + 2));
     for (uint32_t q = 0; q < n_nodes; q++) idx[q] = q;
-    const uint32_t ch = pick_chunk(S, (P.n_features + hist_fpw(P.n_thresholds) - 1) / hist_fpw(P.n_thresholds));
+    const uint32_t ch = pick_chunk(S, P.n_features, P.n_thresholds);
     pd_level_stats st{};
     evaluate(slots, idx, d_actA.as<uint4>(), P, P.n_features, nullptr, nullptr, bnd, tree_id, PD_MODE_LEVEL_BATCHED,
              ch, classTot.data(), 1, false, res_all, st);   // warm-up (module load, buffers)
@@ -2058,7 +2052,7 @@ struct Trainer final : TrainerBase {
     if (!act.empty())
       HIPCHK(hipMemcpyAsync(d_actA.p, act.data(), act.size() * sizeof(uint4), hipMemcpyHostToDevice, stream));
     const Bounds<F> bnd = make_bounds<F>(P);
-    const uint32_t ch = pick_chunk(act.size(), (P.n_features + hist_fpw(P.n_thresholds) - 1) / hist_fpw(P.n_thresholds));
+    const uint32_t ch = pick_chunk(act.size(), P.n_features, P.n_thresholds);
     std::vector<uint32_t> tot((size_t)n_nodes * nC, 0u), hslots;
     hist_slice(slots, 0, slots.size(), d_actA.as<uint4>(), P, bnd, tree_id, PD_MODE_LEVEL_BATCHED, ch, tot, true,
                hslots);
