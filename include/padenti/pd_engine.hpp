@@ -914,44 +914,12 @@ struct Trainer final : TrainerBase {
     }
     // direct: the items are written into pinned staging and copied from there
     size_t n_items = 0;
-    std::vector<uint32_t> order, xcd;   // launch order of the groups and their XCDs (direct)
+    GroupOrder deal;   // (direct)
     if (direct) {
-      // Groups in node order, except that the smallest ones (a tenth of the
-      // samples together) come last, largest first, so that a level does not
-      // end on a long block; each goes to the XCD with the fewest samples so
-      // far.  Dealt round robin, one of 47 random-sized groups an XCD is some
-      // 8% above the mean; sorted by size throughout, the blocks resident on a
-      // CU run their gather-bound and their split phases at the same time.
-      // 351 nodes of 500..6000 samples, 2000 x 20 candidates: 5.7 -> 5.2 ms a
-      // level, 968 nodes 7.6 -> 6.8 ms (round robin -> this); sorted by size
-      // throughout, the histograms of a 16-level tree took 77.7 ms instead of 73.2
-      // (round robin 75.0).
-      const size_t X = n_xcc, ng = groups.size();
-      order.resize(ng);
-      xcd.resize(ng);
-      for (size_t g = 0; g < ng; g++) order[g] = (uint32_t)g;
-      uint64_t all = 0;
-      for (const uint4 &g : groups) all += g.z;
-      std::vector<uint32_t> by_size(order);
-      std::stable_sort(by_size.begin(), by_size.end(),
-                       [&](uint32_t x, uint32_t y) { return groups[x].z > groups[y].z; });
-      uint64_t rest = 0;
-      size_t cut = ng;   // by_size[cut..) come last
-      while (cut > 0 && rest + groups[by_size[cut - 1]].z <= all / 10) rest += groups[by_size[--cut]].z;
-      std::vector<uint8_t> last(ng, 0);
-      for (size_t i = cut; i < ng; i++) last[by_size[i]] = 1;
-      size_t w = 0;
-      for (size_t g = 0; g < ng; g++)
-        if (!last[g]) order[w++] = (uint32_t)g;
-      std::copy(by_size.begin() + cut, by_size.end(), order.begin() + w);
-      std::vector<uint64_t> load(X, 0), len(X, 0);
-      for (uint32_t g : order) {
-        const size_t x = std::min_element(load.begin(), load.end()) - load.begin();
-        xcd[g] = (uint32_t)x;
-        load[x] += groups[g].z + 64u;   // (a block costs something without samples too)
-        len[x] += ftiles;
-      }
-      n_items = *std::max_element(len.begin(), len.end()) * X;
+      std::vector<uint32_t> sizes(groups.size());
+      for (size_t g = 0; g < groups.size(); g++) sizes[g] = groups[g].z;
+      deal = deal_groups(sizes, n_xcc);
+      n_items = deal.rows * ftiles * n_xcc;
     } else {
       item_start[ns] = (uint32_t)items.size();
       group_start.push_back((uint32_t)items.size());
@@ -979,11 +947,12 @@ struct Trainer final : TrainerBase {
       HistItem *it = up.template host<HistItem>(u_items);
       std::fill(it, it + n_items, HistItem{NULL_SLOT, 0u, 0u, 0u});
       std::vector<uint64_t> len(n_xcc, 0);
-      for (uint32_t g : order) {
+      for (uint32_t g : deal.order) {
         const uint4 gr = groups[g];
-        HistItem *dst = it + len[xcd[g]] * n_xcc + xcd[g];
+        const uint32_t x = deal.xcd[g];
+        HistItem *dst = it + len[x] * n_xcc + x;
         for (uint32_t ft = 0; ft < ftiles; ft++) dst[(size_t)ft * n_xcc] = HistItem{gr.x, gr.y, gr.z, ft};
-        len[xcd[g]] += ftiles;
+        len[x] += ftiles;
       }
     }
     up.commit();
@@ -1034,8 +1003,11 @@ struct Trainer final : TrainerBase {
     // table and H zeroing before them are not the kernel being timed)
     if (ev_begin) HIPCHK(hipEventRecord(ev_begin->e, stream));
     if (mode == PD_MODE_LEVEL_BATCHED) {
-      launch_hist((uint32_t)n_items, 0, act, bnd, tree, nF, nT);
-      launches += n_items ? 1 : 0;
+      // (a launch holds fewer than 2^32 threads, 1024 an item at most; the padding
+      // counts too)
+      const size_t most = ((size_t)4000000 / n_xcc) * n_xcc;
+      for (size_t b = 0; b < n_items; b += most, launches++)
+        launch_hist((uint32_t)std::min(most, n_items - b), (uint32_t)b, act, bnd, tree, nF, nT);
     } else {
       for (uint32_t q = 0; q < ns; q++) {
         const uint32_t n = item_start[q + 1] - item_start[q];

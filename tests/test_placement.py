@@ -18,6 +18,13 @@ uint32_t item_chunk(uint64_t level_samples, uint32_t nF, uint32_t ftiles, uint32
 {
   return pd::engine::item_chunk(level_samples, nF, ftiles, nT, nC, cus, blocks_per_cu, launches);
 }
+size_t deal(size_t n, const uint32_t *samples, uint32_t n_xcc, uint32_t *order, uint32_t *xcd)
+{
+  const pd::engine::GroupOrder r = pd::engine::deal_groups(std::vector<uint32_t>(samples, samples + n), n_xcc);
+  std::copy(r.order.begin(), r.order.end(), order);
+  std::copy(r.xcd.begin(), r.xcd.end(), xcd);
+  return r.rows;
+}
 }
 """
 
@@ -29,7 +36,9 @@ def host(tmp_path_factory):
     src.write_text(SRC)
     subprocess.run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-I", os.path.join(ROOT, "include"), str(src), "-o",
                     str(lib)], check=True)
-    return C.CDLL(str(lib))
+    so = C.CDLL(str(lib))
+    so.deal.restype, so.deal.argtypes = C.c_size_t, [C.c_size_t, C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p]
+    return so
 
 
 def _chunk(host, samples, nF, nT, nC, cus=256, blocks=16, launches=1):
@@ -51,3 +60,36 @@ def test_chunks_of_small_levels_weigh_the_flush(host):
     assert _chunk(host, 8000, 500, 10, 8, launches=64) == 8000 * 8 // 512
     assert _chunk(host, 10_000_000, 4000, 32, 16) == 32768   # large levels: blocks_per_cu items a CU
     assert _chunk(host, 1_000_000, 2000, 20, 8) == -(-1_000_000 * 32 // (256 * 16))
+
+
+def _deal(host, samples, X):
+    n = len(samples)
+    a, order, xcd = (C.c_uint32 * n)(*samples), (C.c_uint32 * n)(), (C.c_uint32 * n)()
+    rows = host.deal(n, a, X, order, xcd)
+    return list(order), list(xcd), rows
+
+
+@pytest.mark.parametrize("X", [2, 4, 8])
+@pytest.mark.parametrize("samples", [
+    [1000], [5, 0, 7], [0] * 50, [11] * 64, [11] * 65,
+    [50000] * 16 + [20] * 6000,                       # a few large groups among many tiny ones
+    [400000] + [1] * 3000,
+    [32768] * 3 + [0] * 4000,
+    [30000] * 7 + [20] * 350,                         # the tiny ones would all go to the eighth XCD
+    [(i * 2654435761 >> 7) % 5500 + 500 for i in range(968)],
+])
+def test_groups_are_dealt_once_and_evenly(host, samples, X):
+    """Every group is launched once; the padding of the interleaved lists stays
+    within a quarter of the groups (one row more), and where that does not bind
+    the XCDs' shares differ by at most one group."""
+    order, xcd, rows = _deal(host, samples, X)
+    assert sorted(order) == list(range(len(samples)))
+    per = [xcd.count(x) for x in range(X)]
+    assert sum(per) == len(samples) and max(per) == rows
+    share = -(-len(samples) // X)
+    assert rows <= share + share // 4 + 1
+    load = [sum(samples[g] + 64 for g in range(len(samples)) if xcd[g] == x) for x in range(X)]
+    if rows < share + share // 4 + 1:
+        assert max(load) - min(load) <= max(samples) + 64
+    if len(set(samples)) > 1:   # the smallest ones come last
+        assert samples[order[-1]] == min(samples)
