@@ -726,11 +726,15 @@ __global__ __launch_bounds__(NWAVES * 64) void k_hist(
   // column of the winner (every wave holds the same lane -> column map; the
   // lowest such lane is the column itself)
   const uint64_t wmask = __ballot(fv && f == key_index(m) % nF);
-  if (m != 0ull && tid < nC) {
-    const uint32_t k = key_index(m);
-    const uint32_t wl = (uint32_t)__builtin_ctzll(wmask) % FPW;
-    const uint32_t l = sl[(k / nF) * FPW + wl];
-    cand_left[ci * nC + tid] = prefix_at<WIDE, (int)FPW>(bins, RW, tid, l, wl);
+  if (tid < nC) {
+    uint32_t left = 0;
+    if (m != 0ull) {   // (0: no pair was evaluated, see k_finalize)
+      const uint32_t k = key_index(m);
+      const uint32_t wl = (uint32_t)__builtin_ctzll(wmask) % FPW;
+      const uint32_t l = sl[(k / nF) * FPW + wl];
+      left = prefix_at<WIDE, (int)FPW>(bins, RW, tid, l, wl);
+    }
+    cand_left[ci * nC + tid] = left;
   }
 }
 
@@ -1103,7 +1107,11 @@ __global__ void k_finalize(const uint32_t *__restrict__ H, const unsigned long l
     key = best[slot];
   }
   uint32_t k = key_index(key);
-  if (k >= nT * nF) k = 0;   // unreachable: every slot evaluates pair 0
+  // A search of a slot that holds samples evaluates some pair: k_split all of them,
+  // the fused search at least the one with the tile's largest approximation, which
+  // is finite.  (An empty fused slot, N = 0, would evaluate none: key 0, pair 0, no
+  // left samples.  Frontier nodes hold samples and train() refuses an empty set.)
+  if (k >= nT * nF) k = 0;
   uint32_t *r = res + (size_t)slot * (nC + 2);
   if (c == 0) {
     r[0] = k;
