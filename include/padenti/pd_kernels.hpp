@@ -227,7 +227,7 @@ __device__ __forceinline__ float count_klogk(uint32_t k)
 // samples holding n classes (bits).  Approximate: h - (f(nL) + f(nR) - sum
 // f(lc) - sum f(rc)) / N with f = count_klogk.  The counts of the four groups
 // add up to 2N, and log2 k < 16: logarithms within 2^-20 (the hardware's over
-// all k <= 65535, measured) and the products' roundings (2^-24 of at most 16)
+// all k <= 65535; test_count_logarithm_bound) and the products' roundings (2^-24 of at most 16)
 // add up to 2 * (2^-20 + 2^-20) = 4e-6, each of the 2n + 3 sums rounds by at
 // most 16 * 2^-24 = 1e-6, the last three operations by 3e-6.  The FP32 gain: n
 // terms a side, every partial sum at most log2 n <= 6, so n * 6 * 2^-24 =
@@ -1618,6 +1618,12 @@ __global__ void k_div_int(const float *__restrict__ p, const float *__restrict__
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   q[i] = int_div(p[i], int_div_prep(d[i]));
+}
+
+__global__ void k_count_klogk(const uint32_t *__restrict__ k, float *__restrict__ out, uint32_t n)
+{
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = count_klogk(k[i]);
 }
 
 // Plain streaming copy (16 B per lane per step): HBM bandwidth probe and the

@@ -230,6 +230,8 @@ PD_API int pd_fast_div(int device, uint32_t n, const float *p, const float *d, f
  * hooks (d[i] an integer, 1 <= |d[i]| <= 65535, any p[i]) and of the split
  * search's class fractions (p[i] <= d[i] < 2^21, both integers). */
 PD_API int pd_int_div(int device, uint32_t n, const float *p, const float *d, float *q);
+/* out[i] = k[i] log2 k[i] (0 for 0) as the fused split search approximates it. */
+PD_API int pd_count_klogk(int device, uint32_t n, const uint32_t *k, float *out);
 PD_API int pd_feature_eval(int device, int feature_kind, const void *image, uint32_t w, uint32_t h, uint32_t n,
                     const int32_t *xy, const void *params, void *out);
 

@@ -270,6 +270,22 @@ int pd_int_div(int device, uint32_t n, const float *p, const float *d, float *q)
   });
 }
 
+int pd_count_klogk(int device, uint32_t n, const uint32_t *k, float *out)
+{
+  return guarded([&] {
+    require(n >= 1 && k && out, "bad arguments");
+    set_device(device);
+    DevBuf dk, dout;
+    dk.ensure((size_t)n * 4);
+    dout.ensure((size_t)n * 4);
+    HIPCHK(hipMemcpy(dk.p, k, (size_t)n * 4, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_count_klogk, dim3((n + 255) / 256), dim3(256), 0, nullptr, dk.as<uint32_t>(),
+                       dout.as<float>(), n);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpy(out, dout.p, (size_t)n * 4, hipMemcpyDeviceToHost));
+  });
+}
+
 int pd_log2_det(int device, uint32_t n, const float *x, float *y)
 {
   return guarded([&] {

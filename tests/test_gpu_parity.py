@@ -1004,6 +1004,20 @@ def test_pruned_split_search_equals_exhaustive(gpu, kind, n_classes, nF, nT, lev
     tr.close()
 
 
+def test_count_logarithm_bound(gpu):
+    """The bound of the approximate gain (gain_slack) takes the hardware
+    logarithm of a count as within 2^-20 and its product with the count as
+    rounded once (2^-24 of at most 16 k): k log2 k is within k 2^-19 for every
+    count of a fused node."""
+    k = np.arange(65536, dtype=np.uint32)
+    out = np.full(k.size, np.nan, np.float32)
+    L.check(L.lib().pd_count_klogk(0, k.size, L.ptr(k), L.ptr(out)))
+    assert out[0] == 0.0 and out[1] == 0.0
+    want = k[1:].astype(np.float64) * np.log2(k[1:].astype(np.float64))
+    err = np.abs(out[1:].astype(np.float64) - want) / k[1:]
+    assert err.max() <= 2.0 ** -19, (int(err.argmax()) + 1, err.max())
+
+
 @pytest.mark.parametrize("kind", [pa.PD_FEAT_DEPTH_U16, pa.PD_FEAT_RGBD_U16X4])
 @pytest.mark.parametrize("bound", [1000.0, 4194304.0, 4194308.0, 3e9])
 def test_fast_offset_form_equals_oracle(gpu, kind, bound):
