@@ -160,9 +160,10 @@ __device__ __forceinline__ float gelu_sig(float z, float zz)
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * __builtin_fmaf(zz, GELU_K3, GELU_K1)));
 }
 // d gelu / dz = s + 2 z s (1 - s) u',  s = sigmoid(2u) = gelu_sig(z), h = z s, u' = c (1 + 3 a z^2)
+// (u' kept finite: h (1 - s) is 0 long before z^2 overflows)
 __device__ __forceinline__ float gelu_grad(float zz, float s, float h)
 {
-  const float du = __builtin_fmaf(zz, 6.0f * GELU_A * GELU_C, 2.0f * GELU_C);
+  const float du = __builtin_fmaf(fminf(zz, 1e30f), 6.0f * GELU_A * GELU_C, 2.0f * GELU_C);
   return __builtin_fmaf(h * (1.0f - s), du, s);
 }
 

@@ -85,6 +85,33 @@ def test_gradients_match_oracle(gpu, n):
     net.close()
 
 
+@pytest.mark.parametrize("n", [700, 9000, 33000])
+@pytest.mark.parametrize("z", [3e5, 1e19, 3e19])   # z^2 in FP32: finite, finite, infinite
+def test_gradients_with_saturated_units(gpu, n, z):
+    """Units far out on either side of the GELU (gelu' is 1 and 0 there) leave
+    every gradient finite and the oracle's."""
+    theta = om.init_params(6, scale=2.0)
+    q = om.unpack(theta)
+    q["W1"][:2], q["b1"][:2], q["W2"][:, :2] = 0.0, (z, -z), 0.0   # (views of theta's own values)
+    theta = om.pack(q)
+    net = pp.SplitProposalNet(seed=12)
+    net.params = theta
+    theta = net.params
+    x = _rows(n, 7)
+    t = np.random.default_rng(8).uniform(0, 1, size=n).astype(np.float32)
+    g, loss = net.grad(x, t)
+    lref, gref = om.loss_and_grad(theta, x, t, bf16_mode=True)
+    assert np.all(np.isfinite(g)) and abs(loss - lref) <= 1e-4 * lref
+    p, q = om.unpack(g), om.unpack(gref)
+    big_p, big_q = p["W2"][:, :2].copy(), q["W2"][:, :2].copy()
+    assert np.linalg.norm(big_p - big_q) <= 2e-2 * np.linalg.norm(big_q)
+    p["W2"][:, :2] = q["W2"][:, :2] = 0.0
+    for name, _ in om.SIZES:
+        err = np.linalg.norm(p[name] - q[name]) / np.linalg.norm(q[name])
+        assert err < 2e-2, (name, err)
+    net.close()
+
+
 def test_adam_steps_match_oracle(gpu):
     net = pp.SplitProposalNet(seed=13)
     x = _rows(512, 4)
