@@ -210,19 +210,33 @@ __global__ __launch_bounds__(256) void k_crc32(const CrcJob *__restrict__ jobs, 
 }
 
 // crc32 = pure ^ (0xFFFFFFFF * x^(8 len)) ^ 0xFFFFFFFF, pure = acc_a * x^(8 q) ^ acc_b
-// with q the length of the last block from a0 (at most 4096).  One wave per
-// image: lane k < 16 holds the factor of bit k of q, lane 16 + k that of bit k of
-// len (below 2^44), multiplied in a tree (one thread walking the bits: 11.5 us
-// for 150 images, now 8.2).  The grid is bounded; its waves go on by its size.
-__global__ __launch_bounds__(256) void k_crc_final(const CrcJob *__restrict__ jobs, uint32_t n_images,
-                                                   const uint32_t *__restrict__ acc_a,
-                                                   const uint32_t *__restrict__ acc_b, uint32_t *crc_out)
+// with q the length of the last block from a0 (at most 4096).
+__device__ __forceinline__ uint32_t crc_join(const CrcJob &J, uint32_t a, uint32_t b, uint32_t xq, uint32_t xlen)
+{
+  const uint32_t pure = J.n_blocks ? gf2_mul(a, xq) ^ b : 0u;
+  return pure ^ gf2_mul(0xFFFFFFFFu, xlen) ^ 0xFFFFFFFFu;
+}
+__device__ __forceinline__ uint64_t crc_tail(const CrcJob &J)
+{
+  return J.n_blocks ? J.end - J.a0 - 4096ull * (J.n_blocks - 1u) : 0ull;
+}
+
+// Up to CRC_WAVES images: one wave per image, lane k < 16 holding the factor of
+// bit k of q, lane 16 + k that of bit k of len (below 2^44), multiplied in a tree
+// (a thread walking the bits: 11.5 us for 150 images, the wave 8.2).  A wave does
+// all 1300 operations of the tree whatever the bits, so beyond a wave a SIMD the
+// images add up (5000 of them 20 us, 100000 0.4 ms) and a thread an image is the
+// faster form again (7 us, and 1.16 instead of 1.56 ms for the whole CRC of 100000
+// images of 3000 bytes).  The grids are bounded; they go on by their size.
+constexpr uint32_t CRC_WAVES = 1024;
+__global__ __launch_bounds__(256) void k_crc_final_wave(const CrcJob *__restrict__ jobs, uint32_t n_images,
+                                                        const uint32_t *__restrict__ acc_a,
+                                                        const uint32_t *__restrict__ acc_b, uint32_t *crc_out)
 {
   const uint32_t lane = threadIdx.x & 63u;
   for (uint64_t i = blockIdx.x * 4u + (threadIdx.x >> 6); i < n_images; i += gridDim.x * 4u) {
     const CrcJob J = jobs[i];
-    const uint64_t q = J.n_blocks ? J.end - J.a0 - 4096ull * (J.n_blocks - 1u) : 0ull;
-    const uint64_t n = lane < 16u ? q : J.end - J.start;
+    const uint64_t n = lane < 16u ? crc_tail(J) : J.end - J.start;
     const uint32_t bit = lane < 16u ? lane : lane - 16u;
     uint32_t f = (n >> bit) & 1u ? c_crc.x2k[bit + 3u] : CRC_ONE;
 #pragma unroll
@@ -230,10 +244,16 @@ __global__ __launch_bounds__(256) void k_crc_final(const CrcJob *__restrict__ jo
     const uint32_t a = gf2_mul(f, __shfl_xor(f, 16));   // lanes 32..: bits 16..47 of len
     const uint32_t l = gf2_mul(__shfl(a, 32), __shfl(f, 16));
     const uint32_t fq = __shfl(f, 0);
-    if (lane == 0u) {
-      const uint32_t pure = J.n_blocks ? gf2_mul(acc_a[i], fq) ^ acc_b[i] : 0u;
-      crc_out[i] = pure ^ gf2_mul(0xFFFFFFFFu, l) ^ 0xFFFFFFFFu;
-    }
+    if (lane == 0u) crc_out[i] = crc_join(J, acc_a[i], acc_b[i], fq, l);
+  }
+}
+__global__ __launch_bounds__(64) void k_crc_final(const CrcJob *__restrict__ jobs, uint32_t n_images,
+                                                  const uint32_t *__restrict__ acc_a,
+                                                  const uint32_t *__restrict__ acc_b, uint32_t *crc_out)
+{
+  for (uint64_t i = blockIdx.x * 64u + threadIdx.x; i < n_images; i += gridDim.x * 64u) {
+    const CrcJob J = jobs[i];
+    crc_out[i] = crc_join(J, acc_a[i], acc_b[i], crc_x8n(c_crc, crc_tail(J)), crc_x8n(c_crc, J.end - J.start));
   }
 }
 

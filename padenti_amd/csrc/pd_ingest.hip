@@ -198,8 +198,12 @@ struct CrcBatch {
     if (total)
       hipLaunchKernelGGL(k_crc32, dim3(grid_for(total, 4, 1u << 20)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o),
                          t.at<uint32_t>(chunk0_o), n, total, X.P.as<uint32_t>(), X.gap.as<uint32_t>(), acc, acc + n);
-    hipLaunchKernelGGL(k_crc_final, dim3(grid_for(n, 4)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o), n, acc, acc + n,
-                       d_crc);
+    if (n <= CRC_WAVES)
+      hipLaunchKernelGGL(k_crc_final_wave, dim3(grid_for(n, 4)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o), n, acc,
+                         acc + n, d_crc);
+    else
+      hipLaunchKernelGGL(k_crc_final, dim3(grid_for(n, 64)), dim3(64), 0, X.stream, t.at<CrcJob>(jobs_o), n, acc,
+                         acc + n, d_crc);
     HIPCHK(hipGetLastError());
   }
 };

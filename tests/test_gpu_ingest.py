@@ -60,12 +60,15 @@ def test_crc32_ragged_ranges(gpu):
     crc.free()
 
 
-def test_crc32_more_images_than_one_grid_holds(gpu):
+# a wave an image up to 1024 of them, a thread an image above; four images a block
+# had ended at the bounded grid of 65535 x 16 blocks
+@pytest.mark.parametrize("n", [1, 5, 1023, 1024, 1025, 4 * 65535 * 16 + 65])
+def test_crc32_of_many_images(gpu, n):
     rng = np.random.default_rng(2)
     buf = rng.integers(0, 256, 1 << 16, dtype=np.uint8)
-    n = 4 * 65535 * 16 + 65   # a wave per image, four a block: past a grid of 65535 x 16 blocks
-    off = rng.integers(0, buf.size - 300, 4096).astype(np.uint64)
+    off = rng.integers(0, buf.size - 9000, 4096).astype(np.uint64)
     size = rng.integers(0, 300, 4096).astype(np.uint64)
+    size[::7] = rng.integers(4000, 9000, size[::7].size)
     want = np.array([zlib.crc32(buf[int(o):int(o + k)].tobytes()) for o, k in zip(off, size)], np.uint32)
     reps = -(-n // 4096)
     off, size, want = (np.tile(a, reps)[:n] for a in (off, size, want))
