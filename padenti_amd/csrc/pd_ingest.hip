@@ -28,13 +28,12 @@ struct IngestDev {
   std::recursive_mutex mu;
   hipStream_t stream = nullptr;
   DevBuf draws, mt_state, seg_counts, seg_draw;   // class-weighted sampler
-  DevBuf tables, P, gap, crc, bits, cnt, pre, unsorted, bucket, class_count, seg_end, sort_tmp, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
+  DevBuf tables, late_tables, acc, P, gap, crc, bits, cnt, pre, unsorted, bucket, class_count, seg_end, sort_tmp, data, labels, samples, n_out, crc_out, keys, cls, rgb, lab_out;
   std::vector<uint32_t> hP;  // x^(8 * 4096 j) mod P
   std::vector<uint32_t> hgap;  // [4][256]: byte k of a register times x^(8 * CRC_GAP)
-  std::vector<CrcJob> h_jobs;
   std::vector<SampleJob> h_sjobs;
-  std::vector<uint32_t> h_blk0, h_tile0, h_seg_begin, h_B, h_boff, h_keys;
-  std::vector<uint8_t> h_cls, h_stage, h_tables;
+  std::vector<uint32_t> h_tile0, h_seg_begin, h_B, h_boff, h_keys;
+  std::vector<uint8_t> h_cls, h_stage, h_tables, h_late_tables;
   std::vector<Event> ev{5};   // stage times (Timer)
   size_t n_P = 0;   // entries of P and whether gap are on the device (constants)
   bool have_gap = false;
@@ -71,34 +70,39 @@ void upload(DevBuf &b, const std::vector<T> &v, hipStream_t s)
   if (!v.empty()) HIPCHK(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
 }
 
-// The host tables of a call in one buffer and one copy (a copy costs about 3 us
-// of the GPU's time and as much of the host's).
+// Host tables of a call in one buffer and one copy (a copy costs about 3 us of the
+// GPU's time and as much of the host's).
 struct Tables {
-  IngestDev &X;
-  explicit Tables(IngestDev &x) : X(x) { X.h_tables.clear(); }
+  DevBuf &dev;
+  std::vector<uint8_t> &buf;
+  Tables(DevBuf &d, std::vector<uint8_t> &h) : dev(d), buf(h) { buf.clear(); }
   size_t reserve(size_t bytes)   // zeros
   {
-    const size_t o = X.h_tables.size();
-    X.h_tables.resize(o + ((bytes + 15) & ~(size_t)15), 0);
+    const size_t o = buf.size();
+    buf.resize(o + ((bytes + 15) & ~(size_t)15), 0);
     return o;
   }
   template <class T>
   size_t add(const std::vector<T> &v)
   {
     const size_t o = reserve(v.size() * sizeof(T));
-    if (!v.empty()) std::memcpy(X.h_tables.data() + o, v.data(), v.size() * sizeof(T));
+    if (!v.empty()) std::memcpy(buf.data() + o, v.data(), v.size() * sizeof(T));
     return o;
   }
-  void commit()
+  void commit(hipStream_t s)
   {
-    X.tables.ensure(std::max<size_t>(X.h_tables.size(), 16));
-    if (!X.h_tables.empty())
-      HIPCHK(hipMemcpyAsync(X.tables.p, X.h_tables.data(), X.h_tables.size(), hipMemcpyHostToDevice, X.stream));
+    dev.ensure(std::max<size_t>(buf.size(), 16));
+    if (!buf.empty()) HIPCHK(hipMemcpyAsync(dev.p, buf.data(), buf.size(), hipMemcpyHostToDevice, s));
+  }
+  template <class T>
+  T *host(size_t o) const   // until the next reserve() or add()
+  {
+    return (T *)(buf.data() + o);
   }
   template <class T>
   T *at(size_t o) const
   {
-    return (T *)((char *)X.tables.p + o);
+    return (T *)((char *)dev.p + o);
   }
 };
 
@@ -153,10 +157,11 @@ struct CrcBatch {
   void add(uint32_t n_, const uint8_t *base, const uint64_t *off, const uint64_t *bytes)
   {
     n = n_;
-    std::vector<CrcJob> &jobs = X.h_jobs;
-    std::vector<uint32_t> &chunk0 = X.h_blk0;
-    jobs.assign(n, CrcJob{});
-    chunk0.assign(n, 0u);
+    jobs_o = t.reserve((size_t)n * sizeof(CrcJob));
+    chunk0_o = t.reserve((size_t)n * 4u);
+    if (n <= CRC_WAVES) acc_o = t.reserve(2ull * n * 4u);   // the two accumulators, zero (else X.acc)
+    CrcJob *jobs = t.host<CrcJob>(jobs_o);
+    uint32_t *chunk0 = t.host<uint32_t>(chunk0_o);
     uint64_t chunks = 0;
     uint32_t max_nb = 0;
     for (uint32_t i = 0; i < n; i++) {
@@ -180,9 +185,6 @@ struct CrcBatch {
       for (uint32_t k = 0; k < 4; k++)
         for (uint32_t v = 0; v < 256; v++) X.hgap[k * 256 + v] = gf2_mul(v << (8 * k), C);
     }
-    jobs_o = t.add(jobs);
-    chunk0_o = t.add(chunk0);
-    acc_o = t.reserve(2ull * n * 4u);   // the two accumulators, zero
   }
   void launch(uint32_t *d_crc)
   {
@@ -195,6 +197,11 @@ struct CrcBatch {
       X.have_gap = true;
     }
     uint32_t *acc = t.at<uint32_t>(acc_o);
+    if (n > CRC_WAVES) {
+      X.acc.ensure(2ull * n * 4u);
+      acc = X.acc.as<uint32_t>();
+      hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(2ull * n, 256)), dim3(256), 0, X.stream, acc, 2ull * n, 0u);
+    }
     if (total)
       hipLaunchKernelGGL(k_crc32, dim3(grid_for(total, 4, 1u << 20)), dim3(256), 0, X.stream, t.at<CrcJob>(jobs_o),
                          t.at<uint32_t>(chunk0_o), n, total, X.P.as<uint32_t>(), X.gap.as<uint32_t>(), acc, acc + n);
@@ -270,9 +277,18 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
   tm.mark(0);
   X.crc.ensure((size_t)n * 4u);
   uint32_t *crc = d_crc ? d_crc : X.crc.as<uint32_t>();
-  Tables tab(X);
-  CrcBatch cb{X, tab};
+  // few images: one upload for everything.  Many: the CRC's tables first, the others
+  // are made while it runs (5000 images, class-weighted: 0.05 ms of the call)
+  Tables first(X.tables, X.h_tables), later(X.late_tables, X.h_late_tables);
+  const bool early = n > CRC_WAVES;
+  CrcBatch cb{X, first};
   cb.add(n, (const uint8_t *)d_data, data_off, data_bytes);
+  if (early) {
+    first.commit(st);
+    cb.launch(crc);
+    tm.mark(1);
+  }
+  Tables &tab = early ? later : first;
   const bool weighted = s.kind == PD_SAMPLER_CLASS_WEIGHTED;
   // class-weighted: segments of whole 1024-pixel steps, about 16384 in the batch
   // (64 waves a CU)
@@ -294,13 +310,15 @@ void sample_dev(int device, const pd_sampler &s, uint32_t n, const void *d_data,
   const size_t o_jobs = tab.add(jobs), o_begin = tab.add(seg_begin), o_first = tab.add(tile0);
   const size_t o_B = weighted ? tab.add(X.h_B) : 0, o_boff = weighted ? tab.add(X.h_boff) : 0;
   const size_t o_bad = tab.reserve(4);
-  tab.commit();
+  tab.commit(st);
   const SampleJob *d_jobs = tab.at<SampleJob>(o_jobs);
   const uint32_t *d_begin = tab.at<uint32_t>(o_begin), *d_first = tab.at<uint32_t>(o_first);
   const uint32_t *d_B = tab.at<uint32_t>(o_B), *d_boff = tab.at<uint32_t>(o_boff);
   uint32_t *d_bad = tab.at<uint32_t>(o_bad);
-  cb.launch(crc);
-  tm.mark(1);
+  if (!early) {
+    cb.launch(crc);
+    tm.mark(1);
+  }
   X.seg_end.ensure((size_t)n * 4u);
   X.unsorted.ensure((size_t)n * cap * 4u + 4u);
   uint32_t *uns = X.unsorted.as<uint32_t>();
@@ -514,10 +532,10 @@ int pd_crc32_images_dev(int device, uint32_t n, const void *d_data, uint64_t dat
     Lock g(X.mu);
     Timer tm(X);
     tm.mark(0);
-    Tables tab(X);
+    Tables tab(X.tables, X.h_tables);
     CrcBatch cb{X, tab};
     cb.add(n, (const uint8_t *)d_data, offsets, bytes);
-    tab.commit();
+    tab.commit(X.stream);
     cb.launch(d_crc);
     tm.mark(1);
     HIPCHK(hipStreamSynchronize(X.stream));

@@ -121,6 +121,18 @@ def test_uniform_sampler_matches_oracle(gpu, n_samples, seed):
             assert g.size == n_samples
 
 
+@pytest.mark.parametrize("n", [1024, 1025])   # the CRC's tables with the sampler's, and ahead of them
+def test_uniform_sampler_of_many_images(gpu, n):
+    rng = np.random.default_rng(n)
+    labs = [rng.integers(0, 3, (int(rng.integers(1, 40)), int(rng.integers(1, 40))), dtype=np.uint8) for _ in range(n)]
+    datas = [rng.integers(0, 65536, l.shape, dtype=np.uint16) for l in labs]
+    got, crc = ds.UniformImageSampler(20, seed=4).sample_batch(datas, labs, crc=True)
+    want, wcrc = oi.sample_images(0, datas, labs, 20, seed=4)
+    assert np.array_equal(crc, wcrc)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert np.array_equal(g, w), i
+
+
 @pytest.mark.parametrize("n_classes,weights,n_samples", [
     (8, None, 2000), (8, "random", 300), (8, "zeros", 64), (1, [1.0], 5), (8, "big", 50), (255, None, 3000),
     (8, "big", 2000)])   # the last: 48000 slots per image
