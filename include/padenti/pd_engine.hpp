@@ -899,10 +899,8 @@ struct Trainer final : TrainerBase {
         hslots.push_back(q);
       }
       for (uint32_t k = 0; k < chunks; k++) {
-        // equal shares (at most ch samples each)
-        const uint32_t o = (uint32_t)((uint64_t)cnt * k / chunks);
-        const uint32_t b = si.begin + o;
-        const uint32_t c = (uint32_t)((uint64_t)cnt * (k + 1) / chunks) - o;
+        const uint32_t b = chunk_begin(si.begin, cnt, chunks, k);
+        const uint32_t c = chunk_begin(si.begin, cnt, chunks, k + 1) - b;
         if (direct) {
           groups.push_back(uint4{q, b, c, 0u});
           continue;

@@ -18,6 +18,10 @@ uint32_t item_chunk(uint64_t level_samples, uint32_t nF, uint32_t ftiles, uint32
 {
   return pd::engine::item_chunk(level_samples, nF, ftiles, nT, nC, cus, blocks_per_cu, launches);
 }
+uint32_t chunk_begin(uint32_t begin, uint32_t n, uint32_t chunks, uint32_t k)
+{
+  return pd::engine::chunk_begin(begin, n, chunks, k);
+}
 size_t deal(size_t n, const uint32_t *samples, uint32_t n_xcc, uint32_t *order, uint32_t *xcd)
 {
   const pd::engine::GroupOrder r = pd::engine::deal_groups(std::vector<uint32_t>(samples, samples + n), n_xcc);
@@ -37,6 +41,7 @@ def host(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-I", os.path.join(ROOT, "include"), str(src), "-o",
                     str(lib)], check=True)
     so = C.CDLL(str(lib))
+    so.chunk_begin.restype, so.chunk_begin.argtypes = C.c_uint32, [C.c_uint32] * 4
     so.deal.restype, so.deal.argtypes = C.c_size_t, [C.c_size_t, C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p]
     return so
 
@@ -93,3 +98,18 @@ def test_groups_are_dealt_once_and_evenly(host, samples, X):
         assert max(load) - min(load) <= max(samples) + 64
     if len(set(samples)) > 1:   # the smallest ones come last
         assert samples[order[-1]] == min(samples)
+
+
+@pytest.mark.parametrize("begin", [0, 1, 2, 3, 4, 1001, 4_294_000_000])
+@pytest.mark.parametrize("n,chunk", [(0, 64), (1, 64), (64, 64), (65, 64), (128, 64), (200, 64), (1000, 333),
+                                     (65536, 32768), (65537, 32768), (294_967, 32768)])
+def test_chunks_of_a_node_begin_on_record_lines(host, begin, n, chunk):
+    """The chunks of a node cover its records once and in order, differ by a few
+    records, and every one but the first begins on a 64-byte line of them."""
+    chunks = max(1, -(-n // chunk))
+    cut = [host.chunk_begin(begin, n, chunks, k) & 0xffffffff for k in range(chunks + 1)]
+    assert cut[0] == begin and cut[-1] == begin + n
+    assert all(c % 4 == 0 for c in cut[1:-1])
+    sizes = [b - a for a, b in zip(cut, cut[1:])]
+    assert all(0 <= s <= min(chunk, -(-n // chunks)) + 3 and (n == 0 or s > 0) for s in sizes)
+    assert max(sizes) - min(sizes) <= 7
