@@ -409,8 +409,14 @@ __global__ __launch_bounds__(256) void k_cand_table(uint32_t tree, const int32_t
   }
 }
 
+// Eight waves a SIMD are asked for to bound the scalar registers: a SIMD has 800 and,
+// with 16 a wave for the trap handler, a wave with more than 80 leaves room for
+// seven; the pruned search's loops had taken some instantiations to 82.  Hooks whose
+// tile leaves LDS for more blocks lose by it: the int16 demo hook, 300 images, 1000 x
+// 20 candidates, 14.0 ms of histograms a tree at 74 registers (before the pruned
+// search), 14.6 at 82, 12.6 at 78; the depth hooks are within 0.5% either way.
 template <class F, int NTP, int NWAVES = HIST_THREADS / 64, bool WIDE = false, int SPW = 1>
-__global__ __launch_bounds__(NWAVES * 64) void k_hist(
+__global__ __launch_bounds__(NWAVES * 64, 8) void k_hist(
     const typename F::ImgType *__restrict__ pixels, const ImgDesc *__restrict__ imgs,
     const uint4 *__restrict__ recs, const HistItem *__restrict__ items, uint32_t item_base,
     const int32_t *__restrict__ slot_node, const uint8_t *__restrict__ slot_mode,
