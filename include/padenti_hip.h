@@ -145,7 +145,8 @@ PD_API int pd_trainer_set_data(pd_trainer *tr, uint32_t n_images, const void *pi
  * histograms exceed it are processed in slices (the reference slices at
  * GLOBAL_HISTOGRAM_MAX_SIZE of host RAM, cl_tree_trainer_impl.hpp:50). */
 PD_API int pd_trainer_set_hist_budget(pd_trainer *tr, uint64_t bytes);
-/* Samples per histogram work item (0 = automatic). */
+/* Samples per histogram work item (0 = automatic; an item may hold up to three
+ * more, its node's chunks beginning on 64-byte lines of the sample records). */
 PD_API int pd_trainer_set_chunk(pd_trainer *tr, uint32_t samples_per_chunk);
 /* Probe-coherent candidate tiles (default on): for feature hooks that name
  * the row offset parameters of their probes, each node's candidates are
@@ -191,7 +192,7 @@ typedef struct {
 } pd_tuning_rule;
 PD_API int pd_trainer_set_tuning_rules(pd_trainer *tr, uint32_t n_rules, const pd_tuning_rule *rules);
 /* Placement of the level-batched histogram's work items on the XCDs (each
- * XCD has its own L2): 0 deals the (node, chunk) groups round robin; 1 places
+ * XCD has its own L2): 0 deals the (node, chunk) groups evenly by samples; 1 places
  * a chunk of a node cut into at least as many chunks as there are XCDs on
  * the XCD of its position in the node's (image-ordered) samples, so chunks
  * of different nodes over the same images share one L2.  Timing only: trees

@@ -258,9 +258,9 @@ class HIPTreeTrainer:
         check(lib().pd_trainer_set_proposal_refine(self._h, int(stride), int(min_samples)))
 
     def set_xcd_order(self, by_position):
-        """XCD placement of the level-batched histogram's work items: round
-        robin by (node, chunk) group (False) or by the chunk's position in its
-        node's image-ordered samples (True).  Trees are identical either way."""
+        """XCD placement of the level-batched histogram's work items: (node,
+        chunk) groups dealt evenly by samples (False) or by the chunk's position in
+        its node's image-ordered samples (True).  Trees are identical either way."""
         check(lib().pd_trainer_set_xcd_order(self._h, 1 if by_position else 0))
 
     def set_candidate_table(self, enable):
